@@ -21,6 +21,10 @@ struct alignas(64) DevPrime {
     // 2^64 - 4q and 2^64 - 8q: the NTT's conditional subtractions as one 64-bit add
     // (a constant the compiler cannot see as a negation stays an add)
     uint64_t neg_four_q, neg_eight_q;
+    // primes below FP_PRIME_LIMIT (butterfly_fp.h), else null: the forward table as
+    // (w centred, RN(w / q)) doubles; q and RN(1 / q)
+    const double2 *fwd_fp;
+    double q_fp, q_inv_fp;
 };
 
 // Constants of a divide-and-round by a prime p into prime q_i (p = the special prime

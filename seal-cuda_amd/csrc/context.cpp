@@ -1,6 +1,8 @@
 // context.cpp -- builds and uploads the per-parameter-set tables.
 #include "context.h"
+#include "butterfly_fp.h"
 #include "ckks_encoder.h"
+#include "ntt.h"
 #include <cstring>
 
 namespace shc {
@@ -24,6 +26,15 @@ DevPrime upload_prime(Context &c, uint64_t q) {
     p.fwd = buf.as<const ulonglong2>();
     p.inv = reinterpret_cast<const ulonglong2 *>(static_cast<char *>(buf.ptr) + bytes);
     c.table_bufs.push_back(std::move(buf));
+    if (q < FP_PRIME_LIMIT) {
+        DevBuf fp(c.n * sizeof(double2));
+        build_fp_table(p.fwd, fp.as<double2>(), q, c.logn, nullptr);
+        SHC_HIP(hipStreamSynchronize(nullptr));  // built before any stream's transform reads it
+        p.fwd_fp = fp.as<const double2>();
+        p.q_fp = (double)q;
+        p.q_inv_fp = 1.0 / (double)q;
+        c.table_bufs.push_back(std::move(fp));
+    }
     return p;
 }
 
@@ -66,7 +77,10 @@ std::unique_ptr<Context> make_context(Scheme scheme, int logn, const std::vector
     c->n = uint64_t(1) << logn;
     c->moduli = moduli;
     c->plain = plain;
-    for (uint64_t q : moduli) c->host_primes.push_back(upload_prime(*c, q));
+    for (uint64_t q : moduli) {
+        c->host_primes.push_back(upload_prime(*c, q));
+        c->fp_primes |= q < FP_PRIME_LIMIT;
+    }
 
     const size_t K = moduli.size();
     c->d_primes = upload(c->host_primes);

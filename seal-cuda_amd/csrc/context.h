@@ -28,6 +28,7 @@ struct Context {
     uint64_t n = 0;
     std::vector<uint64_t> moduli;      // key level, special prime last
     uint64_t plain = 0;
+    bool fp_primes = false;            // some modulus takes the fp64 transforms (butterfly_fp.h)
 
     std::vector<DevPrime> host_primes;
     std::vector<DevBuf> table_bufs;

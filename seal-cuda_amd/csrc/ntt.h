@@ -49,7 +49,7 @@ void ntt_inverse_from(const uint64_t *src, LimbGrid src_grid, uint64_t *data, Li
 // `shape` overrides the launch shape (KsShape; rows_group applies to the fused form).
 bool ntt_forward_modup(const uint64_t *d, size_t d_ct_stride, uint64_t *T, uint32_t count, uint32_t L,
                        const DevPrime *targets, const DevPrime *digits, int logn, bool skip_diag, bool reduce_4q,
-                       hipStream_t stream, const KernelProbe *probe = nullptr, KsShape shape = KsShape{});
+                       bool mixed, hipStream_t stream, const KernelProbe *probe = nullptr, KsShape shape = KsShape{});
 
 // The same ModUp with its rows pass fused into the products by the key (N = 2^15, 2^16;
 // returns false and does nothing otherwise): the columns pass fills T as above (diag !=
@@ -72,8 +72,20 @@ struct KsFold {
 bool ntt_modup_keyprod(const uint64_t *d, size_t d_ct_stride, uint64_t *T, const uint64_t *key, uint64_t *P,
                        uint64_t *S, const uint64_t *diag, size_t diag_stride, uint32_t count, uint32_t L,
                        uint32_t key_count, const DevPrime *targets, const DevPrime *digits, int logn,
-                       hipStream_t stream, const KernelProbe *probe = nullptr, KsShape shape = KsShape{},
+                       bool mixed, hipStream_t stream, const KernelProbe *probe = nullptr, KsShape shape = KsShape{},
                        KsFold fold = KsFold{});
+
+// NTT-form permutations sigma_e read on load: polynomial j of a batch goes through
+// elt[j / polys] (polys == 0: none).  sigma maps a whole aligned row of a limb onto another
+// one, so the gathered reads stay within the rows a block reads anyway.
+constexpr uint32_t PERM_MAX = 4;
+struct GaloisPerm {
+    uint32_t polys = 0;
+    uint32_t elt[PERM_MAX] = {};
+};
+// data (grid) = inverse transform of sigma(src) (grid src_grid), N >= 2^13, fully reduced.
+void ntt_inverse_galois(const uint64_t *src, LimbGrid src_grid, const GaloisPerm &perm, uint64_t *data,
+                        LimbGrid grid, const DevPrime *primes, int logn, hipStream_t stream);
 
 // ModDown by the special prime p fused into the last transforms of a key switch, for
 // `count` ciphertexts at L limbs (N >= 2^13; returns false and does nothing otherwise):
@@ -85,6 +97,12 @@ bool ntt_modup_keyprod(const uint64_t *d, size_t d_ct_stride, uint64_t *T, const
 // p_lpp != 0 (CKKS only): P holds p_lpp limbs per polynomial, polynomial (ct, k) at
 // ct * p_ct_stride + k * p_lpp * N words -- a ciphertext with a limb above the L kept
 // ones, divided and rounded by its last prime (a rescale; folded).
+// presum != 0 (at most 15): S holds the sum over `presum` key switches of the rounded special
+// limbs [s + floor(p/2)]_p, as whole numbers, and P the sum of their products: u_i, and so
+// the result, is the sum of the separate corrections (the transforms are linear and the
+// rounding is per key switch), with one transform for all of them.
+// perm (polys != 0): P is read through NTT-form permutations, in place of permuted copies;
+// its (ct, k) polynomials are counted like S's and ct's (BFV: from `P` into `buf`).
 struct ModDownArgs {
     const uint64_t *S;
     const uint64_t *P;
@@ -96,6 +114,8 @@ struct ModDownArgs {
     bool folded;
     size_t p_ct_stride = 0;
     uint32_t p_lpp = 0;
+    uint32_t presum = 0;
+    GaloisPerm perm{};
 };
 bool ntt_moddown(bool ckks, uint64_t *buf, const ModDownArgs &args, uint32_t count, const DevPrime *primes, int logn,
                  hipStream_t stream);
@@ -161,7 +181,7 @@ struct KsGroup {
 // The fused ModUp + key products of every group (N = 2^15, 2^16; false otherwise): one
 // columns-pass launch and one rows-pass launch per ciphertext grouping (4, 2, 1).
 bool ntt_modup_keyprod_groups(const KsGroup *groups, uint32_t n, const uint64_t *key, uint32_t key_count,
-                              const DevPrime *digits, int logn, hipStream_t stream);
+                              const DevPrime *digits, int logn, bool mixed, hipStream_t stream);
 
 // ModDown groups (CKKS, N >= 2^13; false otherwise): buf = U scratch of the group.
 struct ModDownGroup {
@@ -170,5 +190,8 @@ struct ModDownGroup {
     uint32_t count;
 };
 bool ntt_moddown_groups(const ModDownGroup *groups, uint32_t n, const DevPrime *primes, int logn, hipStream_t stream);
+
+// The fp64 form of a forward twiddle table (N entries) of a prime below FP_PRIME_LIMIT.
+void build_fp_table(const ulonglong2 *table, double2 *out, uint64_t q, int logn, hipStream_t stream);
 
 }  // namespace shc

@@ -432,8 +432,8 @@ void switch_key_chunk(const Context &c, const uint64_t *target, size_t target_st
     const KsShape shape = c.ks_shape(L, count);
     const KsFold fold = ckks ? KsFold{fold_c0 ? fold_c0 : ct, ct_stride, c.ks_consts(), fold_c0 != nullptr} : KsFold{};
     const bool fused = ntt_modup_keyprod(digits, dstride, T, key, P, S, diag, target_stride, count, L,
-                                         (uint32_t)c.key_count(), c.keyswitch_primes(L), c.primes(), logn, st, probe,
-                                         shape, fold);
+                                         (uint32_t)c.key_count(), c.keyswitch_primes(L), c.primes(), logn,
+                                         c.fp_primes, st, probe, shape, fold);
     if (fold_c0 && !fused) fail(ERR_LOGIC, "a key switch into (c0, 0) needs the fused key products");
     if (!fused) {
         const bool skipped = modup_to_T(c, digits, dstride, T, count, L, st, probe, diag != nullptr);
@@ -452,8 +452,8 @@ bool modup_to_T(const Context &c, const uint64_t *digits, size_t dstride, uint64
     // T's consumers (inner products with the key, hoisted rotation products) sum L
     // products T * key (key < q < 2^60) and one more term < q in 128 bits: T may stay
     // in [0, 8q) up to L = 31 (31 * 8q^2 < 2^127.95), in [0, 4q) beyond.
-    if (ntt_forward_modup(digits, dstride, T, count, L, targets, c.primes(), logn, skip_diag, L > 31, st, probe,
-                          c.ks_shape(L, count)))
+    if (ntt_forward_modup(digits, dstride, T, count, L, targets, c.primes(), logn, skip_diag, L > 31, c.fp_primes, st,
+                          probe, c.ks_shape(L, count)))
         return skip_diag;
     const size_t twords = ((size_t)count * L * (L + 1)) << logn;
     modup_gather_kernel<<<blocks_for(twords), TPB, 0, st>>>(digits, dstride, T, targets, c.primes(), count, L, logn,
@@ -672,7 +672,7 @@ void relinearize_groups(const Context &c, const RelinGroup *gs, uint32_t n, cons
         // 1. digits: the c2 polynomials to coefficient form (they stay in NTT form for the
         // own-prime terms); 2. ModUp fused with the key products; 3. ModDown
         ntt_inverse_groups(dg, k, logn, NTT_FULL, st);
-        ntt_modup_keyprod_groups(kg, k, key, (uint32_t)K, c.primes(), logn, st);
+        ntt_modup_keyprod_groups(kg, k, key, (uint32_t)K, c.primes(), logn, c.fp_primes, st);
         ntt_inverse_groups(sg, k, logn, NTT_FULL, st);
         ntt_moddown_groups(mg, k, c.primes(), logn, st);
     });

@@ -9,14 +9,20 @@
 //     [0, 8q);
 //   * the key-switch product sums (accum.h): 31 products t k with t < 8q or 63 with
 //     t < 4q (k < q), plus one correction word, equal the exact 128-bit sum;
+//   * for q < 2^50, the fp64 forms (butterfly_fp.h): products and butterflies congruent and
+//     within the bound each layer states for operands at the ends of the passes' ranges,
+//     the passes' schedules within 8q and the ranges they hand over, the conversions, and
+//     the 26-bit product sums (accum.h) over 64 terms;
 // for primes from 17 to 61 bits, random and extreme operands (0, range ends,
 // multiples of q +- 1, all-ones words).  Exact products come from unsigned __int128.
 // Prints "ok <cases>" and exits 0, or prints the first failing case and exits 1.
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <vector>
 #include "accum.h"
 #include "butterfly.h"
+#include "butterfly_fp.h"
 
 using u64 = uint64_t;
 using wide = unsigned __int128;
@@ -72,6 +78,82 @@ static u64 operand(u64 bound, u64 q, int k) {
     }
 }
 
+// x mod q of an integer held in a double.
+static u64 residue(double x, u64 q) {
+    __int128 v = (__int128)x % (__int128)q;
+    return (u64)(v < 0 ? v + q : v);
+}
+
+// The fp64 forms for one prime below 2^50; false (after a message) at the first failure.
+static bool check_fp(u64 q, long &cases) {
+    const double qd = (double)q, qinv = 1.0 / qd;
+    // the bound of |x| / q through a pass: each layer's outputs, the schedule of fp_centers
+    auto layer = [](double c, bool center) { return (center ? 0.5 : c) + 0.5 + c / 8 + 1e-9; };
+    struct Pass {
+        bool rows;
+        int K;
+    };
+    for (int K1 = 6; K1 <= 8; K1++) {
+        for (Pass p : {Pass{false, K1}, Pass{true, K1}, Pass{true, K1 + 1}}) {
+            if (p.K < 7 && p.rows) continue;  // N = 2^13 .. 2^17: K1 = 6..8, K2 = 7..9
+            double in = p.rows ? 3.5 : 2.0;
+            for (int s = 0; s < p.K; s++) {
+                in = layer(in, shc::fp_centers(p.rows, p.K, s));
+                if (in > 7) return std::printf("fp pass bound %d %d\n", p.K, s), false;
+            }
+            if (!p.rows && in > 3.5) return std::printf("fp columns pass leaves %f\n", in), false;
+            if (p.rows && in > 1.7) return std::printf("fp rows pass leaves %f\n", in), false;
+        }
+    }
+    for (int wi = 0; wi < 16; wi++) {
+        const u64 w = wi == 0 ? 0 : wi == 1 ? 1 : wi == 2 ? q - 1 : wi == 3 ? q / 2 : wi == 4 ? q / 2 + 1 : next() % q;
+        const double wc = 2 * w > q ? (double)((int64_t)w - (int64_t)q) : (double)w;
+        const double2 tw{wc, wc / qd};
+        for (int c = 1; c <= 7; c++)
+            for (int k = 0; k < 24; k++) {
+                auto pick = [&](int m) {
+                    const u64 lim = c * q;
+                    const double v = (double)(m == 0 ? lim : m == 1 ? lim - 1 : m == 2 ? q / 2 : next() % (lim + 1));
+                    return next() & 1 ? -v : v;
+                };
+                const double x = pick(k % 4), y = pick(k / 4 % 4);
+                for (bool center : {false, true}) {
+                    double a = x, b = y;
+                    shc::fp_butterfly(a, b, tw, qd, qinv, center);
+                    const u64 v = mulmod(residue(y, q), w, q), xr = residue(x, q);
+                    if (residue(a, q) != (xr + v) % q || residue(b, q) != (xr + q - v) % q)
+                        return std::printf("fp butterfly q=%llu w=%llu x=%.0f y=%.0f\n", (unsigned long long)q,
+                                           (unsigned long long)w, x, y), false;
+                    const double most = layer(c, center) * qd + 1;
+                    if (std::fabs(a) > most || std::fabs(b) > most)
+                        return std::printf("fp range q=%llu w=%llu x=%.0f y=%.0f\n", (unsigned long long)q,
+                                           (unsigned long long)w, x, y), false;
+                    cases++;
+                }
+            }
+    }
+    const double up = 4503599627370496.0 + 2 * qd;
+    for (int k = 0; k < 64; k++) {
+        const u64 d = k < 2 ? k : k == 2 ? 2 * q - 1 : next() % (2 * q);
+        if (shc::fp_from_u52(d) != (double)d) return std::printf("fp_from_u52\n"), false;
+        const double x = (k & 1 ? -1 : 1) * (double)(next() % (17 * (q / 10) + 1));
+        if (shc::fp_to_u52(x, up) != (u64)((int64_t)x + (int64_t)(2 * q))) return std::printf("fp_to_u52\n"), false;
+    }
+    for (int ext = 0; ext < 2; ext++) {
+        shc::Acc26 a{0, 0, 0};
+        wide sum = 0;
+        for (int k = 0; k < 64; k++) {
+            const u64 t = ext ? 4 * q - 1 : next() % (4 * q), f = ext ? q - 1 : next() % q;
+            shc::mac(a, shc::cut26(t), shc::cut26(f));
+            sum += (wide)t * f;
+        }
+        const shc::u128 v = shc::acc_value(a);
+        if ((((wide)v.hi << 64) | v.lo) != sum) return std::printf("Acc26 q=%llu\n", (unsigned long long)q), false;
+        cases += 64;
+    }
+    return true;
+}
+
 int main() {
     std::vector<u64> primes;
     // the largest prime below 2^b (b = 17..61), an NTT prime 1 mod 2^17 near 2^b, 2^61 - 1
@@ -86,6 +168,7 @@ int main() {
     }
     long cases = 0;
     for (u64 q : primes) {
+        if (q < shc::FP_PRIME_LIMIT && !check_fp(q, cases)) return 1;
         const u64 neg_q = 0 - q, four_q = q << 2;
         for (int wi = 0; wi < 24; wi++) {
             const u64 w = wi == 0 ? 0 : wi == 1 ? 1 : wi == 2 ? q - 1 : next() % q;

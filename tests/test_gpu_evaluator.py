@@ -81,6 +81,39 @@ def test_relinearize(scheme, logn, bits, L, count):
         np.testing.assert_array_equal(got[c], ck.relinearize(scheme, ct3[c], key, moduli, L, logn))
 
 
+@pytest.mark.parametrize("scheme,logn,bits,L,count", [
+    # primes below 2^50 take the fp64 transforms and 26-bit product sums: alone, beside 60-bit
+    # targets, with digits far above and below a target (30 to 60 bits), every degree they
+    # run at, a level of one digit (no rows but the own-prime one), groups of 4, 2 and 1
+    (CKKS, 13, [50] * 4, 3, 2),
+    (CKKS, 14, [60, 50, 30, 45, 60], 4, 3),
+    (BFV, 14, [30, 50, 60, 36, 40], 4, 2),
+    (CKKS, 15, [60] + [50] * 5 + [60], 6, 7),
+    (BFV, 15, [45, 50, 60, 50], 3, 5),
+    (CKKS, 15, [50, 50], 1, 5),
+    (CKKS, 15, [60, 60], 1, 3),
+    (CKKS, 16, [50] * 6, 5, 7),
+    (CKKS, 17, [60, 40, 50, 60], 3, 2),
+    # more digits than a step's, at the bound of the primes
+    (CKKS, 15, [50] * 18, 17, 4),
+])
+@pytest.mark.parametrize("words", ["uniform", "largest"])
+def test_relinearize_fp64_primes(scheme, logn, bits, L, count, words):
+    ctx, moduli = make_ctx(scheme, logn, bits, 65537 if scheme == BFV else 0)
+    n = 1 << logn
+    rng = np.random.default_rng(200 + logn + L)
+    ct3 = ck.uniform_residues(rng, (count, 3, L, n), moduli[:L])
+    key = ck.random_key(rng, moduli, logn)
+    if words == "largest":  # every residue q - 1 (and the last ciphertext zero)
+        q = np.array(moduli, dtype=np.uint64)
+        ct3[:] = (q[:L] - 1)[None, None, :, None]
+        ct3[-1] = 0
+        key[:] = (q - 1)[None, None, :, None]
+    got = run_relin(ctx, ct3, key, L)
+    for c in (0, count - 1):
+        np.testing.assert_array_equal(got[c], ck.relinearize(scheme, ct3[c], key, moduli, L, logn))
+
+
 def test_relinearize_columns_all_targets():
     """A batch large enough that each ModUp columns block transforms its digit tile for
     all L + 1 targets (104 x 20 x 8 tiles >= 16384 blocks); three ciphertexts against the
