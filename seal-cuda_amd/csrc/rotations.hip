@@ -28,6 +28,8 @@
 #include "modarith.h"
 #include "ntt.h"
 #include "rns_ops.h"
+#include <algorithm>
+#include <type_traits>
 
 namespace shc {
 namespace {
@@ -78,62 +80,72 @@ __global__ void correction_kernel(const uint64_t *__restrict__ negntt, const uin
 
 // Products of R rotations at once, each T word read once for all of them:
 //   P_r[ct][k][i] = sum_j T[i][ct][j] key'_r[j][k][ki] + corr'_r[k][i]   (S_r for i == L)
+// and with fold.ct (N >= 2^13), P_r[ct][0][i] += p c0[ct][i]: the ModDown then writes the
+// rotation without a pass that permutes and adds c0.
 // One thread per (i, c) position and RG ciphertexts (each key word it loads serves RG
-// products), with three-word sums (Acc3); the loads of digit j + 1 go out before the
-// products of digit j, and in a partial last group the missing ciphertext repeats the
-// last one (in bounds, not stored).  With diag, T holds no limb (i, i) for i < L and
-// that term is the NTT-form input limb diag[ct * diag_stride + i * N].  Blocks of one
-// tile run on one XCD (XCD = block % 8) so that the tile's key words are served from
-// its L2.
+// products); the loads of digit j + 1 go out before the products of digit j, and in a
+// partial last group the missing ciphertext repeats the last one (in bounds, not stored).
+// With diag, T holds no limb (i, i) for i < L and that term is the NTT-form input limb
+// diag[ct * diag_stride + i * N].  The waves of a block take WG groups of the same
+// positions, so that a key line is fetched once per block and its other readers hit the
+// CU's cache; blocks of one tile run on one XCD (XCD = block % 8), whose L2 serves the
+// tile's key words to the other blocks.  Sums are Acc3, or (MIXED, a block of a prime
+// below 2^50: T holds words below 4 q) Acc26 at half the instructions.
 constexpr int RMAX = 4;
+static_assert(RMAX <= (int)PERM_MAX, "a pass's rotations fit one permuted ModDown");
 constexpr int RG = 2;
 struct RotBatch {
     const uint64_t *key[RMAX];   // prepared keys; corr' follows at corr_off words
     uint64_t *P[RMAX], *S[RMAX];
     uint32_t elt[RMAX];          // their Galois elements
 };
+struct RotArgs {
+    const uint64_t *T;
+    size_t corr_off;
+    const DevPrime *targets;
+    uint32_t L, K;
+    int logn;
+    uint32_t count, tiles;
+    const uint64_t *diag;
+    size_t diag_stride;
+    KsFold fold;                 // ct: c0 of ciphertext g at ct + g * ct_stride
+};
 
-template <int R>
-__global__ __launch_bounds__(TPB) void rotation_products_kernel(const uint64_t *__restrict__ T, RotBatch rb,
-                                                                size_t corr_off, const DevPrime *__restrict__ targets,
-                                                                uint32_t L, uint32_t K, int logn, uint32_t count,
-                                                                uint32_t tiles, const uint64_t *__restrict__ diag,
-                                                                size_t diag_stride) {
-    const uint32_t groups = (count + RG - 1) / RG;
-    const uint32_t xcd = blockIdx.x & 7, q8 = blockIdx.x >> 3;
-    const uint32_t tile = (q8 / groups) * 8 + xcd;
-    if (tile >= tiles) return;
-    const uint32_t ct0 = (q8 % groups) * RG;
-    const int gv = (int)min<uint32_t>(RG, count - ct0);
-    const size_t n = (size_t)1 << logn;
-    const size_t flat = (size_t)tile * TPB + threadIdx.x;
-    if (flat >= (size_t)(L + 1) << logn) return;
-    const uint32_t i = (uint32_t)(flat >> logn);
-    const size_t c = flat & (n - 1);
-    const uint32_t ki = (i == L) ? K - 1 : i;
-    const DevPrime &Q = targets[i];
-    const bool short_row = diag && i < L;  // uniform over the block
+template <int R, bool FP>
+__device__ __forceinline__ void rotation_products_core(const RotBatch &rb, const RotArgs &a, uint32_t i, size_t c,
+                                                       uint32_t ct0, int gv) {
+    using Acc = std::conditional_t<FP, Acc26, Acc3>;
+    using Word = std::conditional_t<FP, Cut26, uint64_t>;
+    auto word = [](uint64_t x) -> Word {
+        if constexpr (FP) return cut26(x);
+        else return x;
+    };
+    const uint32_t L = a.L;
+    const size_t n = (size_t)1 << a.logn;
+    const uint32_t ki = (i == L) ? a.K - 1 : i;
+    const DevPrime &Q = a.targets[i];
+    const bool short_row = a.diag && i < L;  // uniform over the block
     const uint32_t Lt = short_row ? L - 1 : L;
-    const uint64_t *Ti = T + (((size_t)i * count * L + (size_t)ct0 * Lt) << logn) + c;
-    const size_t kstride = (size_t)K << logn;
+    const uint64_t *Ti = a.T + (((size_t)i * a.count * L + (size_t)ct0 * Lt) << a.logn) + c;
+    const size_t kstride = (size_t)a.K << a.logn;
     size_t goff[RG];
     const uint64_t *dp[RG];
 #pragma unroll
     for (int g = 0; g < RG; g++) {
-        goff[g] = ((size_t)min(g, gv - 1) * Lt) << logn;
-        dp[g] = short_row ? diag + (ct0 + min(g, gv - 1)) * diag_stride + ((size_t)i << logn) + c : nullptr;
+        goff[g] = ((size_t)min(g, gv - 1) * Lt) << a.logn;
+        dp[g] = short_row ? a.diag + (ct0 + min(g, gv - 1)) * a.diag_stride + ((size_t)i << a.logn) + c : nullptr;
     }
-    Acc3 a0[R][RG], a1[R][RG];
+    Acc a0[R][RG], a1[R][RG];
 #pragma unroll
     for (int r = 0; r < R; r++)
 #pragma unroll
-        for (int g = 0; g < RG; g++) a0[r][g] = a1[r][g] = Acc3{0, 0, 0};
+        for (int g = 0; g < RG; g++) a0[r][g] = a1[r][g] = Acc{0, 0, 0};
     uint64_t tn[RG], k0n[R], k1n[R];
     auto fetch = [&](uint32_t j) {
         const bool dj = short_row && j == i;
         const size_t jt = short_row && j > i ? j - 1 : j;
 #pragma unroll
-        for (int g = 0; g < RG; g++) tn[g] = *(dj ? dp[g] : Ti + goff[g] + (jt << logn));
+        for (int g = 0; g < RG; g++) tn[g] = *(dj ? dp[g] : Ti + goff[g] + (jt << a.logn));
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const uint64_t *kp = rb.key[r] + (size_t)ki * n + c;
@@ -143,11 +155,11 @@ __global__ __launch_bounds__(TPB) void rotation_products_kernel(const uint64_t *
     };
     fetch(0);
     for (uint32_t j = 0; j < L; j++) {
-        uint64_t t[RG], k0[R], k1[R];
+        Word t[RG], k0[R], k1[R];
 #pragma unroll
-        for (int g = 0; g < RG; g++) t[g] = tn[g];
+        for (int g = 0; g < RG; g++) t[g] = word(tn[g]);
 #pragma unroll
-        for (int r = 0; r < R; r++) k0[r] = k0n[r], k1[r] = k1n[r];
+        for (int r = 0; r < R; r++) k0[r] = word(k0n[r]), k1[r] = word(k1n[r]);
         fetch(j + 1 < L ? j + 1 : j);
 #pragma unroll
         for (int r = 0; r < R; r++)
@@ -157,9 +169,18 @@ __global__ __launch_bounds__(TPB) void rotation_products_kernel(const uint64_t *
                 mac(a1[r][g], t[g], k1[r]);
             }
     }
+    if (a.fold.ct && i < L) {
+        const Word pm = word(a.fold.dc[i].p_mod);
+#pragma unroll
+        for (int g = 0; g < RG; g++) {
+            const Word w = word(a.fold.ct[(ct0 + min(g, gv - 1)) * a.fold.ct_stride + ((size_t)i << a.logn) + c]);
+#pragma unroll
+            for (int r = 0; r < R; r++) mac(a0[r][g], w, pm);
+        }
+    }
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        const uint64_t *corr = rb.key[r] + corr_off;
+        const uint64_t *corr = rb.key[r] + a.corr_off;
         const uint64_t c0 = corr[(size_t)i * n + c], c1 = corr[((size_t)(L + 1) + i) * n + c];
 #pragma unroll
         for (int g = 0; g < RG; g++) {
@@ -176,6 +197,99 @@ __global__ __launch_bounds__(TPB) void rotation_products_kernel(const uint64_t *
                 rb.P[r][((ct * 2 + 1) * L + i) * n + c] = r1;
             }
         }
+    }
+}
+
+template <int R, int WG, bool MIXED>
+__global__ __launch_bounds__(TPB) void rotation_products_kernel(RotBatch rb, RotArgs a) {
+    constexpr int PB = TPB / WG;  // positions per block
+    const uint32_t groups = (a.count + RG - 1) / RG, chunks = (groups + WG - 1) / WG;
+    const uint32_t xcd = blockIdx.x & 7, q8 = blockIdx.x >> 3;
+    const uint32_t tile = (q8 / chunks) * 8 + xcd;
+    if (tile >= a.tiles) return;
+    const uint32_t group = (q8 % chunks) * WG + threadIdx.x / PB;
+    const size_t flat = (size_t)tile * PB + threadIdx.x % PB;
+    if (group >= groups || flat >= (size_t)(a.L + 1) << a.logn) return;
+    const uint32_t i = uniform_row(flat, a.logn);
+    const size_t c = flat & (((size_t)1 << a.logn) - 1);
+    const uint32_t ct0 = group * RG;
+    const int gv = (int)min<uint32_t>(RG, a.count - ct0);
+    if constexpr (MIXED) {
+        if (a.targets[i].fwd_fp) {  // uniform
+            rotation_products_core<R, true>(rb, a, i, c, ct0, gv);
+            return;
+        }
+    }
+    rotation_products_core<R, false>(rb, a, i, c, ct0, gv);
+}
+
+// The products of nr rotations; the waves of a block share positions where there are
+// groups enough for them.
+void launch_rotation_products(const RotBatch &rb, RotArgs a, uint32_t nr, bool mixed, hipStream_t st) {
+    const uint32_t groups = (a.count + RG - 1) / RG;
+    uint32_t wg = a.logn < 6 || groups < 2 ? 1 : groups < 4 ? 2 : 4;
+    uint64_t blocks;
+    for (;; wg = 1) {
+        a.tiles = (uint32_t)((((size_t)(a.L + 1) << a.logn) + TPB / wg - 1) / (TPB / wg));
+        blocks = (uint64_t)((a.tiles + 7) / 8) * 8 * ((groups + wg - 1) / wg);
+        if (wg == 1 || blocks * TPB < (uint64_t(1) << 32)) break;
+    }
+    if (blocks * TPB >= (uint64_t(1) << 32)) fail(ERR_INVALID_ARGUMENT, "rotation batch too large for one call");
+    auto go = [&](auto r, auto w) {
+        constexpr int R = decltype(r)::value, WG = decltype(w)::value;
+        if (mixed) rotation_products_kernel<R, WG, true><<<(uint32_t)blocks, TPB, 0, st>>>(rb, a);
+        else rotation_products_kernel<R, WG, false><<<(uint32_t)blocks, TPB, 0, st>>>(rb, a);
+    };
+    auto with_r = [&](auto w) {
+        switch (nr) {
+            case 1: go(std::integral_constant<int, 1>{}, w); break;
+            case 2: go(std::integral_constant<int, 2>{}, w); break;
+            case 3: go(std::integral_constant<int, 3>{}, w); break;
+            default: go(std::integral_constant<int, 4>{}, w); break;
+        }
+    };
+    switch (wg) {
+        case 1: with_r(std::integral_constant<int, 1>{}); break;
+        case 2: with_r(std::integral_constant<int, 2>{}); break;
+        default: with_r(std::integral_constant<int, 4>{}); break;
+    }
+    launch_check("rotation_products");
+}
+
+// The sum over a pass's rotations of their permuted products, Psum[g] (+)= sum_q
+// sigma_q(P_q[g]) for polynomials g < polys of L limbs, and of their rounded special limbs,
+// V[g] (+)= sum_q [S_q[g] + floor(p/2)]_p as whole numbers (at most 15 of them below 2^60):
+// what one ModDown needs for all of them.  HBM: reads each product once.
+struct SumArgs {
+    const uint64_t *P, *S;       // rotation q's at + q * polys limbs * L (1)
+    uint64_t *Psum, *V;
+    uint32_t elt[RMAX];
+    uint64_t p;
+};
+__global__ void sum_products_kernel(SumArgs a, uint32_t nr, const DevPrime *__restrict__ primes, uint32_t L, int logn,
+                                    uint32_t polys, bool first, size_t total) {
+    const uint32_t n = 1u << logn;
+    for (size_t idx = (size_t)blockIdx.x * TPB + threadIdx.x; idx < total; idx += (size_t)gridDim.x * TPB) {
+        const uint32_t r = uniform_row(idx, logn), g = r / (L + 1), i = r - g * (L + 1);
+        const uint32_t off = (uint32_t)(idx & (n - 1));
+        if (i == L) {
+            uint64_t v = first ? 0 : a.V[((size_t)g << logn) + off];
+            for (uint32_t q = 0; q < nr; q++) {
+                const uint64_t s = a.S[((size_t)(q * polys + g) << logn) + off] + (a.p >> 1);
+                v += s >= a.p ? s - a.p : s;
+            }
+            a.V[((size_t)g << logn) + off] = v;
+            continue;
+        }
+        const uint64_t q_i = primes[i].q;
+        const size_t limb = (size_t)g * L + i;
+        uint64_t v = first ? 0 : a.Psum[(limb << logn) + off];
+        const uint32_t rev = __brev(n + off) >> (31 - logn);
+        for (uint32_t q = 0; q < nr; q++) {
+            const uint32_t src = __brev((a.elt[q] * rev >> 1) & (n - 1)) >> (32 - logn);
+            v = addmod(v, a.P[(((size_t)q * polys * L + limb) << logn) + src], q_i);
+        }
+        a.Psum[(limb << logn) + off] = v;
     }
 }
 
@@ -242,14 +356,15 @@ __global__ void clear_words_kernel(unsigned long long *w, size_t words) {
 //   P_r[ct][k][i][s] += sum over zeros (ct, j, p) that sigma_r negates, j's prime not i,
 //                       of (q_j mod q_i) psi_i^((2 brev(s) + 1) p) key'_r[j][k][ki][s],
 // psi_i^((2 brev(s)+1) p) being slot s of NTT_i(X^p); products of a ciphertext whose
-// L N digit words are all zero are set to zero (its exact products).  Exits at once
+// L N digit words are all zero are set to zero (its exact products; p c0 where that is
+// folded in).  Exits at once
 // when the batch has no zero digit.
 template <int R>
 __global__ __launch_bounds__(TPB) void zero_digit_fix_kernel(RotBatch rb, const unsigned long long *__restrict__ zc,
                                                              const uint64_t *__restrict__ list,
                                                              const DevPrime *__restrict__ targets,
                                                              const DevPrime *__restrict__ data, uint32_t L, uint32_t K,
-                                                             int logn, uint32_t count) {
+                                                             int logn, uint32_t count, KsFold fold) {
     const unsigned long long z = zc[0];
     if (z == 0) return;
     const size_t n = (size_t)1 << logn;
@@ -265,8 +380,14 @@ __global__ __launch_bounds__(TPB) void zero_digit_fix_kernel(RotBatch rb, const 
     };
     for (uint32_t ct = 0; ct < count; ct++) {
         if (zc[2 + ct] != all) continue;
+        const uint64_t pc0 = fold.ct && i < L ? mulmod(fold.ct[ct * fold.ct_stride + flat], fold.dc[i].p_mod, Q.q,
+                                                       Q.ratio_lo, Q.ratio_hi)
+                                              : 0;
 #pragma unroll
-        for (int r = 0; r < R; r++) *out(r, ct, 0) = *out(r, ct, 1) = 0;
+        for (int r = 0; r < R; r++) {
+            *out(r, ct, 0) = pc0;
+            *out(r, ct, 1) = 0;
+        }
     }
     const uint64_t two_bs1 = 2 * (uint64_t)(__brev(s) >> (32 - logn)) + 1;
     const size_t kstride = (size_t)K << logn;
@@ -297,21 +418,24 @@ __global__ __launch_bounds__(TPB) void zero_digit_fix_kernel(RotBatch rb, const 
 }
 
 struct RotLayout {
-    size_t gal, tmpct, P2, S2, C0, Pm, Sm, flag, zc, total;
+    size_t ks, list, C0, Pm, Sm, U, S2, flag, zc, total;
 };
 
+// N >= 2^13: a pass's rotations share each launch, so the ModDown's scratch (U, S2) has
+// room for RMAX of them; below, one rotation at a time.
 RotLayout rot_layout(const Context &c, uint32_t count, uint32_t L) {
     const size_t limb = c.n * 8;
     RotLayout l;
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t o = off; off += align256(bytes); return o; };
-    l.gal = take(galois_keyswitch_workspace(c, count, L));
-    l.tmpct = take((size_t)count * 2 * L * limb);
-    l.P2 = take((size_t)count * 2 * L * limb);
-    l.S2 = take((size_t)count * 2 * limb);
+    const size_t m = c.logn >= 13 ? RMAX : 1;
+    l.ks = take(keyswitch_workspace(c, count, L));
+    l.list = take((size_t)count * L * limb);
     l.C0 = take((size_t)count * L * limb);
     l.Pm = take((size_t)RMAX * count * 2 * L * limb);
     l.Sm = take((size_t)RMAX * count * 2 * limb);
+    l.U = take(m * count * 2 * L * limb);
+    l.S2 = take(m * count * 2 * limb);
     l.flag = take(8);
     l.zc = take(8 * (2 + (size_t)count));
     l.total = off;
@@ -384,14 +508,12 @@ void rotate_hoisted(const Context &c, const uint64_t *in, uint32_t count, uint32
     const int logn = c.logn;
     const size_t n = c.n, lw = (size_t)L * n;
     char *base = static_cast<char *>(ws);
-    uint64_t *tmpct = reinterpret_cast<uint64_t *>(base + lay.tmpct);
-    uint64_t *P2 = reinterpret_cast<uint64_t *>(base + lay.P2);
+    uint64_t *list = reinterpret_cast<uint64_t *>(base + lay.list);
+    uint64_t *U = reinterpret_cast<uint64_t *>(base + lay.U);
     uint64_t *S2 = reinterpret_cast<uint64_t *>(base + lay.S2);
     uint64_t *C0 = reinterpret_cast<uint64_t *>(base + lay.C0);
     auto *flag = reinterpret_cast<unsigned long long *>(base + lay.flag);
-    // the hoisted path uses the key-switch regions that follow the Galois scratch row
-    const size_t sigma_bytes = align256((size_t)count * lw * 8);
-    const KsRegions ks = keyswitch_regions(c, count, L, base + lay.gal + sigma_bytes);
+    const KsRegions ks = keyswitch_regions(c, count, L, base + lay.ks);
 
     // each prepared key must be the one of this level and element: checked on the
     // host for keys prepared through this context; other keys' header words are read
@@ -439,22 +561,41 @@ void rotate_hoisted(const Context &c, const uint64_t *in, uint32_t count, uint32
     // 2. zero digits, listed for the products' fix (the list has room for every word)
     auto *zc = reinterpret_cast<unsigned long long *>(base + lay.zc);
     clear_words_kernel<<<1, TPB, 0, st>>>(zc, 2 + (size_t)count);
-    zero_list_kernel<<<blocks_for(count * lw), TPB, 0, st>>>(digits, dstride, L, logn, zc, tmpct, count * lw);
+    zero_list_kernel<<<blocks_for(count * lw), TPB, 0, st>>>(digits, dstride, L, logn, zc, list, count * lw);
     launch_check("zero digits");
     const size_t ct_words = (size_t)count * 2 * lw;
     // 3. one ModUp for every rotation
     const bool skipped = modup_to_T(c, digits, dstride, ks.T, count, L, st, nullptr, ckks);
+    // T words below 4 q_i where the fp64 transforms (N >= 2^13) or full reduction made them
+    const bool acc26 = c.fp_primes;
     const uint64_t *diag = skipped ? in + lw : nullptr;
     const DevPrime *targets = c.keyswitch_primes(L);
     const size_t K = c.key_count();
     const size_t corr_off = (K - 1) * 2 * K * n;
     uint64_t *Pm = reinterpret_cast<uint64_t *>(base + lay.Pm);
     uint64_t *Sm = reinterpret_cast<uint64_t *>(base + lay.Sm);
-    const uint32_t tiles = (uint32_t)((((size_t)(L + 1) << logn) + TPB - 1) / TPB);
-    const uint64_t blocks = (uint64_t)((tiles + 7) / 8) * 8 * ((count + RG - 1) / RG);
-    if (blocks * TPB >= (uint64_t(1) << 32)) fail(ERR_INVALID_ARGUMENT, "rotation batch too large for one call");
-    for (uint32_t r0 = 0; r0 < rotations; r0 += RMAX) {
-        const uint32_t nr = rotations - r0 < (uint32_t)RMAX ? rotations - r0 : (uint32_t)RMAX;
+    // N >= 2^13: c0 joins the products (in NTT form: BFV's c0 is transformed once for all
+    // rotations), the products are permuted as the ModDown reads them, and a pass's
+    // rotations -- or, when summing, up to 15 of them -- take one ModDown
+    const bool batched = logn >= 13;
+    KsFold fold{};
+    if (batched) {
+        fold = KsFold{in, 2 * lw, c.ks_consts()};
+        if (!ckks) {
+            const NttGroup g{C0, in, LimbGrid{1, L, L, count}, LimbGrid{1, 2 * L, L, count}, c.primes()};
+            ntt_forward_groups(&g, 1, logn, NTT_FULL, st);
+            fold = KsFold{C0, lw, c.ks_consts()};
+        }
+    }
+    const RotArgs args{ks.T, corr_off, targets, L, (uint32_t)K, logn, count, 0, diag, 2 * lw, fold};
+    constexpr uint32_t SUM_MAX = 15;  // rotations per summed ModDown (15 words below 2^60)
+    // rotations per pass: RMAX, fewer where one launch cannot hold their limbs
+    uint32_t pass = RMAX;
+    while (batched && pass > 1 && (uint64_t)pass * count * 2 * L > ((uint64_t(1) << 34) >> logn)) pass--;
+    const uint64_t p = c.moduli[K - 1];
+    uint32_t summed = 0;  // rotations in ks.U, ks.S
+    for (uint32_t r0 = 0; r0 < rotations; r0 += pass) {
+        const uint32_t nr = std::min(rotations - r0, pass);
         // products with the prepared keys (corrections included), RMAX rotations per pass over T
         RotBatch rb{};
         for (uint32_t q = 0; q < nr; q++) {
@@ -464,34 +605,60 @@ void rotate_hoisted(const Context &c, const uint64_t *in, uint32_t count, uint32
             rb.elt[q] = elts[r0 + q];
         }
         if (armed && r0 == 0) SHC_HIP(hipEventRecord(probe.begin, st));
-        switch (nr) {
-            case 1: rotation_products_kernel<1><<<(uint32_t)blocks, TPB, 0, st>>>(ks.T, rb, corr_off, targets, L, (uint32_t)K, logn, count, tiles, diag, 2 * lw); break;
-            case 2: rotation_products_kernel<2><<<(uint32_t)blocks, TPB, 0, st>>>(ks.T, rb, corr_off, targets, L, (uint32_t)K, logn, count, tiles, diag, 2 * lw); break;
-            case 3: rotation_products_kernel<3><<<(uint32_t)blocks, TPB, 0, st>>>(ks.T, rb, corr_off, targets, L, (uint32_t)K, logn, count, tiles, diag, 2 * lw); break;
-            default: rotation_products_kernel<4><<<(uint32_t)blocks, TPB, 0, st>>>(ks.T, rb, corr_off, targets, L, (uint32_t)K, logn, count, tiles, diag, 2 * lw); break;
-        }
-        launch_check("rotation_products");
+        launch_rotation_products(rb, args, nr, acc26, st);
         if (armed && r0 == 0) SHC_HIP(hipEventRecord(probe.end, st));
         const uint32_t fix_blocks = (uint32_t)((((size_t)(L + 1) << logn) + TPB - 1) / TPB);
         switch (nr) {
-            case 1: zero_digit_fix_kernel<1><<<fix_blocks, TPB, 0, st>>>(rb, zc, tmpct, targets, c.primes(), L, (uint32_t)K, logn, count); break;
-            case 2: zero_digit_fix_kernel<2><<<fix_blocks, TPB, 0, st>>>(rb, zc, tmpct, targets, c.primes(), L, (uint32_t)K, logn, count); break;
-            case 3: zero_digit_fix_kernel<3><<<fix_blocks, TPB, 0, st>>>(rb, zc, tmpct, targets, c.primes(), L, (uint32_t)K, logn, count); break;
-            default: zero_digit_fix_kernel<4><<<fix_blocks, TPB, 0, st>>>(rb, zc, tmpct, targets, c.primes(), L, (uint32_t)K, logn, count); break;
+            case 1: zero_digit_fix_kernel<1><<<fix_blocks, TPB, 0, st>>>(rb, zc, list, targets, c.primes(), L, (uint32_t)K, logn, count, fold); break;
+            case 2: zero_digit_fix_kernel<2><<<fix_blocks, TPB, 0, st>>>(rb, zc, list, targets, c.primes(), L, (uint32_t)K, logn, count, fold); break;
+            case 3: zero_digit_fix_kernel<3><<<fix_blocks, TPB, 0, st>>>(rb, zc, list, targets, c.primes(), L, (uint32_t)K, logn, count, fold); break;
+            default: zero_digit_fix_kernel<4><<<fix_blocks, TPB, 0, st>>>(rb, zc, list, targets, c.primes(), L, (uint32_t)K, logn, count, fold); break;
         }
         launch_check("zero_digit_fix");
+        if (!batched) {
+            for (uint32_t q = 0; q < nr; q++) {
+                const uint32_t r = r0 + q;
+                uint64_t *dst = sum ? out : out + r * ct_words;
+                // (sigma(c0), 0) into dst (accumulated when summing)
+                apply_galois(c, in, 2 * lw, C0, lw, count, L, elts[r], ckks, st);
+                accumulate_c0_kernel<<<blocks_for(count * lw), TPB, 0, st>>>(dst, C0, c.primes(), L, logn,
+                                                                             !sum || r == 0, count * lw);
+                launch_check("accumulate_c0");
+                // the products permuted by sigma, then this rotation's ModDown added into dst
+                apply_galois(c, rb.P[q], lw, U, lw, count * 2, L, elts[r], true, st);
+                apply_galois(c, rb.S[q], n, S2, n, count * 2, 1, elts[r], true, st);
+                moddown_into(c, U, S2, ks.U, dst, 2 * lw, count, L, st);
+            }
+            continue;
+        }
+        GaloisPerm perm{2 * count, {}};
         for (uint32_t q = 0; q < nr; q++) {
-            const uint32_t r = r0 + q;
-            uint64_t *dst = sum ? out : out + r * ct_words;
-            // (sigma(c0), 0) into dst (accumulated when summing)
-            apply_galois(c, in, 2 * lw, C0, lw, count, L, elts[r], ckks, st);
-            accumulate_c0_kernel<<<blocks_for(count * lw), TPB, 0, st>>>(dst, C0, c.primes(), L, logn,
-                                                                         !sum || r == 0, count * lw);
-            launch_check("accumulate_c0");
-            // the products permuted by sigma, then this rotation's ModDown added into dst
-            apply_galois(c, rb.P[q], lw, P2, lw, count * 2, L, elts[r], true, st);
-            apply_galois(c, rb.S[q], n, S2, n, count * 2, 1, elts[r], true, st);
-            moddown_into(c, P2, S2, ks.U, dst, 2 * lw, count, L, st);
+            if (!(elts[r0 + q] & 1) || elts[r0 + q] >= 2 * n) fail(ERR_INVALID_ARGUMENT, "Galois element is not valid");
+            perm.elt[q] = elts[r0 + q];
+        }
+        const uint32_t polys = 2 * count * nr;
+        ntt_inverse_galois(Sm, LimbGrid{1, 1, 1, polys}, perm, S2, LimbGrid{1, 1, 1, polys}, targets + L, logn, st);
+        ModDownArgs md{S2, Pm, out + r0 * ct_words, 2 * lw, c.ks_consts(), p, L, true};
+        if (!sum) {
+            md.perm = perm;
+            ntt_moddown(ckks, U, md, count * nr, c.primes(), logn, st);
+            continue;
+        }
+        SumArgs sa{Pm, S2, ks.U, ks.S, {}, p};
+        for (uint32_t q = 0; q < nr; q++) sa.elt[q] = elts[r0 + q];
+        const size_t total = (size_t)2 * count * (L + 1) * n;
+        sum_products_kernel<<<blocks_for(total), TPB, 0, st>>>(sa, nr, c.primes(), L, logn, 2 * count, summed == 0, total);
+        launch_check("sum_products");
+        summed += nr;
+        const uint32_t next = std::min(rotations - (r0 + nr), pass);
+        if (!next || summed + next > SUM_MAX) {
+            md.S = ks.S;
+            md.P = ks.U;
+            md.ct = out;
+            md.folded = r0 + nr == summed;  // the first sums write out, later ones add
+            md.presum = summed;
+            ntt_moddown(ckks, ckks ? U : ks.U, md, count, c.primes(), logn, st);
+            summed = 0;
         }
     }
 }

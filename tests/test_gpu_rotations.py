@@ -101,6 +101,26 @@ def test_rotate_sum_many_zero_digits_and_zero_c1(scheme):
     run_case(scheme, 12, [40, 40, 50], 2, 2, [1, 2, -1, 3, 5], zero_digits="heavy", seed=6)
 
 
+@pytest.mark.parametrize("scheme,bits,L,count,rotations", [
+    # N >= 2^13: passes of up to 4 rotations share their launches, a block's waves share
+    # positions from 3 ciphertexts up, one summed ModDown takes up to 15 rotations
+    (CKKS, [60, 40, 50], 2, 1, 1),
+    (CKKS, [60, 40, 50], 2, 9, 5),
+    (CKKS, [50, 45], 1, 4, 16),
+    (CKKS, [60, 55, 60], 2, 3, 17),
+    (BFV, [43, 44, 44], 2, 5, 16),
+    (BFV, [60, 60, 60], 2, 2, 3),
+])
+def test_rotation_passes(scheme, bits, L, count, rotations):
+    run_case(scheme, 13, bits, L, count, list(range(1, rotations + 1)), seed=rotations)
+
+
+@pytest.mark.parametrize("scheme", [CKKS, BFV])
+@pytest.mark.parametrize("zeros", [True, "heavy"])
+def test_rotation_passes_zero_digits(scheme, zeros):
+    run_case(scheme, 13, [60, 40, 50], 2, 2, [1, 2, -1, 3, 5], zero_digits=zeros, seed=8)
+
+
 def test_rotate_sum_in_a_captured_graph():
     """The hoisted rotation sum waits for nothing on the host, so it can be captured: a
     captured call (with zero digits in the batch, so the fix runs) replays to the eager
