@@ -124,4 +124,9 @@ __device__ __forceinline__ uint64_t acc_reduce(const Acc26 &a, const DevPrime &Q
     return barrett128(acc_value(a), Q.q, Q.ratio_lo, Q.ratio_hi);
 }
 
+__device__ __forceinline__ void acc_fold(Acc26 &a, const DevPrime &Q) {
+    const Cut26 r = cut26(acc_reduce(a, Q));
+    a = Acc26{r.lo, r.hi, 0};
+}
+
 }  // namespace shc

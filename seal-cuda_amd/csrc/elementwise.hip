@@ -11,6 +11,7 @@
 // this build follows the GPU path it replaces.
 #include "elementwise.h"
 #include "accum.h"
+#include <type_traits>
 #include "behz.h"
 #include "crypto.h"
 #include "modarith.h"
@@ -205,6 +206,116 @@ __global__ __launch_bounds__(TPB, 3) void plain_dot_many_kernel(const uint64_t *
     }
 }
 
+// The same sums where both outputs and polynomials are many (a batch of diagonal matrix-vector
+// products): a product of small matrices per word position.  A block owns PT positions x
+// 16 outputs x 16 polynomials and stages JC terms at a time in LDS, so that a word is loaded
+// polys / 16 or outputs / 16 times instead of once per 2 or 8 sums: the per-thread form moved
+// 80 GB through L2 for 12 GB of operands (32 terms x 32 outputs x 32 polynomials, N = 2^15,
+// L = 15) and waited for it.  A thread keeps 4 x 4 sums of its position (8 LDS words for 16
+// products); the words of the next JC terms are requested while these are summed.  Primes
+// below 2^50 stage the words cut at 26 bits and sum in Acc26.  That product took 10.2 ms, now
+// 4.8 (12 GB at 2.5 TB/s; 158 VGPRs, three blocks per CU).  32 positions per block (512
+// threads) measured 5.2 ms held to 128 VGPRs (13 spilled) and 5.7 ms without.
+constexpr int PT = 16;           // positions per block (128-byte rows)
+constexpr int DT = 16;           // outputs, and polynomials, per block
+constexpr int JC = 2;            // terms per stage
+constexpr int DB = PT * 16;      // threads: 4 x 4 tiles of 4 x 4 sums per position
+
+struct DotArgs {
+    const uint64_t *cts, *plains;
+    uint64_t *out;
+    const DevPrime *primes;
+    uint32_t terms, outputs, polys, L;
+    int logn;
+    uint32_t tiles, hb, gb;      // position tiles, output and polynomial blocks
+};
+
+template <bool FP>
+__device__ __forceinline__ void plain_dot_tile(uint2 (*lds)[JC][2 * DT][PT], const DotArgs &a, size_t r0,
+                                               const DevPrime &P, uint32_t h0, uint32_t g0) {
+    using Acc = std::conditional_t<FP, Acc26, Acc3>;
+    using Word = std::conditional_t<FP, Cut26, uint64_t>;
+    const size_t lw = (size_t)a.L << a.logn, pw = (size_t)a.polys * lw;
+    const int tid = threadIdx.x, pos = tid % PT, tl = tid / PT;
+    const int th = (tl / 4) * 4, tg = (tl % 4) * 4;  // this thread's 4 x 4 sums
+    // loads: row tl (< 16) of the outputs' plaintexts and of the polynomials, per term
+    const uint64_t *pp = a.plains + (size_t)min(h0 + tl, a.outputs - 1) * a.terms * lw + r0 + pos;
+    const uint64_t *cp = a.cts + (size_t)min(g0 + tl, a.polys - 1) * lw + r0 + pos;
+    uint64_t nx[2 * JC];
+    auto request = [&](uint32_t j0) {
+#pragma unroll
+        for (int k = 0; k < JC; k++) {
+            const size_t j = min<uint32_t>(j0 + k, a.terms - 1);
+            nx[2 * k] = pp[j * lw];
+            nx[2 * k + 1] = cp[j * pw];
+        }
+    };
+    auto cut = [](uint64_t x) -> uint2 {
+        if constexpr (FP) {
+            const Cut26 c = cut26(x);
+            return uint2{c.lo, c.hi};
+        }
+        return uint2{(uint32_t)x, (uint32_t)(x >> 32)};
+    };
+    auto word = [](uint2 w) -> Word {
+        if constexpr (FP) return Cut26{w.x, w.y};
+        else return (uint64_t)w.y << 32 | w.x;
+    };
+    Acc acc[4][4];
+#pragma unroll
+    for (int h = 0; h < 4; h++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) acc[h][g] = Acc{0, 0, 0};
+    request(0);
+    for (uint32_t j0 = 0, b = 0; j0 < a.terms; j0 += JC, b ^= 1) {
+        // two buffers: the barrier of the stage before has passed its readers of this one
+#pragma unroll
+        for (int k = 0; k < JC; k++) {
+            lds[b][k][tl][pos] = cut(nx[2 * k]);
+            lds[b][k][DT + tl][pos] = cut(nx[2 * k + 1]);
+        }
+        __syncthreads();
+        if (j0 + JC < a.terms) request(j0 + JC);
+#pragma unroll 1
+        for (int k = 0; k < JC; k++) {
+            if (j0 + k >= a.terms) break;  // uniform
+            Word w[4], t[4];
+#pragma unroll
+            for (int x = 0; x < 4; x++) w[x] = word(lds[b][k][th + x][pos]), t[x] = word(lds[b][k][DT + tg + x][pos]);
+#pragma unroll
+            for (int h = 0; h < 4; h++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) mac(acc[h][g], t[g], w[h]);
+        }
+        if ((j0 & 63) + JC == 64) {
+#pragma unroll
+            for (int h = 0; h < 4; h++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) acc_fold(acc[h][g], P);
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < 4; h++)
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+            if (h0 + th + h < a.outputs && g0 + tg + g < a.polys)
+                a.out[(size_t)(h0 + th + h) * pw + (size_t)(g0 + tg + g) * lw + r0 + pos] = acc_reduce(acc[h][g], P);
+}
+
+__global__ __launch_bounds__(DB, 3) void plain_dot_tiles_kernel(DotArgs a) {
+    __shared__ uint2 lds[2][JC][2 * DT][PT];
+    // the blocks of one position tile run one after another on one XCD (block % 8), whose L2
+    // serves the words they share
+    const uint32_t subs = a.hb * a.gb, k = blockIdx.x >> 3;
+    const uint32_t tile = k / subs * 8 + (blockIdx.x & 7), sub = k % subs;
+    if (tile >= a.tiles) return;  // uniform
+    const size_t r0 = (size_t)tile * PT;
+    const DevPrime &P = a.primes[r0 >> a.logn];
+    const uint32_t h0 = sub / a.gb * DT, g0 = sub % a.gb * DT;
+    if (P.fwd_fp) plain_dot_tile<true>(lds, a, r0, P, h0, g0);
+    else plain_dot_tile<false>(lds, a, r0, P, h0, g0);
+}
+
 template <int H>
 void launch_plain_dot(uint32_t G, const uint64_t *cts, const uint64_t *plains, uint64_t *out, const DevPrime *primes,
                       uint32_t terms, uint32_t h0, uint32_t hn, uint32_t polys, uint32_t L, int logn, hipStream_t st) {
@@ -312,6 +423,17 @@ void multiply_plain_accumulate_many(const Context &c, const uint64_t *cts, const
     const uint32_t G = polys >= 2 ? 2 : 1;
     const DevPrime *primes = c.primes();
     const int logn = c.logn;
+    // tiles of 16 outputs x 16 polynomials where both are at least half of one (below, a
+    // tile's idle sums cost more than the per-thread form's repeated loads)
+    const uint64_t tiles = ((uint64_t)L << logn) / PT;
+    const uint64_t tile_blocks = (tiles + 7) / 8 * 8 * ((outputs + DT - 1) / DT) * ((polys + DT - 1) / DT);
+    if (polys >= DT / 2 && outputs >= DT / 2 && logn >= 5 && tile_blocks < (uint64_t(1) << 32) / DB) {
+        const DotArgs a{cts, plains, out, primes, terms, outputs, polys, L, logn, (uint32_t)tiles,
+                        (outputs + DT - 1) / DT, (polys + DT - 1) / DT};
+        plain_dot_tiles_kernel<<<(uint32_t)tile_blocks, DB, 0, st>>>(a);
+        launch_check("plain_dot_tiles");
+        return;
+    }
     for (uint32_t h0 = 0; h0 < outputs;) {
         const uint32_t left = outputs - h0;
         const uint32_t hn = left >= 8 ? 8 : left;

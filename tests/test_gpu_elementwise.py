@@ -138,6 +138,30 @@ def test_plain_ops_reject_bad_arguments():
         ctx.bfv_add_plain(d.data_ptr(), d.data_ptr(), d.data_ptr(), 1, 2, 2, False, stream())   # CKKS context
 
 
+@pytest.mark.parametrize("terms,outputs,polys,logn", [
+    (1, 8, 8, 5), (3, 16, 16, 10), (2, 17, 15, 11), (65, 9, 33, 10), (130, 33, 8, 6), (64, 16, 17, 12)])
+@pytest.mark.parametrize("words", ["uniform", "largest"])
+def test_plain_dot_tiles(terms, outputs, polys, logn, words):
+    """Tiles of 16 outputs x 16 polynomials (edges, odd stage counts, folds every 64 terms,
+    integer and fp64 primes) against the same sums one output at a time (the per-thread
+    kernel, checked against the oracle below)."""
+    L, n = 3, 1 << logn
+    moduli = ck.coeff_modulus_create(n, [60, 50, 40, 60])
+    ctx = hip().Context(CKKS, n, moduli)
+    rng = np.random.default_rng(terms)
+    cts = ck.uniform_residues(rng, (terms, polys, L, n), moduli[:L])
+    plains = ck.uniform_residues(rng, (outputs, terms, L, n), moduli[:L])
+    if words == "largest":
+        q = np.array(moduli[:L], dtype=np.uint64)[:, None]
+        cts[:], plains[:] = q - 1, q - 1
+    dc, dp = to_dev(cts), to_dev(plains)
+    out, each = empty_dev((outputs, polys, L, n)), empty_dev((outputs, polys, L, n))
+    ctx.multiply_plain_accumulate_many(dc.data_ptr(), dp.data_ptr(), terms, outputs, polys, L, out.data_ptr(), stream())
+    for o in range(outputs):
+        ctx.multiply_plain_accumulate(dc.data_ptr(), dp[o].data_ptr(), terms, polys, L, each[o].data_ptr(), stream())
+    np.testing.assert_array_equal(from_dev(out), from_dev(each))
+
+
 @pytest.mark.parametrize("scheme,terms,outputs,polys,logn", [
     (CKKS, 70, 11, 4, 10), (BFV, 5, 2, 4, 10),
     (CKKS, 3, 3, 6, 10),    # a partial group of polynomials (4 + 2)
