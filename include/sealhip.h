@@ -467,6 +467,16 @@ int shc_rotate_many(const shc_context *ctx, const uint64_t *d_in, uint32_t count
                     const uint64_t *const *d_galois_keys, uint32_t rotations, uint64_t *d_out, void *d_workspace,
                     size_t workspace_bytes, void *stream);
 
+/* d_out[c] = sum_h rotate_{galois_elts[h]}(d_in[h][c]) for h < n, d_in
+ * [n][count][2][L][N] (not overlapping d_out): the words of separate
+ * shc_apply_galois_keyswitch calls summed, with one ModDown for up to 15 of them -- the
+ * giant steps of a BSGS matrix-vector product.  An element of 1 adds d_in[h] as it is (its
+ * key may be NULL); d_galois_keys is a host array of device pointers. */
+int shc_rotate_accumulate_workspace_size(const shc_context *ctx, uint32_t count, uint32_t limb_count, size_t *bytes);
+int shc_rotate_accumulate(const shc_context *ctx, const uint64_t *d_in, uint32_t count, uint32_t limb_count,
+                          const uint32_t *galois_elts, const uint64_t *const *d_galois_keys, uint32_t n,
+                          uint64_t *d_out, void *d_workspace, size_t workspace_bytes, void *stream);
+
 /* Instrumentation (no counterpart in the reference; for benchmarks and profilers):
  * arms `ctx` so that its next key switch (shc_relinearize, shc_switch_key,
  * shc_apply_galois_keyswitch) records the caller-created hipEvent_t `begin_event`

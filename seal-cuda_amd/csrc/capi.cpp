@@ -745,6 +745,21 @@ int shc_rotate_many(const shc_context *ctx, const uint64_t *in, uint32_t count, 
     });
 }
 
+int shc_rotate_accumulate_workspace_size(const shc_context *ctx, uint32_t count, uint32_t limbs, size_t *bytes) {
+    return guarded([&] {
+        if (!bytes) shc::fail(shc::ERR_INVALID_ARGUMENT, "null argument");
+        *bytes = shc::rotate_accumulate_workspace(ctx_of(ctx), count, limbs);
+    });
+}
+
+int shc_rotate_accumulate(const shc_context *ctx, const uint64_t *in, uint32_t count, uint32_t limbs,
+                          const uint32_t *elts, const uint64_t *const *keys, uint32_t n, uint64_t *out, void *ws,
+                          size_t ws_bytes, void *stream) {
+    return guarded([&] {
+        shc::rotate_accumulate(ctx_of(ctx), in, count, limbs, elts, keys, n, out, ws, ws_bytes, (hipStream_t)stream);
+    });
+}
+
 int shc_multiply_plain_accumulate(const shc_context *ctx, const uint64_t *cts, const uint64_t *plains, uint32_t terms,
                                   uint32_t polys, uint32_t limbs, uint64_t *out, void *stream) {
     return guarded([&] {

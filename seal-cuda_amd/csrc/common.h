@@ -59,6 +59,14 @@ __device__ __forceinline__ uint32_t uniform_row(size_t idx, int logn) {
     return logn >= 6 ? __builtin_amdgcn_readfirstlane(r) : r;
 }
 
+// Slot of x that NTT-form sigma_elt(x) holds at slot off: 2 brev(src) + 1 =
+// elt (2 brev(off) + 1) mod 2N (GaloisTool's permutation table, computed in registers).
+__device__ __forceinline__ uint32_t galois_slot(uint32_t off, uint32_t elt, int logn) {
+    const uint32_t n = 1u << logn;
+    const uint32_t rev = __brev(n + off) >> (31 - logn);
+    return __brev((elt * rev >> 1) & (n - 1)) >> (32 - logn);
+}
+
 // Error raised by host code; carries the exception family of the reference
 // (std::invalid_argument / logic_error / out_of_range / runtime_error).
 enum ErrKind { ERR_OK = 0, ERR_INVALID_ARGUMENT = -1, ERR_LOGIC = -2, ERR_OUT_OF_RANGE = -3, ERR_RUNTIME = -4,

@@ -27,7 +27,7 @@ __device__ __forceinline__ uint64_t moddown_u(const ModDownArgs &a, uint32_t i, 
 // Word (limb i of polynomial j, coefficient off) of a ModDown's P.
 template <int LOGN>
 __device__ __forceinline__ uint64_t moddown_p(const ModDownArgs &a, uint32_t i, uint32_t j, size_t off) {
-    if (a.perm.polys) off = galois_slot<LOGN>(off, a.perm.elt[j / a.perm.polys]);  // uniform
+    if (a.perm.polys) off = galois_slot((uint32_t)off, a.perm.elt[j / a.perm.polys], LOGN);  // uniform
     if (a.p_lpp)  // uniform
         return a.P[(size_t)(j >> 1) * a.p_ct_stride + ((size_t)((j & 1) * a.p_lpp + i) << LOGN) + off];
     return a.P[((size_t)(j * a.L + i) << LOGN) + off];
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(SUBS << (K - E)) void ntt_rows_galois_kernel(const 
     rows_body<LOGN, K, E, SUBS, true, false, MX>(
         blockIdx.x, primes, lg.I, 0, lg.J,
         [&](uint32_t i, uint32_t j, size_t off) {
-            return *s.at(i, j, galois_slot<LOGN>(off, perm.elt[j / perm.polys]));
+            return *s.at(i, j, galois_slot((uint32_t)off, perm.elt[j / perm.polys], LOGN));
         },
         [&](uint32_t i, uint32_t j, size_t off, uint64_t x) { *g.at(i, j, off) = x; });
 }

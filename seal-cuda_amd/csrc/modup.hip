@@ -176,8 +176,9 @@ __device__ __forceinline__ void rows_keyprod_core(
         for (int c = 0; c < NS; c++) {
             const Word k0 = word(kp[(2 * i) * kstride + (c / CG) * SZ]);
             const Word k1 = word(kp[(2 * i + 1) * kstride + (c / CG) * SZ]);
+            const size_t off = row_off(c / CG) + tid;
             const Word x = word(diag[(ct0 + min<uint32_t>(c % CG, gv - 1)) * diag_stride + ((size_t)i << LOGN) +
-                                     row_off(c / CG) + tid]);
+                                     (fold.diag_elt ? galois_slot((uint32_t)off, fold.diag_elt, LOGN) : off)]);
             mac(a0[c], x, k0);
             mac(a1[c], x, k1);
         }

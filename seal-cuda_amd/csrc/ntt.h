@@ -68,6 +68,7 @@ struct KsFold {
     size_t ct_stride;
     const DivRoundConst *dc;
     bool c1_zero = false;
+    uint32_t diag_elt = 0;
 };
 bool ntt_modup_keyprod(const uint64_t *d, size_t d_ct_stride, uint64_t *T, const uint64_t *key, uint64_t *P,
                        uint64_t *S, const uint64_t *diag, size_t diag_stride, uint32_t count, uint32_t L,

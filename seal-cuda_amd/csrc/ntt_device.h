@@ -389,16 +389,6 @@ __global__ __launch_bounds__(SUBS << (K - E)) void ntt_cols_kernel(uint64_t *__r
         });
 }
 
-// Word of NTT-form sigma_elt(x) at slot off: slot src of x, where 2 brev(src) + 1 =
-// elt (2 brev(off) + 1) mod 2N (GaloisTool's permutation table, computed in registers).
-template <int LOGN>
-__device__ __forceinline__ size_t galois_slot(size_t off, uint32_t elt) {
-    const uint32_t n = 1u << LOGN;
-    const uint32_t rev = __brev(n + (uint32_t)off) >> (31 - LOGN);
-    const uint32_t raw = (elt * rev >> 1) & (n - 1);
-    return __brev(raw) >> (32 - LOGN);
-}
-
 // Block prefix table of a grouped launch; sizes[g] blocks for group g.
 template <class Table>
 uint32_t fill_starts(Table &t, const std::vector<uint64_t> &sizes) {

@@ -2,6 +2,7 @@
 #pragma once
 #include "common.h"
 #include "context.h"
+#include "ntt.h"
 
 namespace shc {
 
@@ -54,6 +55,15 @@ bool modup_to_T(const Context &c, const uint64_t *digits, size_t dstride, uint64
 void keyswitch_inner_product(const Context &c, const uint64_t *T, const uint64_t *key, uint64_t *P, uint64_t *S,
                              uint32_t count, uint32_t L, hipStream_t st, const uint64_t *diag = nullptr,
                              size_t diag_stride = 0);
+// The same for a batch under several keys (at most PERM_MAX): ciphertext ct takes key
+// ct / per, and with elt != 0 its own-prime words diag through sigma_elt (NTT form).
+struct InnerKeys {
+    const uint64_t *key[PERM_MAX];
+    uint32_t elt[PERM_MAX];
+    uint32_t n, per;
+};
+void keyswitch_inner_products(const Context &c, const uint64_t *T, const InnerKeys &keys, uint64_t *P, uint64_t *S,
+                              uint32_t L, hipStream_t st, const uint64_t *diag, size_t diag_stride);
 void moddown_into(const Context &c, uint64_t *P, uint64_t *S, uint64_t *U, uint64_t *ct, size_t ct_stride,
                   uint32_t count, uint32_t L, hipStream_t st, bool folded = false);
 

@@ -22,6 +22,7 @@
 #include "modarith.h"
 #include "ntt.h"
 #include "rns_ops.h"
+#include <type_traits>
 #include <vector>
 
 namespace shc {
@@ -86,42 +87,39 @@ __global__ void modup_gather_kernel(const uint64_t *__restrict__ d, size_t d_str
 // Blocks are dealt to the 8 XCDs round-robin (XCD = block % 8); the mapping below puts
 // every group of one tile on the same XCD, one after another, so the tile's key words
 // come from HBM once and then from that XCD's L2.
-template <int G>
-__global__ __launch_bounds__(TPB) void inner_product_kernel(const uint64_t *__restrict__ T,
-                                                            const uint64_t *__restrict__ key,
-                                                            uint64_t *__restrict__ P, uint64_t *__restrict__ S,
-                                                            const DevPrime *__restrict__ targets, uint32_t L,
-                                                            uint32_t K, int logn, uint32_t count, uint32_t tiles,
-                                                            uint32_t groups, const uint64_t *__restrict__ diag,
-                                                            size_t diag_stride) {
-    const uint32_t xcd = blockIdx.x & 7, k = blockIdx.x >> 3;
-    const uint32_t tile = (k / groups) * 8 + xcd;
-    if (tile >= tiles) return;
-    const uint32_t grp = k % groups;
+// Several keys (a batch of `per` ciphertexts under each, as InnerKeys lists them) share a
+// launch: ciphertext ct takes key ct / per, and its own-prime words, with elt != 0, through
+// the permutation sigma_elt.  Targets below 2^50 (their T words are below 4 q) sum in Acc26.
+template <int G, bool FP>
+__device__ __forceinline__ void inner_product_core(const uint64_t *__restrict__ T, const uint64_t *__restrict__ key,
+                                                   uint32_t elt, uint64_t *__restrict__ P, uint64_t *__restrict__ S,
+                                                   const DevPrime &Q, uint32_t i, size_t c, uint32_t L, uint32_t K,
+                                                   int logn, uint32_t count, size_t ct0, int g_valid,
+                                                   const uint64_t *__restrict__ diag, size_t diag_stride) {
+    using Acc = std::conditional_t<FP, Acc26, Acc3>;
+    using Word = std::conditional_t<FP, Cut26, uint64_t>;
+    auto word = [](uint64_t x) -> Word {
+        if constexpr (FP) return cut26(x);
+        else return x;
+    };
     const size_t n = (size_t)1 << logn;
-    const size_t flat = (size_t)tile * TPB + threadIdx.x;
-    if (flat >= (size_t)(L + 1) << logn) return;
-    const uint32_t i = (uint32_t)(flat >> logn);
-    const size_t c = flat & (n - 1);
     const uint32_t ki = (i == L) ? K - 1 : i;
-    const DevPrime &Q = targets[i];
-    const size_t ct0 = (size_t)grp * G;
-    const int g_valid = (int)min<size_t>(G, count - ct0);
     const bool short_row = diag && i < L;  // uniform over the block
     const uint32_t Lt = short_row ? L - 1 : L;
     const uint64_t *Ti = T + (((size_t)i * count * L + ct0 * Lt) << logn) + c;
     const uint64_t *kp = key + (size_t)ki * n + c;
     const size_t kstride = (size_t)K << logn;  // key[j][k] -> key[j][k+1]
+    const size_t cd = elt ? galois_slot((uint32_t)c, elt, logn) : c;
     size_t goff[G];
     const uint64_t *dp[G];
 #pragma unroll
     for (int g = 0; g < G; g++) {
         goff[g] = ((size_t)min(g, g_valid - 1) * Lt) << logn;
-        dp[g] = short_row ? diag + (ct0 + min(g, g_valid - 1)) * diag_stride + ((size_t)i << logn) + c : nullptr;
+        dp[g] = short_row ? diag + (ct0 + min(g, g_valid - 1)) * diag_stride + ((size_t)i << logn) + cd : nullptr;
     }
-    Acc3 acc0[G], acc1[G];
+    Acc acc0[G], acc1[G];
 #pragma unroll
-    for (int g = 0; g < G; g++) acc0[g] = acc1[g] = Acc3{0, 0, 0};
+    for (int g = 0; g < G; g++) acc0[g] = acc1[g] = Acc{0, 0, 0};
     // two digits in flight: buffer b holds digit j while the loads of digit j + 2 go out
     uint64_t tb[2][G], kb[2][2];
     auto fetch = [&](int b, uint32_t j) {
@@ -134,10 +132,10 @@ __global__ __launch_bounds__(TPB) void inner_product_kernel(const uint64_t *__re
         for (int g = 0; g < G; g++) tb[b][g] = *(dj ? dp[g] : Ti + goff[g] + (jt << logn));
     };
     auto step = [&](int b, uint32_t jnext) {
-        uint64_t t[G];
+        Word t[G];
 #pragma unroll
-        for (int g = 0; g < G; g++) t[g] = tb[b][g];
-        const uint64_t k0 = kb[b][0], k1 = kb[b][1];
+        for (int g = 0; g < G; g++) t[g] = word(tb[b][g]);
+        const Word k0 = word(kb[b][0]), k1 = word(kb[b][1]);
         fetch(b, jnext);
 #pragma unroll
         for (int g = 0; g < G; g++) {
@@ -168,6 +166,37 @@ __global__ __launch_bounds__(TPB) void inner_product_kernel(const uint64_t *__re
             }
         }
     }
+}
+
+template <int G, bool MIXED>
+__global__ __launch_bounds__(TPB) void inner_product_kernel(const uint64_t *__restrict__ T, InnerKeys ks,
+                                                            uint64_t *__restrict__ P, uint64_t *__restrict__ S,
+                                                            const DevPrime *__restrict__ targets, uint32_t L,
+                                                            uint32_t K, int logn, uint32_t count, uint32_t tiles,
+                                                            uint32_t groups, const uint64_t *__restrict__ diag,
+                                                            size_t diag_stride) {
+    const uint32_t xcd = blockIdx.x & 7, k = blockIdx.x >> 3;
+    const uint32_t tile = (k / groups) * 8 + xcd;
+    if (tile >= tiles) return;
+    const uint32_t grp = k % groups, per_key = groups / ks.n, h = grp / per_key;
+    const size_t n = (size_t)1 << logn;
+    const size_t flat = (size_t)tile * TPB + threadIdx.x;
+    if (flat >= (size_t)(L + 1) << logn) return;
+    const uint32_t i = (uint32_t)(flat >> logn);
+    const size_t c = flat & (n - 1);
+    const uint32_t g0 = (grp - h * per_key) * G;
+    const size_t ct0 = (size_t)h * ks.per + g0;
+    const int g_valid = (int)min<uint32_t>(G, ks.per - g0);
+    const DevPrime &Q = targets[i];
+    if constexpr (MIXED) {
+        if (Q.fwd_fp) {  // uniform over the block where N >= TPB, else per lane
+            inner_product_core<G, true>(T, ks.key[h], ks.elt[h], P, S, Q, i, c, L, K, logn, count, ct0, g_valid, diag,
+                                        diag_stride);
+            return;
+        }
+    }
+    inner_product_core<G, false>(T, ks.key[h], ks.elt[h], P, S, Q, i, c, L, K, logn, count, ct0, g_valid, diag,
+                                 diag_stride);
 }
 
 // U[g][i][c] = ([S[g][c] + floor(p/2)]_p mod q_i - floor(p/2) mod q_i) mod q_i
@@ -467,15 +496,27 @@ bool modup_to_T(const Context &c, const uint64_t *digits, size_t dstride, uint64
 
 void keyswitch_inner_product(const Context &c, const uint64_t *T, const uint64_t *key, uint64_t *P, uint64_t *S,
                              uint32_t count, uint32_t L, hipStream_t st, const uint64_t *diag, size_t diag_stride) {
+    InnerKeys ks{};
+    ks.key[0] = key;
+    ks.n = 1;
+    ks.per = count;
+    keyswitch_inner_products(c, T, ks, P, S, L, st, diag, diag_stride);
+}
+
+void keyswitch_inner_products(const Context &c, const uint64_t *T, const InnerKeys &ks, uint64_t *P, uint64_t *S,
+                              uint32_t L, hipStream_t st, const uint64_t *diag, size_t diag_stride) {
     constexpr int G = 4;
     const int logn = c.logn;
-    const uint32_t groups = (count + G - 1) / G;
+    const uint32_t groups = ks.n * ((ks.per + G - 1) / G);
     const uint32_t tiles = (uint32_t)((((size_t)(L + 1) << logn) + TPB - 1) / TPB);
     const uint64_t ip_blocks = (uint64_t)((tiles + 7) / 8) * 8 * groups;
     if (ip_blocks * TPB >= (uint64_t(1) << 32)) fail(ERR_INVALID_ARGUMENT, "key-switch batch too large");
-    inner_product_kernel<G><<<(uint32_t)ip_blocks, TPB, 0, st>>>(T, key, P, S, c.keyswitch_primes(L), L,
-                                                                (uint32_t)c.key_count(), logn, count, tiles, groups,
-                                                                diag, diag_stride);
+    auto go = [&](auto kernel) {
+        kernel<<<(uint32_t)ip_blocks, TPB, 0, st>>>(T, ks, P, S, c.keyswitch_primes(L), L, (uint32_t)c.key_count(), logn,
+                                                    ks.n * ks.per, tiles, groups, diag, diag_stride);
+    };
+    if (c.fp_primes) go(inner_product_kernel<G, true>);
+    else go(inner_product_kernel<G, false>);
     launch_check("inner_product");
 }
 

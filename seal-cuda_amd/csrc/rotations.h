@@ -29,4 +29,12 @@ void rotate_many(const Context &c, const uint64_t *in, uint32_t count, uint32_t 
                  const uint64_t *const *hoisted, const uint64_t *const *keys, uint32_t rotations, uint64_t *out,
                  void *ws, size_t ws_bytes, hipStream_t st);
 
+// out[ct] = sum_h rotate_{elts[h]}(in[h][ct]), in: [n][count][2][L][N] (elts[h] == 1: in[h]
+// itself, no key), with the words of separate apply_galois_keyswitch calls summed, and one
+// ModDown for up to 15 of them: the giant steps of a BSGS matrix-vector product.
+size_t rotate_accumulate_workspace(const Context &c, uint32_t count, uint32_t L);
+void rotate_accumulate(const Context &c, const uint64_t *in, uint32_t count, uint32_t L, const uint32_t *elts,
+                       const uint64_t *const *keys, uint32_t n, uint64_t *out, void *ws, size_t ws_bytes,
+                       hipStream_t st);
+
 }  // namespace shc

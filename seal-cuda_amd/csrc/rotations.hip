@@ -677,4 +677,206 @@ void rotate_many(const Context &c, const uint64_t *in, uint32_t count, uint32_t 
     rotate_hoisted(c, in, count, L, elts, hoisted, keys, rotations, out, ws, ws_bytes, st, false);
 }
 
+// ---- sums of rotations of different ciphertexts --------------------------------------
+namespace {
+
+// The c0 part of a rotation sum, and the ciphertexts that stay as they are:
+//   out[ct][0] (+)= sum_h sigma_h(in[h][ct][0]),  out[ct][1] (+)= sum_{h: elt 1} in[h][ct][1]
+constexpr uint32_t C0_MAX = 16;
+struct SumC0Args {
+    const uint64_t *in;   // [n][count][2][L][N]
+    uint64_t *out;        // [count][2][L][N]
+    uint32_t elt[C0_MAX], elt_inv[C0_MAX];
+    uint32_t n, count, L;
+    int logn;
+    bool first;
+};
+template <bool NTT>
+__global__ void sum_c0_kernel(SumC0Args a, const DevPrime *__restrict__ primes, size_t total) {
+    const uint32_t n = 1u << a.logn;
+    const size_t lw = (size_t)a.L << a.logn, ctw = 2 * lw;
+    for (size_t idx = (size_t)blockIdx.x * TPB + threadIdx.x; idx < total; idx += (size_t)gridDim.x * TPB) {
+        const uint32_t r = uniform_row(idx, a.logn), ct = r / a.L, i = r - ct * a.L;
+        const uint32_t off = (uint32_t)(idx & (n - 1));
+        const uint64_t q = primes[i].q;
+        const size_t limb = (size_t)ct * ctw + ((size_t)i << a.logn);
+        uint64_t v0 = a.first ? 0 : a.out[limb + off], v1 = a.first ? 0 : a.out[limb + lw + off];
+        for (uint32_t h = 0; h < a.n; h++) {
+            const uint64_t *src = a.in + (size_t)h * a.count * ctw + limb;
+            const uint32_t e = a.elt[h];
+            uint64_t x;
+            if constexpr (NTT) {
+                x = src[galois_slot(off, e, a.logn)];
+            } else {
+                const uint32_t k = (uint32_t)(((uint64_t)off * a.elt_inv[h]) & (n - 1));
+                x = src[k];
+                if (((uint64_t)k * e >> a.logn) & 1) x = negmod(x, q);
+            }
+            v0 = addmod(v0, x, q);
+            if (e == 1) v1 = addmod(v1, src[lw + off], q);
+        }
+        a.out[limb + off] = v0;
+        a.out[limb + lw + off] = v1;
+    }
+}
+
+// d[h][ct][i] = sigma_h(in[h][ct][1][i]) in coefficient form, h < n (at most PERM_MAX).
+__global__ void galois_digits_kernel(SumC0Args a, uint64_t *__restrict__ d, const DevPrime *__restrict__ primes,
+                                     size_t total) {
+    const uint32_t n = 1u << a.logn;
+    for (size_t idx = (size_t)blockIdx.x * TPB + threadIdx.x; idx < total; idx += (size_t)gridDim.x * TPB) {
+        const uint32_t r = uniform_row(idx, a.logn), g = r / a.L, i = r - g * a.L, h = g / a.count;
+        const uint32_t off = (uint32_t)(idx & (n - 1));
+        const uint32_t k = (uint32_t)(((uint64_t)off * a.elt_inv[h]) & (n - 1));
+        uint64_t x = a.in[(((size_t)g * 2 + 1) * a.L + i << a.logn) + k];
+        if (((uint64_t)k * a.elt[h] >> a.logn) & 1) x = negmod(x, primes[i].q);
+        d[idx] = x;
+    }
+}
+
+struct AccLayout {
+    bool batched;   // else one rotation at a time through tmp
+    uint32_t nb;    // rotations per batch
+    size_t d, T, P, S, Psum, V, U, tmp, total;
+};
+
+// N = 2^15, 2^16: the fused key products take one rotation's T at a time; other degrees a
+// batch's.
+AccLayout acc_layout(const Context &c, uint32_t count, uint32_t L) {
+    const size_t limb = c.n * 8;
+    AccLayout l{};
+    size_t off = 0;
+    auto take = [&](size_t limbs) { size_t o = off; off += align256(limbs * limb); return o; };
+    const uint64_t most = (uint64_t(1) << 34) >> c.logn, per = (uint64_t)count * L * (L + 1);
+    l.batched = c.logn >= 13 && per <= most;
+    if (!l.batched) {
+        l.tmp = take((size_t)count * 2 * L);
+        off += galois_keyswitch_workspace(c, count, L);
+        l.total = off;
+        return l;
+    }
+    const bool fused = c.logn == 15 || c.logn == 16;
+    l.nb = PERM_MAX;
+    while (l.nb > 1 && l.nb * per > most) l.nb--;
+    l.d = take((size_t)l.nb * count * L);
+    l.T = take((fused ? 1 : l.nb) * (size_t)count * L * (L + 1));
+    l.P = take((size_t)l.nb * count * 2 * L);
+    l.S = take((size_t)l.nb * count * 2);
+    l.Psum = take((size_t)count * 2 * L);
+    l.V = take((size_t)count * 2);
+    l.U = take((size_t)count * 2 * L);
+    l.total = off;
+    return l;
+}
+
+}  // namespace
+
+size_t rotate_accumulate_workspace(const Context &c, uint32_t count, uint32_t L) {
+    return acc_layout(c, count, L).total;
+}
+
+void rotate_accumulate(const Context &c, const uint64_t *in, uint32_t count, uint32_t L, const uint32_t *elts,
+                       const uint64_t *const *keys, uint32_t n, uint64_t *out, void *ws, size_t ws_bytes,
+                       hipStream_t st) {
+    check_level(c, L);
+    if (!count) return;
+    if (!n || !elts || !keys) fail(ERR_INVALID_ARGUMENT, "no rotations given");
+    if (in == out) fail(ERR_INVALID_ARGUMENT, "rotate_accumulate cannot run in place");
+    const AccLayout lay = acc_layout(c, count, L);
+    if (!ws || ws_bytes < lay.total) fail(ERR_INVALID_ARGUMENT, "workspace too small for rotation sums");
+    const size_t N = c.n, lw = (size_t)L * N, ctw = 2 * lw, step = (size_t)count * ctw;
+    for (uint32_t h = 0; h < n; h++) {
+        if (!(elts[h] & 1) || elts[h] >= 2 * N) fail(ERR_INVALID_ARGUMENT, "Galois element is not valid");
+        if (elts[h] != 1 && !keys[h]) fail(ERR_INVALID_ARGUMENT, "null key pointer");
+    }
+    char *base = static_cast<char *>(ws);
+    auto at = [base](size_t off) { return reinterpret_cast<uint64_t *>(base + off); };
+    const bool ckks = c.scheme == SCHEME_CKKS;
+    const int logn = c.logn;
+    if (!lay.batched) {
+        uint64_t *tmp = at(lay.tmp);
+        char *gws = base + align256(step * 8);
+        for (uint32_t h = 0; h < n; h++) {
+            uint64_t *dst = h ? tmp : out;
+            SHC_HIP(hipMemcpyAsync(dst, in + h * step, step * 8, hipMemcpyDeviceToDevice, st));
+            if (elts[h] != 1)
+                apply_galois_keyswitch(c, dst, count, L, elts[h], keys[h], gws, ws_bytes - (gws - base), st);
+            if (h) poly_add(c, out, tmp, out, count * 2, L, st);
+        }
+        return;
+    }
+    SumC0Args ca{in, out, {}, {}, 0, count, L, logn, true};
+    for (uint32_t h0 = 0; h0 < n; h0 += C0_MAX) {
+        ca.in = in + h0 * step;
+        ca.n = std::min(n - h0, C0_MAX);
+        ca.first = h0 == 0;
+        for (uint32_t h = 0; h < ca.n; h++) {
+            ca.elt[h] = elts[h0 + h];
+            ca.elt_inv[h] = (uint32_t)hm::invmod(elts[h0 + h], 2 * N);
+        }
+        const size_t total = (size_t)count * lw;
+        if (ckks) sum_c0_kernel<true><<<blocks_for(total), TPB, 0, st>>>(ca, c.primes(), total);
+        else sum_c0_kernel<false><<<blocks_for(total), TPB, 0, st>>>(ca, c.primes(), total);
+        launch_check("sum_c0");
+    }
+    const DevPrime *targets = c.keyswitch_primes(L);
+    const uint32_t K = (uint32_t)c.key_count();
+    uint64_t *d = at(lay.d), *T = at(lay.T), *P = at(lay.P), *S = at(lay.S), *Psum = at(lay.Psum), *V = at(lay.V);
+    uint32_t summed = 0, left = 0;  // key switches in Psum, V; and still to come
+    for (uint32_t h = 0; h < n; h++) left += elts[h] != 1;
+    for (uint32_t h0 = 0; h0 < n;) {
+        if (elts[h0] == 1) {
+            h0++;
+            continue;
+        }
+        uint32_t nb = 1;  // consecutive switches, at most a summed ModDown's 15 in all
+        while (nb < lay.nb && h0 + nb < n && elts[h0 + nb] != 1 && summed + nb < 15) nb++;
+        const uint64_t *x = in + h0 * step;
+        GaloisPerm perm{count, {}};
+        InnerKeys ik{};
+        ik.n = nb;
+        ik.per = count;
+        SumC0Args ga{x, nullptr, {}, {}, nb, count, L, logn, true};
+        for (uint32_t h = 0; h < nb; h++) {
+            perm.elt[h] = ga.elt[h] = ik.elt[h] = elts[h0 + h];
+            ga.elt_inv[h] = (uint32_t)hm::invmod(elts[h0 + h], 2 * N);
+            ik.key[h] = keys[h0 + h];
+        }
+        // digits of sigma(c1): CKKS through the permutation on load (c1 itself, permuted on
+        // load, supplies the own-prime terms), BFV permuted in coefficient form
+        if (ckks) {
+            ntt_inverse_galois(x + lw, LimbGrid{1, 2 * L, L, nb * count}, perm, d, LimbGrid{1, L, L, nb * count},
+                               c.primes(), logn, st);
+        } else {
+            const size_t total = (size_t)nb * count * lw;
+            galois_digits_kernel<<<blocks_for(total), TPB, 0, st>>>(ga, d, c.primes(), total);
+            launch_check("galois_digits");
+        }
+        if (logn == 15 || logn == 16) {
+            for (uint32_t h = 0; h < nb; h++)
+                ntt_modup_keyprod(d + h * count * lw, lw, T, ik.key[h], P + h * step, S + (size_t)h * count * 2 * N,
+                                  ckks ? x + h * step + lw : nullptr, ctw, count, L, K, targets, c.primes(), logn,
+                                  c.fp_primes, st, nullptr, c.ks_shape(L, count),
+                                  KsFold{nullptr, 0, nullptr, false, ik.elt[h]});
+        } else {
+            const bool skipped = modup_to_T(c, d, lw, T, nb * count, L, st, nullptr, ckks);
+            keyswitch_inner_products(c, T, ik, P, S, L, st, skipped ? x + lw : nullptr, ctw);
+        }
+        ntt_inverse(S, nb * count * 2, 1, targets + L, logn, NTT_FULL, st);
+        const SumArgs sa{P, S, Psum, V, {1, 1, 1, 1}, c.moduli[K - 1]};
+        const size_t total = (size_t)2 * count * (L + 1) * N;
+        sum_products_kernel<<<blocks_for(total), TPB, 0, st>>>(sa, nb, c.primes(), L, logn, 2 * count, summed == 0, total);
+        launch_check("sum_products");
+        summed += nb;
+        left -= nb;
+        h0 += nb;
+        if (summed == 15 || !left) {
+            ModDownArgs md{V, Psum, out, ctw, c.ks_consts(), c.moduli[K - 1], L, false};
+            md.presum = summed;
+            ntt_moddown(ckks, ckks ? at(lay.U) : Psum, md, count, c.primes(), logn, st);
+            summed = 0;
+        }
+    }
+}
+
 }  // namespace shc

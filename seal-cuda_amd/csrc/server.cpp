@@ -23,7 +23,7 @@ namespace {
 size_t ct_words(const ServerProgram &p) { return 2 * (size_t)p.L * p.ctx->n; }
 
 size_t matvec_ws(const ServerProgram &p, uint32_t m) {
-    return std::max(rotate_sum_workspace(*p.ctx, m, p.L), galois_keyswitch_workspace(*p.ctx, m, p.L));
+    return std::max(rotate_sum_workspace(*p.ctx, m, p.L), rotate_accumulate_workspace(*p.ctx, m, p.L));
 }
 
 struct MulRelinLayout {
@@ -109,13 +109,14 @@ static const uint64_t *run_program(const ServerProgram &p, uint64_t *d_in, char 
     if (bfv) ntt_forward(baby, (size_t)p.b * m * 2 * L, L, c.primes(), c.logn, NTT_FULL, st);
     multiply_plain_accumulate_many(c, baby, p.plains, p.b, p.g, m * 2, L, inner, st);
     if (bfv) ntt_inverse(inner, (size_t)p.g * m * 2 * L, L, c.primes(), c.logn, NTT_FULL, st);
-    for (uint32_t h = 1; h < p.g; h++)
-        apply_galois_keyswitch(c, inner + h * ct, m, L, p.giant_elts[h - 1], p.giant_keys[h - 1], q, ws_bytes, st);
     if (p.g == 1) {
         SHC_HIP(hipMemcpyAsync(out, inner, ct * 8, hipMemcpyDeviceToDevice, st));
     } else {
-        poly_add(c, inner, inner + ct, out, m * 2, L, st);
-        for (uint32_t h = 2; h < p.g; h++) poly_add(c, out, inner + h * ct, out, m * 2, L, st);
+        std::vector<uint32_t> elts(1, 1);
+        std::vector<const uint64_t *> keys(1, nullptr);
+        elts.insert(elts.end(), p.giant_elts.begin(), p.giant_elts.end());
+        keys.insert(keys.end(), p.giant_keys.begin(), p.giant_keys.end());
+        rotate_accumulate(c, inner, m, L, elts.data(), keys.data(), p.g, out, q, ws_bytes, st);
     }
     *stride = cw;
     return out;

@@ -11,11 +11,11 @@ BFV: each of the two rows of N/2 slots, which rotateRows turns independently):
 
 where rot_k(x)[i] = x[i + k] (rotateVector / rotateRows(k)).  The b - 1 baby rotations
 share one ModUp (shc_rotate_many), the g inner sums come from one
-shc_multiply_plain_accumulate_many call over NTT-form operands (each baby rotation read
-once per 8 giant steps), and the g - 1 giant rotations are ordinary key switches.  BFV
-ciphertexts live in coefficient form: the b baby rotations go to NTT form once, and the
-inner sums come back by one inverse transform before the giant rotations.  All
-ciphertexts of a batch share the diagonals and keys.
+shc_multiply_plain_accumulate_many call over NTT-form operands, and the g - 1 giant
+rotations are summed by shc_rotate_accumulate.  BFV ciphertexts live in coefficient form:
+the b baby rotations go to NTT form once, and the inner sums come back by one inverse
+transform before the giant rotations.  All ciphertexts of a batch share the diagonals and
+keys.
 """
 import numpy as np
 
@@ -55,7 +55,7 @@ class BsgsMatvec:
 
     def workspace_sizes(self, count):
         ctx, L = self.ctx, self.L
-        return max(ctx.rotate_sum_workspace_size(count, L), ctx.galois_workspace_size(count, L))
+        return max(ctx.rotate_sum_workspace_size(count, L), ctx.rotate_accumulate_workspace_size(count, L))
 
     def run(self, d_in, count, d_out, d_baby, d_inner, d_ws, ws_bytes, stream=None, around_sums=None):
         """d_in, d_out: [count][2][L][N]; d_baby: scratch [b][count][2][L][N];
@@ -82,15 +82,11 @@ class BsgsMatvec:
         if self.bfv:
             ctx.ntt_inverse(d_inner, g * count * 2, L, stream)
         # giant steps: rot_{h b}(inner[h]), summed
-        for h in range(1, g):
-            ctx.apply_galois_keyswitch(d_inner + h * ct_bytes, self.giant_keys[h - 1], self.giant_elts[h - 1], count,
-                                       L, d_ws, ws_bytes, stream)
         if g == 1:
             _memcpy_d2d(d_out, d_inner, ct_bytes, stream)
         else:
-            ctx.add(d_inner, d_inner + ct_bytes, d_out, count * 2, L, stream)
-            for h in range(2, g):
-                ctx.add(d_out, d_inner + h * ct_bytes, d_out, count * 2, L, stream)
+            ctx.rotate_accumulate(d_inner, count, L, [1] + self.giant_elts, [None] + list(self.giant_keys), d_out, d_ws,
+                                  ws_bytes, stream)
 
 
 _rt = None

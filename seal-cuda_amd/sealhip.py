@@ -106,6 +106,9 @@ def lib():
         L.shc_rotate_sum.argtypes = [_vp, _vp, u32, u32, ctypes.POINTER(u32), ctypes.POINTER(_vp),
                                      ctypes.POINTER(_vp), u32, _vp, _vp, sz, _vp]
         L.shc_rotate_many.argtypes = L.shc_rotate_sum.argtypes
+        L.shc_rotate_accumulate_workspace_size.argtypes = [_vp, u32, u32, ctypes.POINTER(sz)]
+        L.shc_rotate_accumulate.argtypes = [_vp, _vp, u32, u32, ctypes.POINTER(u32), ctypes.POINTER(_vp), u32, _vp, _vp,
+                                            sz, _vp]
         L.shc_multiply_plain_accumulate.argtypes = [_vp, _vp, _vp, u32, u32, u32, _vp, _vp]
         L.shc_multiply_plain_accumulate_many.argtypes = [_vp, _vp, _vp, u32, u32, u32, u32, _vp, _vp]
         L.shc_autotune_relinearize.argtypes = [_vp, _vp, _vp, u32, u32, _vp, sz, ctypes.c_int, _vp,
@@ -484,6 +487,15 @@ class Context:
         h = (_vp * r)(*d_hoisted)
         k = (_vp * r)(*d_keys)
         check(lib().shc_rotate_many(self.handle, d_in, count, limbs, e, h, k, r, d_out, d_ws, ws_bytes, stream))
+
+    def rotate_accumulate_workspace_size(self, count, limbs):
+        return self._size(lib().shc_rotate_accumulate_workspace_size, count, limbs)
+
+    def rotate_accumulate(self, d_in, count, limbs, elts, d_keys, d_out, d_ws, ws_bytes, stream=None):
+        n = len(elts)
+        e = (ctypes.c_uint32 * n)(*elts)
+        k = (_vp * n)(*d_keys)
+        check(lib().shc_rotate_accumulate(self.handle, d_in, count, limbs, e, k, n, d_out, d_ws, ws_bytes, stream))
 
     def multiply_plain_accumulate(self, d_cts, d_plains, terms, polys, limbs, d_out, stream=None):
         check(lib().shc_multiply_plain_accumulate(self.handle, d_cts, d_plains, terms, polys, limbs, d_out, stream))

@@ -121,6 +121,38 @@ def test_rotation_passes_zero_digits(scheme, zeros):
     run_case(scheme, 13, [60, 40, 50], 2, 2, [1, 2, -1, 3, 5], zero_digits=zeros, seed=8)
 
 
+@pytest.mark.parametrize("scheme,logn,bits,L,count,steps", [
+    (CKKS, 12, [60, 40, 40, 60], 3, 2, [None, 1, -2]),                  # one at a time
+    (CKKS, 13, [60, 40, 50, 60], 3, 3, [None] + list(range(1, 18))),    # two summed ModDowns
+    (BFV, 13, [43, 44, 44], 2, 5, [1, 2, None, 3, 0, 4, 5]),            # batches around the identity
+    (BFV, 14, [60, 50, 60], 2, 1, [None]),
+    (CKKS, 15, [60, 40, 50, 60], 3, 5, [None, 2, 4, 6, 8, 10]),         # the fused key products
+    (CKKS, 15, [60, 60], 1, 1, [3]),
+    (BFV, 15, [60, 50, 60], 2, 2, [1, 0]),
+])
+def test_rotate_accumulate(scheme, logn, bits, L, count, steps):
+    n = 1 << logn
+    moduli = ck.coeff_modulus_create(n, bits)
+    ctx = hip().Context(scheme, n, moduli, 65537 if scheme == BFV else 0)
+    rng = np.random.default_rng(len(steps) + logn)
+    cts = ck.uniform_residues(rng, (len(steps), count, 2, L, n), moduli[:L])
+    elts = [1 if s is None else ck.galois_elt(logn, s) for s in steps]
+    keys = [None if s is None else ck.random_key(rng, moduli, logn) for s in steps]
+    dkeys = [None if k is None else to_dev(k) for k in keys]
+    din, out = to_dev(cts), empty_dev((count, 2, L, n))
+    wb = ctx.rotate_accumulate_workspace_size(count, L)
+    ctx.rotate_accumulate(din.data_ptr(), count, L, elts, [None if k is None else k.data_ptr() for k in dkeys],
+                          out.data_ptr(), ws(wb).data_ptr(), wb, stream())
+    got = from_dev(out)
+    for c in range(count):
+        want = None
+        for h, (e, k) in enumerate(zip(elts, keys)):
+            rot = cts[h, c] if k is None else ck.apply_galois_keyswitch(scheme, cts[h, c], e, k, moduli, L, logn)
+            want = rot if want is None else ck.mod_add(want, rot, moduli)
+        np.testing.assert_array_equal(got[c], want, err_msg=f"ciphertext {c}")
+    np.testing.assert_array_equal(from_dev(din), cts)
+
+
 def test_rotate_sum_in_a_captured_graph():
     """The hoisted rotation sum waits for nothing on the host, so it can be captured: a
     captured call (with zero digits in the batch, so the fix runs) replays to the eager
