@@ -106,13 +106,10 @@ __global__ __launch_bounds__(SUBS << (K - E)) void ntt_rows_encrypt_kernel(const
         });
 }
 
-template <int LOGN>
-void launch_encrypt(const EncArgs &a, uint32_t jn, const DevPrime *primes, hipStream_t st) {
-    constexpr int K1 = LOGN / 2;
-    constexpr int K2 = LOGN - K1;
-    constexpr int E = 4;
-    constexpr int CS = 16;
-    constexpr int RS = 4096 >> K2;
+template <int LOGN, bool SMALL>
+void launch_encrypt_as(const EncArgs &a, uint32_t jn, const DevPrime *primes, hipStream_t st) {
+    using S = PassShape<LOGN, SMALL>;
+    constexpr int K1 = S::K1, K2 = S::K2, E = S::E, CS = S::CS, RS = S::RS;
     const uint32_t col_blocks = a.L * jn * ((1u << K2) / CS);
     const bool mx = rows_mixed<LOGN, K2, RS>(jn);
     const uint32_t row_blocks = a.L * rows_blocks_per_prime<LOGN, K2, E, RS>(jn, mx);
@@ -121,6 +118,13 @@ void launch_encrypt(const EncArgs &a, uint32_t jn, const DevPrime *primes, hipSt
         ntt_rows_encrypt_kernel<LOGN, K2, E, RS, true><<<row_blocks, RS << (K2 - E), 0, st>>>(primes, a, jn);
     else
         ntt_rows_encrypt_kernel<LOGN, K2, E, RS, false><<<row_blocks, RS << (K2 - E), 0, st>>>(primes, a, jn);
+}
+
+template <int LOGN>
+void launch_encrypt(const EncArgs &a, uint32_t jn, const DevPrime *primes, hipStream_t st) {
+    with_shape<LOGN>((uint64_t)a.L * jn, [&](auto s) {
+        launch_encrypt_as<LOGN, decltype(s)::value>(a, jn, primes, st);
+    });
 }
 
 struct ModDownGroupDev {
@@ -195,14 +199,11 @@ __global__ __launch_bounds__(SUBS << (K - E)) void ntt_rows_galois_kernel(const 
         [&](uint32_t i, uint32_t j, size_t off, uint64_t x) { *g.at(i, j, off) = x; });
 }
 
-template <int LOGN>
-void launch_inverse_galois(const uint64_t *src, LimbGrid slg, const GaloisPerm &perm, uint64_t *data, LimbGrid lg,
+template <int LOGN, bool SMALL>
+void launch_inverse_galois_as(const uint64_t *src, LimbGrid slg, const GaloisPerm &perm, uint64_t *data, LimbGrid lg,
                            const DevPrime *primes, hipStream_t st) {
-    constexpr int K1 = LOGN / 2;
-    constexpr int K2 = LOGN - K1;
-    constexpr int E = 4;
-    constexpr int CS = 16;
-    constexpr int RS = 4096 >> K2;
+    using S = PassShape<LOGN, SMALL>;
+    constexpr int K1 = S::K1, K2 = S::K2, E = S::E, CS = S::CS, RS = S::RS;
     const bool mx = rows_mixed<LOGN, K2, RS>(lg.J);
     const uint32_t row_blocks = lg.I * rows_blocks_per_prime<LOGN, K2, E, RS>(lg.J, mx);
     const uint32_t col_blocks = lg.I * lg.J * ((1u << K2) / CS);
@@ -214,13 +215,18 @@ void launch_inverse_galois(const uint64_t *src, LimbGrid slg, const GaloisPerm &
 }
 
 template <int LOGN>
-void launch_moddown(bool ckks, uint64_t *buf, const ModDownArgs &a, uint32_t jn, const DevPrime *primes,
+void launch_inverse_galois(const uint64_t *src, LimbGrid slg, const GaloisPerm &perm, uint64_t *data, LimbGrid lg,
+                           const DevPrime *primes, hipStream_t st) {
+    with_shape<LOGN>((uint64_t)lg.I * lg.J, [&](auto s) {
+        launch_inverse_galois_as<LOGN, decltype(s)::value>(src, slg, perm, data, lg, primes, st);
+    });
+}
+
+template <int LOGN, bool SMALL>
+void launch_moddown_as(bool ckks, uint64_t *buf, const ModDownArgs &a, uint32_t jn, const DevPrime *primes,
                     hipStream_t st) {
-    constexpr int K1 = LOGN / 2;
-    constexpr int K2 = LOGN - K1;
-    constexpr int E = 4;
-    constexpr int CS = 16;
-    constexpr int RS = 4096 >> K2;
+    using S = PassShape<LOGN, SMALL>;
+    constexpr int K1 = S::K1, K2 = S::K2, E = S::E, CS = S::CS, RS = S::RS;
     const uint32_t col_blocks = a.L * jn * ((1u << K2) / CS);
     const bool mx = rows_mixed<LOGN, K2, RS>(jn);
     const uint32_t row_blocks = a.L * rows_blocks_per_prime<LOGN, K2, E, RS>(jn, mx);
@@ -248,12 +254,23 @@ void launch_moddown(bool ckks, uint64_t *buf, const ModDownArgs &a, uint32_t jn,
 }
 
 template <int LOGN>
-void launch_moddown_groups(const ModDownGroup *gs, uint32_t n, const DevPrime *primes, hipStream_t st) {
-    constexpr int K1 = LOGN / 2;
-    constexpr int K2 = LOGN - K1;
-    constexpr int E = 4;
-    constexpr int CS = 16;
-    constexpr int RS = 4096 >> K2;
+void launch_moddown(bool ckks, uint64_t *buf, const ModDownArgs &a, uint32_t jn, const DevPrime *primes,
+                    hipStream_t st) {
+    with_shape<LOGN>((uint64_t)a.L * jn, [&](auto s) {
+        launch_moddown_as<LOGN, decltype(s)::value>(ckks, buf, a, jn, primes, st);
+    });
+}
+
+uint64_t group_limbs(const ModDownGroup *gs, uint32_t n) {
+    uint64_t limbs = 0;
+    for (uint32_t g = 0; g < n; g++) limbs += (uint64_t)gs[g].a.L * 2 * gs[g].count;
+    return limbs;
+}
+
+template <int LOGN, bool SMALL>
+void launch_moddown_groups_as(const ModDownGroup *gs, uint32_t n, const DevPrime *primes, hipStream_t st) {
+    using S = PassShape<LOGN, SMALL>;
+    constexpr int K1 = S::K1, K2 = S::K2, E = S::E, CS = S::CS, RS = S::RS;
     ModDownGroups cols{}, rmx{}, rfull{};
     std::vector<uint64_t> csz, msz, fsz;
     for (uint32_t g = 0; g < n; g++) {
@@ -281,6 +298,13 @@ void launch_moddown_groups(const ModDownGroup *gs, uint32_t n, const DevPrime *p
         const uint32_t b = fill_starts(rfull, fsz);
         ntt_rows_moddown_grouped_kernel<LOGN, K2, E, RS, false><<<b, RS << (K2 - E), 0, st>>>(primes, rfull);
     }
+}
+
+template <int LOGN>
+void launch_moddown_groups(const ModDownGroup *gs, uint32_t n, const DevPrime *primes, hipStream_t st) {
+    with_shape<LOGN>(group_limbs(gs, n), [&](auto s) {
+        launch_moddown_groups_as<LOGN, decltype(s)::value>(gs, n, primes, st);
+    });
 }
 
 }  // namespace

@@ -369,7 +369,8 @@ __device__ __forceinline__ void cols_modup_body(uint32_t bid, const uint64_t *__
     // the second phase's twiddles (the first 2^K entries of the target's table) go through
     // LDS, each thread bringing one, requested a target ahead
     __shared__ ulonglong2 tws[1 << K];
-    static_assert(SUBS << (K - E) == 1 << K, "one twiddle per thread");
+    static_assert(SUBS << (K - E) >= 1 << K, "one twiddle per thread");
+    const bool brings = tid < 1 << K;
     auto table = [&](uint32_t i) {
         return MIXED && targets[i].fwd_fp ? (const ulonglong2 *)targets[i].fwd_fp : targets[i].fwd;
     };
@@ -406,18 +407,18 @@ __device__ __forceinline__ void cols_modup_body(uint32_t bid, const uint64_t *__
         // one target per block (small batches): the first phase loads straight from the
         // digit, nothing held across targets (fewer registers, more waves)
         if (skip_diag && i0 == j) return;  // uniform: the whole block
-        tws[tid] = load_tw(table(i0), tid);
+        if (brings) tws[tid] = load_tw(table(i0), tid);
         transform(i0, [&](int idx, int) { return in[(size_t)idx * C]; });
         return;
     }
-    ulonglong2 tw = load_tw(table(i0), tid);
+    ulonglong2 tw = load_tw(table(i0), brings ? tid : 0);
     uint64_t dv[1 << E];
 #pragma unroll
     for (int k = 0; k < (1 << E); k++) dv[k] = in[(size_t)phase_index<K, E, 0, E>(t, k) * C];
     for (uint32_t i = i0; i < i1; i++) {
         __syncthreads();  // the previous target's second phase has read the tile
-        tws[tid] = tw;
-        if (i + 1 < i1) tw = load_tw(table(i + 1), tid);
+        if (brings) tws[tid] = tw;
+        if (i + 1 < i1) tw = load_tw(table(i + 1), brings ? tid : 0);
         if (skip_diag && i == j) continue;  // uniform
         transform(i, [&](int, int k) { return dv[k]; });
     }
@@ -469,15 +470,12 @@ inline uint32_t modup_targets_per_block(uint32_t tile_blocks, uint32_t L, uint32
     return (L + chunks) / chunks;  // ceil((L + 1) / chunks)
 }
 
-template <int LOGN>
-void launch_modup(const uint64_t *d, size_t d_stride, uint64_t *T, uint32_t cts, uint32_t L, const DevPrime *targets,
+template <int LOGN, bool SMALL>
+void launch_modup_as(const uint64_t *d, size_t d_stride, uint64_t *T, uint32_t cts, uint32_t L, const DevPrime *targets,
                   const DevPrime *digits, bool skip_diag, bool reduce_4q, bool mixed, const KernelProbe *probe,
                   hipStream_t st, KsShape shape) {
-    constexpr int K1 = LOGN / 2;
-    constexpr int K2 = LOGN - K1;
-    constexpr int E = 4;
-    constexpr int CS = 16;
-    constexpr int RS = 4096 >> K2;
+    using S = PassShape<LOGN, SMALL>;
+    constexpr int K1 = S::K1, K2 = S::K2, E = S::E, CS = S::CS, RS = S::RS;
     const uint32_t tc = modup_targets_per_block(cts * L * ((1u << K2) / CS), L, shape.cols_targets);
     const uint32_t col_grid = cts * L * ((L + tc) / tc) * ((1u << K2) / CS);
     with_bool(mixed, [&](auto mx) {
@@ -503,6 +501,16 @@ void launch_modup(const uint64_t *d, size_t d_stride, uint64_t *T, uint32_t cts,
                 <<<row_blocks, RS << (K2 - E), 0, st>>>(T, targets, lg, jn_short);
     });
     if (probe) SHC_HIP(hipEventRecord(probe->end, st));
+}
+
+template <int LOGN>
+void launch_modup(const uint64_t *d, size_t d_stride, uint64_t *T, uint32_t cts, uint32_t L, const DevPrime *targets,
+                  const DevPrime *digits, bool skip_diag, bool reduce_4q, bool mixed, const KernelProbe *probe,
+                  hipStream_t st, KsShape shape) {
+    with_shape<LOGN>((uint64_t)cts * L * (L + 1), [&](auto s) {
+        launch_modup_as<LOGN, decltype(s)::value>(d, d_stride, T, cts, L, targets, digits, skip_diag, reduce_4q, mixed,
+                                                  probe, st, shape);
+    });
 }
 
 // The fused rows pass + key products over a batch: groups of 4 ciphertexts, then the
@@ -535,6 +543,12 @@ void launch_keyprod_groups(const uint64_t *T, const uint64_t *key, uint64_t *P, 
     }
 }
 
+// log2 of the values per thread of the ModUp columns pass: 8 where targets take the fp64
+// butterflies, whose pass waits more than it issues (289 -> 271 us for 16 ciphertexts at
+// N = 2^15, L = 15 against 16 values), 16 for integer ones (13.5 ms for 128 at N = 2^16,
+// L = 24 against 13.9 with 8, 16.6 with 4).
+constexpr int modup_cols_log(bool mixed) { return mixed ? 3 : 4; }
+
 template <int LOGN>
 void launch_modup_keyprod(const uint64_t *d, size_t d_stride, uint64_t *T, const uint64_t *key, uint64_t *P,
                           uint64_t *S, const uint64_t *diag, size_t diag_stride, uint32_t cts, uint32_t L,
@@ -542,18 +556,16 @@ void launch_modup_keyprod(const uint64_t *d, size_t d_stride, uint64_t *T, const
                           const KernelProbe *probe, hipStream_t st, KsShape shape, const KsFold &fold) {
     constexpr int K1 = LOGN / 2;
     constexpr int K2 = LOGN - K1;
-    constexpr int E = 4;
     constexpr int CS = 16;
     const uint32_t tc = modup_targets_per_block(cts * L * ((1u << K2) / CS), L, shape.cols_targets);
     const uint32_t col_grid = cts * L * ((L + tc) / tc) * ((1u << K2) / CS);
     with_bool(mixed, [&](auto mx) {
-        constexpr bool MIXED = decltype(mx)::value;
-        if (tc == 1)
-            ntt_cols_modup_kernel<LOGN, K1, E, CS, true, MIXED><<<col_grid, CS << (K1 - E), 0, st>>>(
+        with_bool(tc == 1, [&](auto one) {
+            constexpr bool MIXED = decltype(mx)::value;
+            constexpr int E = modup_cols_log(MIXED);
+            ntt_cols_modup_kernel<LOGN, K1, E, CS, decltype(one)::value, MIXED><<<col_grid, CS << (K1 - E), 0, st>>>(
                 d, d_stride, T, targets, digits, cts, L, diag != nullptr, tc);
-        else
-            ntt_cols_modup_kernel<LOGN, K1, E, CS, false, MIXED><<<col_grid, CS << (K1 - E), 0, st>>>(
-                d, d_stride, T, targets, digits, cts, L, diag != nullptr, tc);
+        });
     });
     const uint32_t tiles = (L + 1) << K1;
     const uint64_t tile_slots = (uint64_t)((tiles + 7) / 8) * 8;
@@ -603,8 +615,9 @@ void launch_modup_keyprod_groups(const KsGroup *gs, uint32_t n, const uint64_t *
     const uint32_t cb = fill_starts(mg, msz);
     with_bool(all_one, [&](auto one) {
         with_bool(mixed, [&](auto mx) {
-            ntt_cols_modup_grouped_kernel<LOGN, K1, E, CS, decltype(one)::value, decltype(mx)::value>
-                <<<cb, CS << (K1 - E), 0, st>>>(mg);
+            constexpr int EC = modup_cols_log(decltype(mx)::value);
+            ntt_cols_modup_grouped_kernel<LOGN, K1, EC, CS, decltype(one)::value, decltype(mx)::value>
+                <<<cb, CS << (K1 - EC), 0, st>>>(mg);
         });
     });
     // fused rows pass + key products: groups of 4, then of 2, then single ciphertexts

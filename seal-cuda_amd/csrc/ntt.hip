@@ -45,8 +45,8 @@ __global__ __launch_bounds__(SUBS << (K - E)) void ntt_rows_from_kernel(const ui
         });
 }
 
-template <int LOGN, bool INV, bool FULL>
-void launch_ntt(uint64_t *data, LimbGrid lg, uint32_t j0, uint32_t jn, const DevPrime *primes, hipStream_t st) {
+template <int LOGN, bool INV, bool FULL, bool SMALL>
+void launch_ntt_as(uint64_t *data, LimbGrid lg, uint32_t j0, uint32_t jn, const DevPrime *primes, hipStream_t st) {
     if constexpr (LOGN <= 12) {
         constexpr int K = LOGN;
         constexpr int E = K < 4 ? K : 4;
@@ -55,11 +55,8 @@ void launch_ntt(uint64_t *data, LimbGrid lg, uint32_t j0, uint32_t jn, const Dev
         const uint32_t blocks = lg.I * ((jn + SUBS - 1) / SUBS);
         ntt_rows_kernel<LOGN, K, E, SUBS, INV, true, FULL><<<blocks, SUBS * T, 0, st>>>(data, primes, lg, j0, jn);
     } else {
-        constexpr int K1 = LOGN / 2;
-        constexpr int K2 = LOGN - K1;
-        constexpr int E = 4;
-        constexpr int CS = 16;                                    // columns per block
-        constexpr int RS = (4096 >> K2) < 1 ? 1 : (4096 >> K2);  // rows per block
+        using S = PassShape<LOGN, SMALL>;
+        constexpr int K1 = S::K1, K2 = S::K2, E = S::E, CS = S::CS, RS = S::RS;
         const uint32_t col_blocks = lg.I * jn * ((1u << K2) / CS);
         const bool mx = rows_mixed<LOGN, K2, RS>(jn);
         const uint32_t row_blocks = lg.I * rows_blocks_per_prime<LOGN, K2, E, RS>(jn, mx);
@@ -85,9 +82,19 @@ void launch_ntt(uint64_t *data, LimbGrid lg, uint32_t j0, uint32_t jn, const Dev
     }
 }
 
+template <int LOGN, bool INV, bool FULL>
+void launch_ntt(uint64_t *data, LimbGrid lg, uint32_t j0, uint32_t jn, const DevPrime *primes, hipStream_t st) {
+    if constexpr (LOGN <= 12)
+        launch_ntt_as<LOGN, INV, FULL, false>(data, lg, j0, jn, primes, st);
+    else
+        with_shape<LOGN>((uint64_t)lg.I * jn, [&](auto s) {
+            launch_ntt_as<LOGN, INV, FULL, decltype(s)::value>(data, lg, j0, jn, primes, st);
+        });
+}
+
 // Inverse transform of src's limbs into data (rows pass from src, columns pass in place).
-template <int LOGN, bool FULL>
-void launch_inverse_from(const uint64_t *src, LimbGrid slg, uint64_t *data, LimbGrid lg, uint32_t j0, uint32_t jn,
+template <int LOGN, bool FULL, bool SMALL>
+void launch_inverse_from_as(const uint64_t *src, LimbGrid slg, uint64_t *data, LimbGrid lg, uint32_t j0, uint32_t jn,
                          const DevPrime *primes, hipStream_t st) {
     if constexpr (LOGN <= 12) {
         constexpr int K = LOGN;
@@ -98,11 +105,8 @@ void launch_inverse_from(const uint64_t *src, LimbGrid slg, uint64_t *data, Limb
         ntt_rows_from_kernel<LOGN, K, E, SUBS, true, true, FULL>
             <<<blocks, SUBS * T, 0, st>>>(src, slg, data, primes, lg, j0, jn);
     } else {
-        constexpr int K1 = LOGN / 2;
-        constexpr int K2 = LOGN - K1;
-        constexpr int E = 4;
-        constexpr int CS = 16;
-        constexpr int RS = (4096 >> K2) < 1 ? 1 : (4096 >> K2);
+        using S = PassShape<LOGN, SMALL>;
+        constexpr int K1 = S::K1, K2 = S::K2, E = S::E, CS = S::CS, RS = S::RS;
         const uint32_t col_blocks = lg.I * jn * ((1u << K2) / CS);
         const bool mx = rows_mixed<LOGN, K2, RS>(jn);
         const uint32_t row_blocks = lg.I * rows_blocks_per_prime<LOGN, K2, E, RS>(jn, mx);
@@ -115,6 +119,17 @@ void launch_inverse_from(const uint64_t *src, LimbGrid slg, uint64_t *data, Limb
         ntt_cols_kernel<LOGN, K1, E, CS, true, true, FULL>
             <<<col_blocks, CS << (K1 - E), 0, st>>>(data, primes, lg, j0, jn);
     }
+}
+
+template <int LOGN, bool FULL>
+void launch_inverse_from(const uint64_t *src, LimbGrid slg, uint64_t *data, LimbGrid lg, uint32_t j0, uint32_t jn,
+                         const DevPrime *primes, hipStream_t st) {
+    if constexpr (LOGN <= 12)
+        launch_inverse_from_as<LOGN, FULL, false>(src, slg, data, lg, j0, jn, primes, st);
+    else
+        with_shape<LOGN>((uint64_t)lg.I * jn, [&](auto s) {
+            launch_inverse_from_as<LOGN, FULL, decltype(s)::value>(src, slg, data, lg, j0, jn, primes, st);
+        });
 }
 
 template <bool FULL>

@@ -403,6 +403,36 @@ uint32_t fill_starts(Table &t, const std::vector<uint64_t> &sizes) {
     return (uint32_t)acc;
 }
 
+// The passes' shape at one degree: the first K1 layers along columns (CS columns per block),
+// the last K2 inside rows (RS rows per block), 2^E values per thread.  Large launches take 16
+// values per thread (fewest LDS round trips and twiddle loads).  SMALL ones take 4: with few
+// waves per SIMD a pass is one wave's latency, of which a quarter is left.  A product, its
+// relinearization and rescale of one ciphertext at N = 2^13, L = 3 took 102.6 us with 16
+// values and takes 54.4 with 4; 37 of them at N = 2^14, L = 7 645 and 581 us; a chain round
+// over 64 at N = 2^15 7.41 and 6.82 ms.  The line lies at 2^26 words (1,024 limbs of 2^16):
+// beyond it the forms differ by under 1% (encryption) or 16 values win (decryption of 128
+// ciphertexts at N = 2^16, L = 24: 3.13 against 3.26 ms).
+constexpr uint64_t SMALL_WORDS = uint64_t(1) << 26;
+template <int LOGN, bool SMALL>
+struct PassShape {
+    static constexpr int K1 = LOGN / 2;
+    static constexpr int K2 = LOGN - K1;
+    static constexpr int E = SMALL ? 2 : 4;
+    static constexpr int CS = 16;
+    static constexpr int RS = SMALL ? 256 >> (K2 - E) : (4096 >> K2) < 1 ? 1 : 4096 >> K2;
+};
+// f(std::true_type) for a small launch over `limbs` limbs, else f(std::false_type).
+template <int LOGN, class F>
+void with_shape(uint64_t limbs, F &&f) {
+    if constexpr (LOGN <= 16) {
+        if (limbs << LOGN <= SMALL_WORDS) {
+            f(std::true_type{});
+            return;
+        }
+    }
+    f(std::false_type{});
+}
+
 // f(std::true_type / std::false_type) for a run-time flag.
 template <class F>
 void with_bool(bool b, F &&f) {

@@ -120,14 +120,11 @@ __global__ __launch_bounds__(256) void ntt_cols_multi_kernel(NttMulti ng) {
     }
 }
 
-template <int LOGN, bool INV, bool FULL>
-void launch_ntt_groups(const NttGroup *gs, uint32_t n, hipStream_t st) {
+template <int LOGN, bool INV, bool FULL, bool SMALL>
+void launch_ntt_groups_as(const NttGroup *gs, uint32_t n, hipStream_t st) {
     static_assert(LOGN > 12, "grouped transforms run the two-pass schedule");
-    constexpr int K1 = LOGN / 2;
-    constexpr int K2 = LOGN - K1;
-    constexpr int E = 4;
-    constexpr int CS = 16;
-    constexpr int RS = 4096 >> K2;
+    using S = PassShape<LOGN, SMALL>;
+    constexpr int K1 = S::K1, K2 = S::K2, E = S::E, CS = S::CS, RS = S::RS;
     // the first pass reads src where a group has one; the second runs in place
     NttGroups cols{}, rows_mx{}, rows_full{};
     std::vector<uint64_t> csz, msz, fsz;
@@ -169,6 +166,13 @@ void launch_ntt_groups(const NttGroup *gs, uint32_t n, hipStream_t st) {
         ntt_cols_grouped_kernel<LOGN, K1, E, CS, true, true, FULL><<<cb, CS << (K1 - E), 0, st>>>(cols);
     }
     launch_check("grouped ntt launch");
+}
+
+template <int LOGN, bool INV, bool FULL>
+void launch_ntt_groups(const NttGroup *gs, uint32_t n, hipStream_t st) {
+    uint64_t limbs = 0;
+    for (uint32_t g = 0; g < n; g++) limbs += (uint64_t)gs[g].lg.I * gs[g].lg.J;
+    with_shape<LOGN>(limbs, [&](auto s) { launch_ntt_groups_as<LOGN, INV, FULL, decltype(s)::value>(gs, n, st); });
 }
 
 template <bool INV, bool FULL>

@@ -129,3 +129,26 @@ def test_multi_degree_transforms_in_one_launch():
         hip().ntt_forward_multi([(ctx, devs[2].data_ptr(), 1, 9)], stream())
     with pytest.raises(hip().SealHipError, match="16"):
         hip().ntt_forward_multi([(ctx, devs[2].data_ptr(), 1, 1)] * 17, stream())
+
+
+@pytest.mark.parametrize("logn", [13, 14, 15, 16])
+def test_launch_forms_agree(logn):
+    """A batch past 2^26 words (16 values per thread) against the same limbs in slices below it
+    (4 values per thread), forward and inverse; the small form is checked against the oracle
+    above."""
+    import torch
+    n = 1 << logn
+    moduli = ck.coeff_modulus_create(n, [60, 40])
+    ctx = hip().Context(2, n, moduli)
+    polys = (1 << 26) // n // 2 + 9  # of two limbs each, not a multiple of a block's rows
+    gen = torch.Generator(device="cuda").manual_seed(logn)
+    data = torch.empty((polys, 2, n), dtype=torch.int64, device="cuda")
+    for i, q in enumerate(moduli):
+        data[:, i] = torch.randint(0, q, (polys, n), generator=gen, device="cuda", dtype=torch.int64)
+    for transform in (ctx.ntt_forward, ctx.ntt_inverse):
+        whole, parts = data.clone(), data.clone()
+        transform(whole.data_ptr(), polys, 2, stream())
+        for p0 in range(0, polys, polys // 3):
+            transform(parts[p0].data_ptr(), min(polys // 3, polys - p0), 2, stream())
+        torch.cuda.synchronize()
+        assert torch.equal(whole, parts)
