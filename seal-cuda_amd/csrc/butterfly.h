@@ -28,19 +28,20 @@ __host__ __device__ __forceinline__ uint64_t sub_if_ge_neg(uint64_t v, uint64_t 
 // 2^64 - 4q.
 // Same congruences as the reference's Harvey butterflies (src/utils/dwthandler.h:88-372),
 // with wider lazy ranges.
-template <bool INV>
+// UNI: the twiddle is the same in every lane.
+template <bool INV, bool UNI = false>
 __host__ __device__ __forceinline__ void butterfly(uint64_t &x, uint64_t &y, ulonglong2 w, uint64_t four_q,
                                                    uint64_t neg_q, bool red, uint64_t neg_red) {
     if (!INV) {
         const uint64_t u = red ? sub_if_ge_neg(x, neg_red) : x;
-        const uint64_t v = shoup_lazier(y, w.x, w.y, neg_q);
+        const uint64_t v = shoup_lazier<UNI>(y, w.x, w.y, neg_q);
         x = u + v;
         y = u + four_q - v;
     } else {
         const uint64_t s = x + y;
         const uint64_t d = x + four_q - y;
         x = sub_if_ge_neg(s, neg_red);
-        y = shoup_lazier(d, w.x, w.y, neg_q);
+        y = shoup_lazier<UNI>(d, w.x, w.y, neg_q);
     }
 }
 

@@ -50,16 +50,34 @@ __host__ __device__ __forceinline__ uint64_t mulhi64_approx(uint64_t x, uint64_t
 // x * w mod q in [0, 4q), for any 64-bit x, w < q < 2^62, wq = floor(w 2^64 / q) and
 // neg_q = 2^64 - q.  The quotient estimate is Shoup's minus at most 2, so the remainder
 // x w - Q q lies in [0, 4q) and equals its low 64 bits, computed as x w + Q neg_q with
-// only the low halves of the cross products (9 multiplies in all).
+// only the low halves of the cross products (9 multiplies in all).  The four cross products
+// reach the high word alone: a chain of v_mad_u64_u32 and one 32-bit add (a v_mad_u64_u32
+// issues in 5.1 cycles, a v_mul_lo_u32 in 4.7 and a v_add3_u32 in 4.4, so four and an add
+// take 23 where four products and two three-way adds take 28), in inline assembly since the
+// compiler turns the chain back into them.  UNI: w and wq are the same in every lane (scalar
+// operands, one per instruction); neg_q always is.
+template <bool UNI = false>
 __host__ __device__ __forceinline__ uint64_t shoup_lazier(uint64_t x, uint64_t w, uint64_t wq, uint64_t neg_q) {
     const uint64_t Q = mulhi64_approx(x, wq);
     const uint32_t xl = (uint32_t)x, xh = (uint32_t)(x >> 32), wl = (uint32_t)w, wh = (uint32_t)(w >> 32);
     const uint32_t ql = (uint32_t)Q, qh = (uint32_t)(Q >> 32), nl = (uint32_t)neg_q, nh = (uint32_t)(neg_q >> 32);
     const uint64_t p = (uint64_t)xl * wl + (uint64_t)ql * nl;
-    // the cross products only reach the high word: 32-bit arithmetic there
-    uint32_t hi = (uint32_t)(p >> 32) + xl * wh + xh * wl + ql * nh + qh * nl;
 #if defined(__HIP_DEVICE_COMPILE__)
+    uint64_t c, sd;
+    if constexpr (UNI)
+        asm("v_mad_u64_u32 %0, %1, %2, %3, 0\n\tv_mad_u64_u32 %0, %1, %4, %5, %0\n\t"
+            "v_mad_u64_u32 %0, %1, %6, %7, %0\n\tv_mad_u64_u32 %0, %1, %8, %9, %0"
+            : "=&v"(c), "=&s"(sd)
+            : "v"(xl), "s"(wh), "v"(xh), "s"(wl), "v"(ql), "s"(nh), "v"(qh), "s"(nl));
+    else
+        asm("v_mad_u64_u32 %0, %1, %2, %3, 0\n\tv_mad_u64_u32 %0, %1, %4, %5, %0\n\t"
+            "v_mad_u64_u32 %0, %1, %6, %7, %0\n\tv_mad_u64_u32 %0, %1, %8, %9, %0"
+            : "=&v"(c), "=&s"(sd)
+            : "v"(xl), "v"(wh), "v"(xh), "v"(wl), "v"(ql), "s"(nh), "v"(qh), "s"(nl));
+    uint32_t hi = (uint32_t)(p >> 32) + (uint32_t)c;
     asm("" : "+v"(hi));  // keeps the 32-bit add from being widened back to 64 bits
+#else
+    const uint32_t hi = (uint32_t)(p >> 32) + xl * wh + xh * wl + ql * nh + qh * nl;
 #endif
     return ((uint64_t)hi << 32) | (uint32_t)p;
 }

@@ -50,8 +50,10 @@ __device__ __forceinline__ BfConst bf_const(const DevPrime &P) {
 // TileTw: the first phase from there (scalar loads), later phases from the sub-transform's
 // own 2^K entries in LDS (entry 2^s + lg, see stage_twiddles), whose latency is a few dozen
 // cycles where a table load in the middle of a pass takes hundreds.
-template <int LOGN, bool INV, class W2>
+// UNIFORM: g is the same in every lane, and so are the first phase's twiddles.
+template <int LOGN, bool INV, class W2, bool UNIFORM = true>
 struct GlobalTw {
+    static constexpr bool uniform = UNIFORM;
     const W2 *tw;
     int g, L0;
     template <bool FIRST>
@@ -62,6 +64,7 @@ struct GlobalTw {
 };
 template <int LOGN, class W2>
 struct TileTw {
+    static constexpr bool uniform = true;
     const W2 *tw;
     int g, L0;
     const W2 *lds;
@@ -97,7 +100,7 @@ __device__ __forceinline__ void phase_compute(uint64_t (&r)[1 << E], int t, cons
             const int idx = phase_index<K, E, S0, EP>(S0 == 0 ? 0 : t, j);
             const ulonglong2 w = tw.template at<S0 == 0>(s, idx >> (K - s));
             const bool red = !W || (s >= 2 && !(s & 1));
-            butterfly<INV>(r[j], r[j | (1 << b)], w, bc.four_q, bc.neg_q, red, W ? bc.neg_eight_q : bc.neg_four_q);
+            butterfly<INV, S0 == 0 && Tw::uniform>(r[j], r[j | (1 << b)], w, bc.four_q, bc.neg_q, red, W ? bc.neg_eight_q : bc.neg_four_q);
         }
     }
 }
@@ -272,7 +275,7 @@ __device__ __forceinline__ void rows_body_t(uint64_t *tile, uint32_t bid, const 
     }
     const size_t row_off = (size_t)g << K;
     const DevPrime &P = primes[i];
-    const GlobalTw<LOGN, INV, ulonglong2> tw{INV ? P.inv : P.fwd, g, RPL};
+    const GlobalTw<LOGN, INV, ulonglong2, !MX> tw{INV ? P.inv : P.fwd, g, RPL};
     auto addr = [sub](int idx) { return sub * row_words(K) + row_slot(idx); };
     auto load = [&](int idx, int) { return load_elem(i, j, row_off + idx); };
     if constexpr (NP == 1) {
