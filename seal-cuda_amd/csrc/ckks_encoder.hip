@@ -194,9 +194,12 @@ __global__ void round_reduce_kernel(const double2 *__restrict__ a, uint64_t *__r
         const double hid = floor(d * (1.0 / two64));
         const uint64_t hi = (uint64_t)hid;
         const uint64_t lo = (uint64_t)(d - hid * two64);
+        // below 2^64 (any usual scale) one word per coefficient: a third of the instructions
+        const bool wide = __any(hi != 0);
         for (uint32_t l = 0; l < L; l++) {
             const DevPrime &P = primes[l];
-            const uint64_t r = barrett128(u128{lo, hi}, P.q, P.ratio_lo, P.ratio_hi);
+            const uint64_t r = wide ? barrett128(u128{lo, hi}, P.q, P.ratio_lo, P.ratio_hi)
+                                    : barrett64(lo, P.q, P.ratio_hi);
             out[l * n + c] = neg ? negmod(r, P.q) : r;
         }
     }
@@ -418,8 +421,9 @@ void encode_body(const Context &c, const double *values, uint32_t count, size_t 
     launch_check("ckks encode");
     if (d_status) {
         encode_check_kernel<<<(batch + TPB - 1) / TPB, TPB, 0, st>>>(maxbits, T.total_bits, d_status, batch);
-        zero_if_rejected_kernel<<<dim3(blocks_for((size_t)L * n), batch), TPB, 0, st>>>(plain, d_status,
-                                                                                         (size_t)L * n);
+        // (few blocks per plaintext: hardly ever is there anything to clear)
+        zero_if_rejected_kernel<<<dim3(std::min<uint32_t>(16, blocks_for((size_t)L * n)), batch), TPB, 0, st>>>(
+            plain, d_status, (size_t)L * n);
         launch_check("ckks encode check");
         return;
     }

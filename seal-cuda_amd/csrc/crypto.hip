@@ -447,50 +447,46 @@ __global__ void keygen_combine_kernel(uint64_t *__restrict__ key, const uint64_t
 // is linear modulo each q_i): L1 + 2 + 2L transforms per ciphertext instead of
 // 3 L1 + 2 + 2L.  BFV stays in coefficient form: c_j[i] = p^-1 (INTT_i(pk_j[i] NTT_i(u))
 // + e_j - r_j), r_j from limb L of the same sum.
-
-// u lifted to the L1 limbs of U[g]; e0, e1 as signed integers in Es[g][0 / 1].
+// u, e0, e1 as bytes: u in {-1, 0, 1} at Us[g], |e| <= 21 at Es[g][0 / 1].  The transforms
+// that take them lift a byte to each prime as they load it; written here as lifted limbs, by
+// threads that each hold 8 coefficients, u alone cost 2.6 ms for 128 ciphertexts at N = 2^16,
+// L = 24 (8-byte stores 64 bytes apart), and its transform read them back.
 template <bool KEYED>
-__global__ void sample_encrypt_kernel(SamplerKey key, uint64_t seed, const DevPrime *__restrict__ primes, uint32_t L1,
-                                      int logn, size_t total, uint64_t *__restrict__ U, int64_t *__restrict__ Es) {
+__global__ void sample_encrypt_kernel(SamplerKey key, uint64_t seed, int logn, size_t total, int8_t *__restrict__ Us,
+                                      int8_t *__restrict__ Es) {
     const size_t n = (size_t)1 << logn;
     // per ciphertext: 2^ulog keystream blocks (8 coefficients each) or coefficients
     const int ulog = KEYED ? (logn > 3 ? logn - 3 : 0) : logn;
     for (size_t idx = (size_t)blockIdx.x * TPB + threadIdx.x; idx < total; idx += (size_t)gridDim.x * TPB) {
         const size_t g = idx >> ulog, b = idx & (((size_t)1 << ulog) - 1);
-        uint64_t *Ug = U + g * L1 * n;
-        int64_t *Eg = Es + g * 2 * n;
         for (int k = 0; k < 3; k++) {
             const uint64_t s = sub_seed(seed + g, (uint64_t)k);
             const int kind = k == 0 ? SAMPLE_TERNARY : SAMPLE_CBD;
+            int8_t *out = k == 0 ? Us + g * n : Es + (2 * g + (k - 1)) * n;
             if (KEYED) {
                 uint32_t ks[16];
                 chacha20_block(key, b, s, ks);
+                uint64_t word = 0;
 #pragma unroll
-                for (int w = 0; w < 8; w++) {
-                    const size_t c = b * 8 + w;
-                    if (c >= n) break;
-                    const int64_t v = small_from_word(kind, block_word(ks, w));
-                    if (k == 0) {
-                        for (uint32_t l = 0; l < L1; l++) {
-                            const uint64_t q = primes[l].q;
-                            Ug[(size_t)l * n + c] = v < 0 ? q - (uint64_t)(-v) : (uint64_t)v;
-                        }
-                    } else {
-                        Eg[(size_t)(k - 1) * n + c] = v;
-                    }
-                }
+                for (int w = 0; w < 8; w++)
+                    word |= (uint64_t)(uint8_t)(int8_t)small_from_word(kind, block_word(ks, w)) << (8 * w);
+                if (n >= 8) *reinterpret_cast<uint64_t *>(out + b * 8) = word;  // n is a power of two
+                else
+                    for (size_t w = 0; w < n; w++) out[w] = (int8_t)(word >> (8 * w));
             } else {
-                const int64_t v = small_from_word(kind, stream_word(s, b));
-                if (k == 0) {
-                    for (uint32_t l = 0; l < L1; l++) {
-                        const uint64_t q = primes[l].q;
-                        Ug[(size_t)l * n + b] = v < 0 ? q - (uint64_t)(-v) : (uint64_t)v;
-                    }
-                } else {
-                    Eg[(size_t)(k - 1) * n + b] = v;
-                }
+                out[b] = (int8_t)small_from_word(kind, stream_word(s, b));
             }
         }
+    }
+}
+
+// U[g][l][c] = Us[g][c] mod q_l, l < L1.
+__global__ void lift_small_kernel(const int8_t *__restrict__ Us, uint64_t *__restrict__ U,
+                                  const DevPrime *__restrict__ primes, uint32_t L1, int logn, size_t total) {
+    for (size_t idx = (size_t)blockIdx.x * TPB + threadIdx.x; idx < total; idx += (size_t)gridDim.x * TPB) {
+        const uint32_t r = uniform_row(idx, logn), g = r / L1, l = r - g * L1;
+        const int8_t v = Us[((size_t)g << logn) + (idx & (((size_t)1 << logn) - 1))];
+        U[idx] = v < 0 ? primes[l].q - (uint64_t)(-v) : (uint64_t)v;
     }
 }
 
@@ -531,7 +527,7 @@ __global__ void enc_products_kernel(const uint64_t *__restrict__ pk, uint32_t K,
 
 // CKKS, before the forward transform: out[g][j][i] = e_j - r_j (mod q_i), i < L (r_j = 0
 // when nothing is dropped); Pl[g][j] = INTT_p(pk_j[L] NTT_p(u)), coefficient form.
-__global__ void enc_error_kernel(const int64_t *__restrict__ Es, const uint64_t *__restrict__ Pl,
+__global__ void enc_error_kernel(const int8_t *__restrict__ Es, const uint64_t *__restrict__ Pl,
                                  uint64_t *__restrict__ out, const DevPrime *__restrict__ primes,
                                  const DivRoundConst *__restrict__ dc, uint64_t p, uint32_t L, int logn, size_t total) {
     const size_t n = (size_t)1 << logn;
@@ -568,7 +564,7 @@ __global__ void enc_finish_ckks_kernel(const uint64_t *__restrict__ pk, uint32_t
 
 // BFV: out[g][j][i] = (P[g][j][i] + e_j - r_j) p^-1 (mod q_i), P = INTT(pk_j NTT(u)) with
 // L1 limbs per polynomial; without a dropped prime, P[g][j][i] + e_j.
-__global__ void enc_finish_bfv_kernel(const uint64_t *__restrict__ P, const int64_t *__restrict__ Es,
+__global__ void enc_finish_bfv_kernel(const uint64_t *__restrict__ P, const int8_t *__restrict__ Es,
                                       uint64_t *__restrict__ out, const DevPrime *__restrict__ primes,
                                       const DivRoundConst *__restrict__ dc, uint64_t p, bool drop, uint32_t L,
                                       uint32_t L1, int logn, size_t total) {
@@ -751,7 +747,7 @@ void bfv_add_plain_scaled(const Context &c, uint64_t *c0, const uint64_t *plain,
 
 namespace {
 
-// Words of encrypt_many's workspace per ciphertext: U [L1][N], e0 and e1 [2][N], and
+// Words of encrypt_many's workspace per ciphertext: U [L1][N], e0, e1 and u (bytes) in [2][N], and
 // the products P ([2][N] of the dropped limb for CKKS, [2][L1][N] for BFV).
 size_t encrypt_many_words(const Context &c, uint32_t L) {
     const size_t L1 = upper_limbs(c, L);
@@ -766,8 +762,9 @@ void encrypt_chunk(const Context &c, const uint64_t *pk, const uint64_t *plain, 
     const int logn = c.logn;
     const DevPrime *primes = c.primes();
     uint64_t *U = static_cast<uint64_t *>(ws);
-    int64_t *Es = reinterpret_cast<int64_t *>(U + (size_t)m * L1 * n);
-    uint64_t *P = reinterpret_cast<uint64_t *>(Es + (size_t)m * 2 * n);
+    // e0, e1 and u as bytes in a region of two limbs per ciphertext
+    int8_t *Es = reinterpret_cast<int8_t *>(U + (size_t)m * L1 * n), *Us = Es + (size_t)m * 2 * n;
+    uint64_t *P = U + (size_t)m * (L1 + 2) * n;
     // drop: divide-and-round by q_L (row L1 of the rescale constants, entries i < L)
     const DivRoundConst *dc = drop ? c.rescale_consts(L1) : nullptr;
     const uint64_t p = drop ? c.moduli[L] : 0;
@@ -776,13 +773,18 @@ void encrypt_chunk(const Context &c, const uint64_t *pk, const uint64_t *plain, 
     for (int i = 0; i < 8; i++) key.k[i] = c.sampler_key[i];
     if (c.sampler_keyed) {
         const size_t total = (size_t)m * ((n + 7) / 8);
-        sample_encrypt_kernel<true><<<blocks_for(total), TPB, 0, st>>>(key, seed, primes, L1, logn, total, U, Es);
+        sample_encrypt_kernel<true><<<blocks_for(total), TPB, 0, st>>>(key, seed, logn, total, Us, Es);
     } else {
         const size_t total = (size_t)m * n;
-        sample_encrypt_kernel<false><<<blocks_for(total), TPB, 0, st>>>(key, seed, primes, L1, logn, total, U, Es);
+        sample_encrypt_kernel<false><<<blocks_for(total), TPB, 0, st>>>(key, seed, logn, total, Us, Es);
     }
     launch_check("sample_encrypt");
-    ntt_forward(U, m * L1, L1, primes, logn, NTT_FULL, st);
+    if (!ntt_forward_small(Us, U, L1, m, primes, logn, st)) {
+        const size_t uw = (size_t)m * L1 * n;
+        lift_small_kernel<<<blocks_for(uw), TPB, 0, st>>>(Us, U, primes, L1, logn, uw);
+        launch_check("lift_small");
+        ntt_forward(U, m * L1, L1, primes, logn, NTT_FULL, st);
+    }
     const size_t out_words = (size_t)m * 2 * L * n;
     if (ckks) {
         if (drop) {

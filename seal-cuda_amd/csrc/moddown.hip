@@ -70,6 +70,33 @@ __global__ __launch_bounds__(SUBS << (K - E)) void ntt_rows_moddown_kernel(const
 // ---- CKKS public-key encryption fused into the error term's forward transform ----
 __device__ __forceinline__ uint64_t enc_lift(int64_t v, uint64_t q) { return v < 0 ? q - (uint64_t)(-v) : (uint64_t)v; }
 
+// Columns pass of the transforms of signed bytes: every prime of polynomial j reads the same
+// bytes (i fastest), lifted on load.
+template <int LOGN, int K, int E, int SUBS>
+__global__ __launch_bounds__(SUBS << (K - E)) void ntt_cols_small_kernel(const int8_t *__restrict__ Us,
+                                                                        uint64_t *__restrict__ U,
+                                                                        const DevPrime *__restrict__ primes,
+                                                                        uint32_t L1, uint32_t m) {
+    cols_body<LOGN, K, E, SUBS, false, true>(
+        blockIdx.x, primes, 0, m,
+        [&](uint32_t i, uint32_t j, size_t off) { return enc_lift(Us[((size_t)j << LOGN) + off], primes[i].q); },
+        [&](uint32_t i, uint32_t j, size_t off, uint64_t x) { U[((size_t)(j * L1 + i) << LOGN) + off] = x; }, L1);
+}
+
+template <int LOGN, bool SMALL>
+void launch_small_as(const int8_t *Us, uint64_t *U, uint32_t L1, uint32_t m, const DevPrime *primes, hipStream_t st) {
+    using S = PassShape<LOGN, SMALL>;
+    constexpr int K1 = S::K1, K2 = S::K2, E = S::E, CS = S::CS, RS = S::RS;
+    const bool mx = rows_mixed<LOGN, K2, RS>(m);
+    const uint32_t row_blocks = L1 * rows_blocks_per_prime<LOGN, K2, E, RS>(m, mx);
+    ntt_cols_small_kernel<LOGN, K1, E, CS><<<L1 * m * ((1u << K2) / CS), CS << (K1 - E), 0, st>>>(Us, U, primes, L1, m);
+    const LimbGrid lg{1, L1, L1, m};
+    with_bool(mx, [&](auto x) {
+        ntt_rows_kernel<LOGN, K2, E, RS, false, true, true, decltype(x)::value>
+            <<<row_blocks, RS << (K2 - E), 0, st>>>(U, primes, lg, 0, m);
+    });
+}
+
 template <int LOGN, int K, int E, int SUBS>
 __global__ __launch_bounds__(SUBS << (K - E)) void ntt_cols_encrypt_kernel(const DevPrime *__restrict__ primes,
                                                                           EncArgs a, uint32_t jn) {
@@ -346,6 +373,26 @@ void ntt_inverse_galois(const uint64_t *src, LimbGrid slg, const GaloisPerm &per
         case 17: launch_inverse_galois<17>(src, slg, perm, data, lg, primes, st); break;
     }
     launch_check("permuted inverse ntt launch");
+}
+
+bool ntt_forward_small(const int8_t *Us, uint64_t *U, uint32_t L1, uint32_t m, const DevPrime *primes, int logn,
+                       hipStream_t st) {
+    if (logn < 13 || logn > 17 || m == 0 || (uint64_t)L1 * m > ((uint64_t(1) << 34) >> logn)) return false;
+    auto go = [&](auto n) {
+        constexpr int LOGN = decltype(n)::value;
+        with_shape<LOGN>((uint64_t)L1 * m, [&](auto s) {
+            launch_small_as<LOGN, decltype(s)::value>(Us, U, L1, m, primes, st);
+        });
+    };
+    switch (logn) {
+        case 13: go(std::integral_constant<int, 13>{}); break;
+        case 14: go(std::integral_constant<int, 14>{}); break;
+        case 15: go(std::integral_constant<int, 15>{}); break;
+        case 16: go(std::integral_constant<int, 16>{}); break;
+        case 17: go(std::integral_constant<int, 17>{}); break;
+    }
+    launch_check("small ntt launch");
+    return true;
 }
 
 bool ntt_encrypt_ckks(const EncArgs &a, uint32_t m, const DevPrime *primes, int logn, hipStream_t st) {

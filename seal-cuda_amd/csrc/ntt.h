@@ -131,10 +131,10 @@ bool ntt_moddown_polys(uint64_t *U, const ModDownArgs &args, uint32_t polys, con
 // ciphertext g: the columns pass computes x = e_k - r_k (mod q_i) on load -- r_k the
 // divide-and-round correction of the dropped prime p from Pl[g][k] + e_k (mod p), when
 // drop -- and the rows pass stores out[g][k][i] = (pk_k[i] U[g][i] + NTT_i(x)) (times
-// p^-1 when drop) (+ plain[g][i] for k = 0).  Es: [m][2][N] signed errors; Pl: [m][2][N]
+// p^-1 when drop) (+ plain[g][i] for k = 0).  Es: [m][2][N] signed errors (bytes); Pl: [m][2][N]
 // coefficient form; U: [m][L1][N] NTT(u); pk: [2][K][N]; out: [m][2][L][N].
 struct EncArgs {
-    const int64_t *Es;
+    const int8_t *Es;
     const uint64_t *Pl;
     const uint64_t *pk;
     const uint64_t *U;
@@ -145,6 +145,10 @@ struct EncArgs {
     uint32_t K, L1, L;
     bool drop;
 };
+// U[g][i] = forward transform (fully reduced) of the signed bytes Us[g] modulo primes[i],
+// g < m, i < L1 (N >= 2^13; returns false and does nothing otherwise).
+bool ntt_forward_small(const int8_t *Us, uint64_t *U, uint32_t L1, uint32_t m, const DevPrime *primes, int logn,
+                       hipStream_t stream);
 bool ntt_encrypt_ckks(const EncArgs &args, uint32_t m, const DevPrime *primes, int logn, hipStream_t stream);
 
 // ---- grouped launches (ciphertexts at several levels, one launch per stage) ----------
