@@ -13,6 +13,21 @@ struct Context;
 
 // Offsets (in 64-bit words) into one device buffer; all Shoup operands are stored as
 // (w, floor(w 2^64 / p)) pairs.
+// A base conversion's matrix for the matrix cores (conv_tile in behz.hip): operand A of
+// 32 x 32 x 32 int8 products, 4 outputs x 8 byte weights by 4 terms x 8 byte digits per
+// step, and each output's reduction constants.  terms == 0: the shape or the primes are
+// outside its range, and the conversion runs on the vector unit.
+struct ConvOut {
+    uint64_t p, neg_p;
+    uint64_t bias_lo, bias_hi;       // K p = bias_hi 2^32 + bias_lo, K p above every negative sum
+    uint32_t shift, m;               // floor(V / p) >= mulhi(V >> (32 + shift), m) > V / p - 3
+};
+struct ConvDev {
+    uint32_t terms = 0, steps = 0, outputs = 0;
+    const uint64_t *a = nullptr;     // [ceil(outputs / 4)][steps][64 lanes][2]
+    const ConvOut *out = nullptr;    // [outputs]
+};
+
 struct BehzDev {
     uint32_t L, bsz, bsk;            // |q|, |B|, |Bsk| = |B| + 1
     uint64_t m_sk, m_tilde_neg_inv_q; // m_sk; -prod(q)^-1 mod 2^32
@@ -41,6 +56,7 @@ struct BehzDev {
     // multiplyAddPlainWithScalingVariant (src/utils/scalingvariant.cpp:48-86)
     uint64_t q_mod_t;                // prod(q) mod t
     const uint64_t *delta;           // [L][2]   floor(prod(q)/t) mod q_j
+    ConvDev ext_conv, floor_conv, sk_conv;
 };
 
 struct BehzLevel {

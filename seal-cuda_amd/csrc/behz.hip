@@ -224,6 +224,180 @@ __global__ __launch_bounds__(BT) void behz_sk_kernel(const uint64_t *__restrict_
     }
 }
 
+// ---- the same conversions on the matrix cores --------------------------------------
+// A conversion sum_j y_j M[i][j] mod p_i is a product by a constant matrix, the same for every
+// coefficient.  With y_j in balanced bytes (y_j = sum_a d_a 2^(8a), d_a in [-128, 127]) and the
+// constants C[i][j][a] = M[i][j] 2^(8a) mod p_i in balanced bytes too,
+//   V_i = sum_b 2^(8b) s_b,  s_b = sum_{j,a} d_{j,a} c_{i,j,a,b},
+// is congruent to the sum and below terms 2^10 p_i in magnitude: 8 int8 dot products of
+// 8 terms each (v_mfma_i32_32x32x32_i8, |s_b| < terms 2^17), put together and reduced with some
+// 25 vector instructions, where the vector unit spends 8 multiply-adds per term and output.
+// A term of its own carries smMrq's / Shenoy-Kumaresan's centred correction word.
+// A wave owns 4 outputs x 64 coefficients at a time: a lane's 16 accumulators are the 8 sums of
+// 2 outputs at one coefficient.  CF coefficients' digits are staged in LDS once for all outputs.
+// At N = 2^16, L = 24, 32 pairs: extend 1,073 -> 692 us (each operand), floor 1,836 -> 1,286,
+// Shenoy-Kumaresan 1,626 -> 1,003 (2.4, 3.0 and 2.5 TB/s).  The vector-unit kernels above keep
+// N < 128, more than 48 terms, and outputs below 2^33.
+constexpr int CF = 128;
+constexpr int CT = 256;
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+__host__ __device__ __forceinline__ uint64_t balanced(uint64_t y) {
+    return (y + 0x8080808080808080ull) ^ 0x8080808080808080ull;
+}
+__device__ __forceinline__ uint64_t unbalanced(uint64_t d) {
+    return (d ^ 0x8080808080808080ull) - 0x8080808080808080ull;
+}
+
+// V mod p from the 8 sums of one output.
+__device__ __forceinline__ uint64_t conv_value(const int (&s)[8], const ConvOut &c) {
+    const int t01 = s[0] + s[1] * 256, t23 = s[2] + s[3] * 256, t45 = s[4] + s[5] * 256, t67 = s[6] + s[7] * 256;
+    const int64_t lo = (int64_t)c.bias_lo + t01 + (int64_t)t23 * 65536;
+    const int64_t hi = (int64_t)c.bias_hi + t45 + (int64_t)t67 * 65536 + (lo >> 32);  // V = hi 2^32 + lo mod 2^32
+    const uint32_t Q = __umulhi((uint32_t)((uint64_t)hi >> c.shift), c.m);
+    const uint64_t v = (uint64_t)hi << 32 | (uint32_t)lo;
+    uint64_t r = v + (uint64_t)Q * c.neg_p;  // V - Q p in [0, 3p)
+    r = csub(r, c.p);
+    return csub(r, c.p);
+}
+
+// All outputs of the block's CF coefficients: emit(output, coefficient, value, x) with
+// x = fetch(output, coefficient) requested before the products.
+template <class Fetch, class Emit>
+__device__ __forceinline__ void conv_outputs(const ulonglong2 *dig, const ConvOut *outs, const ConvDev &C,
+                                             const Fetch &fetch, const Emit &emit) {
+    const int lane = threadIdx.x & 63, h = lane >> 5, col = lane & 31;
+    const uint32_t units = (C.outputs + 3) / 4 * 2;
+    for (uint32_t u = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); u < units; u += CT / 64) {
+        const uint32_t og = u >> 1;
+        const int c0 = (int)(u & 1) * 64 + col;
+        const v4i *a = (const v4i *)C.a + (size_t)og * C.steps * 64 + lane;
+        decltype(fetch(0u, 0)) x[2][2];
+#pragma unroll
+        for (int q = 0; q < 2; q++)
+#pragma unroll
+            for (int t = 0; t < 2; t++) x[q][t] = fetch(min(og * 4 + 2 * h + q, C.outputs - 1), c0 + 32 * t);
+        v16i acc[2] = {};
+        v4i an = a[0];
+        for (uint32_t s = 0; s < C.steps; s++) {
+            const v4i av = an;
+            an = a[(size_t)min(s + 1, C.steps - 1) * 64];
+            const ulonglong2 *d = dig + (2 * s + h) * CF + c0;
+            const v4i b0 = *(const v4i *)d, b1 = *(const v4i *)(d + 32);
+            acc[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, b0, acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, b1, acc[1], 0, 0, 0);
+        }
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const uint32_t o = og * 4 + 2 * h + q;
+            if (o >= C.outputs) continue;
+            const ConvOut co = outs[o];
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                int sum[8];
+#pragma unroll
+                for (int b = 0; b < 8; b++) sum[b] = acc[t][8 * q + b];
+                emit(o, c0 + 32 * t, conv_value(sum, co), x[q][t]);
+            }
+        }
+    }
+}
+
+enum ConvStage { CONV_EXTEND, CONV_FLOOR, CONV_SK };
+
+// (1)-(2) extend: in [P][L][N] base q -> out [P][bsk][N]; (6)-(7) floor: in = Tq [P][L][N], tb
+// [P][bsk][N] -> out [P][bsk][N]; (8) sk: in = Z [P][bsk][N] -> out [P][L][N].  N >= CF.
+template <int STAGE>
+__global__ __launch_bounds__(CT) void behz_conv_kernel(const uint64_t *__restrict__ in, const uint64_t *__restrict__ tb,
+                                                       uint64_t *__restrict__ out, BehzDev B,
+                                                       const DevPrime *__restrict__ qp, int logn, uint32_t blocks) {
+    extern __shared__ ulonglong2 dig[];  // [2 steps][CF] digit pairs, then the outputs' constants
+    const ConvDev &C = STAGE == CONV_EXTEND ? B.ext_conv : STAGE == CONV_FLOOR ? B.floor_conv : B.sk_conv;
+    ConvOut *outs = (ConvOut *)(dig + 2 * C.steps * CF);
+    const size_t n = (size_t)1 << logn;
+    const int tid = threadIdx.x, cc = tid % CF, part = tid / CF;
+    for (uint32_t e = tid; e < C.outputs; e += CT) outs[e] = C.out[e];
+    const uint32_t terms = STAGE == CONV_SK ? B.bsz : B.L;  // without the correction's
+    const uint32_t rows_in = STAGE == CONV_SK ? B.bsk : B.L, rows_out = STAGE == CONV_SK ? B.L : B.bsk;
+    const uint64_t *pair = STAGE == CONV_EXTEND ? B.mt_qhat_inv : STAGE == CONV_FLOOR ? B.t_qhat_inv : B.bhat_inv;
+    const DevPrime *from = STAGE == CONV_SK ? B.bsk_primes : qp;
+    auto put = [&](uint32_t j, uint64_t d) { ((uint64_t *)(dig + (j >> 1) * CF + cc))[j & 1] = d; };
+    for (uint32_t blk = blockIdx.x; blk < blocks; blk += gridDim.x) {
+        const size_t at = (size_t)blk * CF, p = at >> logn, c = (at & (n - 1)) + cc;
+        const uint64_t *x = in + p * rows_in * n + c;
+        // eight words requested at a time (one by one, their latencies were most of the block)
+        constexpr int STEP = CT / CF, AHEAD = 8;
+        for (uint32_t j0 = part; j0 < C.steps * 4; j0 += AHEAD * STEP) {
+            uint64_t v[AHEAD];
+#pragma unroll
+            for (int k = 0; k < AHEAD; k++) v[k] = x[(size_t)min<uint32_t>(j0 + k * STEP, terms - 1) * n];
+#pragma unroll
+            for (int k = 0; k < AHEAD; k++) {
+                const uint32_t j = j0 + k * STEP;
+                if (j >= C.steps * 4) break;
+                uint64_t d = 0;
+                if (j < terms) d = balanced(shoup_pair(v[k], pair + 2 * j, from[j].q));
+                if (STAGE == CONV_FLOOR || j != terms) put(j, d);
+            }
+        }
+        if constexpr (STAGE != CONV_FLOOR) {
+            __syncthreads();
+            if (part == 0) {  // the correction's word
+                auto y = [&](uint32_t j) { return unbalanced(((const uint64_t *)(dig + (j >> 1) * CF + cc))[j & 1]); };
+                int64_t w;
+                if constexpr (STAGE == CONV_EXTEND) {
+                    const uint64_t *row_mt = B.qhat_ext + (size_t)B.bsk * B.L;
+                    uint64_t s_mt = 0;
+                    for (uint32_t j = 0; j < terms; j++) s_mt += y(j) * row_mt[j];
+                    // centred: m_tilde is a power of two
+                    w = (int64_t)(int32_t)(uint32_t)((s_mt & 0xffffffffull) * B.m_tilde_neg_inv_q);
+                } else {
+                    const DevPrime &Msk = B.bsk_primes[B.bsz];
+                    const_u64 *bm = (const_u64 *)B.bhat_mod_msk;
+                    Acc3 acc{0, 0, 0};
+                    for (uint32_t j = 0; j < terms; j++) mac<true>(acc, y(j), bm[j]);
+                    const uint64_t conv = acc_reduce(acc, Msk), zmsk = x[(size_t)B.bsz * n];
+                    const uint64_t alpha = shoup(conv + B.m_sk - zmsk, B.inv_prod_B_msk, B.inv_prod_B_msk_shoup, B.m_sk);
+                    w = alpha > B.m_sk_half ? (int64_t)(B.m_sk - alpha) : -(int64_t)alpha;
+                }
+                put(terms, balanced((uint64_t)w));
+            }
+        }
+        __syncthreads();
+        const size_t o0 = p * rows_out * n + (c - cc);
+        if constexpr (STAGE == CONV_FLOOR) {
+            // the rows carry prod(q)^-1: Z = t Tb q^-1 - conv q^-1 mod p
+            struct Tb {
+                uint64_t v;
+                ulonglong2 w;
+            };
+            conv_outputs(
+                dig, outs, C,
+                [&](uint32_t o, int col) {
+                    return Tb{tb[o0 + (size_t)o * n + col], *(const ulonglong2 *)(B.t_inv_q_bsk + 2 * o)};
+                },
+                [&](uint32_t o, int col, uint64_t v, const Tb &x) {
+                    const uint64_t q = outs[o].p;
+                    out[o0 + (size_t)o * n + col] = submod(shoup(x.v, x.w.x, x.w.y, q), v, q);
+                });
+        } else {
+            conv_outputs(
+                dig, outs, C, [](uint32_t, int) { return 0; },
+                [&](uint32_t o, int col, uint64_t v, int) { out[o0 + (size_t)o * n + col] = v; });
+        }
+        __syncthreads();  // the digits are read before the next coefficients' overwrite them
+    }
+}
+
+template <int STAGE>
+void launch_conv(const uint64_t *in, const uint64_t *tb, uint64_t *out, const BehzDev &B, const ConvDev &C,
+                 const DevPrime *qp, int logn, size_t total, hipStream_t st) {
+    const uint32_t blocks = (uint32_t)(total / CF);
+    const size_t lds = (size_t)C.steps * 2 * CF * sizeof(ulonglong2) + C.outputs * sizeof(ConvOut);
+    behz_conv_kernel<STAGE><<<blocks < (1u << 20) ? blocks : 1u << 20, CT, lds, st>>>(in, tb, out, B, qp, logn, blocks);
+}
+
 // Runs f(std::integral_constant<int, OB>) for the OB out_group picks.
 template <class F>
 void with_group(int ob, F &&f) {
@@ -316,6 +490,7 @@ void build_behz_level(Context &c, uint32_t L, BehzLevel &out) {
     const size_t o_qhat_floor = put(v);
     v.clear();
     for (uint32_t i = 0; i < bsk; i++) v.push_back(mulmod(t % Bsk[i], inv_q[i], Bsk[i]));
+    if (words.size() & 1) words.push_back(0);  // read as 16-byte pairs
     const size_t o_t_inv_q = put(shoup_vec(v, Bsk));
     v.clear();
     for (uint32_t j = 0; j < L; j++) v.push_back(mulmod(t % q[j], qhat_inv[j], q[j]));
@@ -353,6 +528,59 @@ void build_behz_level(Context &c, uint32_t L, BehzLevel &out) {
     for (uint32_t j = 0; j < L; j++) dl.push_back(big_mod_word(qd, q[j]));
     const size_t o_delta = put(shoup_vec(dl, q));
 
+    // the conversions' matrices for the matrix cores, the correction word's column last
+    struct Conv {
+        ConvDev *dev;
+        size_t o_a, o_out;
+    };
+    std::vector<Conv> convs;
+    auto put_conv = [&](ConvDev &dev, size_t o_rows, uint32_t terms, const uint64_t *extra,
+                        const std::vector<uint64_t> &mods) {
+        const uint32_t T = terms + (extra ? 1 : 0), O = (uint32_t)mods.size();
+        for (uint64_t p : mods)
+            if (p >> 61 || p < (uint64_t(1) << 33)) return;  // the quotient estimate's range
+        if (T > 48 || c.n < CF) return;  // 64 KB of staged digits; whole tiles of coefficients
+        dev.terms = T;
+        dev.steps = (T + 3) / 4;
+        dev.outputs = O;
+        std::vector<uint64_t> a((size_t)((O + 3) / 4) * dev.steps * 128, 0);
+        for (uint32_t o = 0; o < O; o++)
+            for (uint32_t j = 0; j < T; j++) {
+                uint64_t v = j < terms ? words[o_rows + (size_t)o * terms + j] : extra[o];
+                for (int dgt = 0; dgt < 8; dgt++) {
+                    const uint64_t bytes = balanced(v);
+                    for (int b = 0; b < 8; b++) {
+                        // row of (output o % 4, weight b): accumulator r of lane half hr
+                        const uint32_t hr = (o % 4) / 2, r = (o % 2) * 8 + b;
+                        const uint32_t row = (r & 3) + 8 * (r >> 2) + 4 * hr, lane = row + 32 * ((j % 4) / 2);
+                        const size_t word = (((size_t)(o / 4) * dev.steps + j / 4) * 64 + lane) * 2 + (j & 1);
+                        a[word] |= (bytes >> (8 * b) & 0xff) << (8 * dgt);
+                    }
+                    v = (uint64_t)(((unsigned __int128)v << 8) % mods[o]);
+                }
+            }
+        std::vector<uint64_t> oc;
+        for (uint64_t p : mods) {
+            const unsigned __int128 bias = (unsigned __int128)p * (T * 1024);
+            int bits = 64 - __builtin_clzll(p);
+            const uint32_t shift = bits > 46 ? bits - 46 : 0;
+            const uint32_t m = (uint32_t)(((unsigned __int128)1 << (64 + shift)) / p);
+            oc.insert(oc.end(), {p, 0 - p, (uint64_t)bias & 0xffffffffull, (uint64_t)(bias >> 32),
+                                 (uint64_t)m << 32 | shift});
+        }
+        if (words.size() & 1) words.push_back(0);  // 16-byte operand loads
+        const size_t o_a = put(a);
+        convs.push_back(Conv{&dev, o_a, put(oc)});
+    };
+    static_assert(sizeof(ConvOut) == 40, "five words per output");
+    {
+        const std::vector<uint64_t> qe(words.begin() + o_q_ext, words.begin() + o_q_ext + bsk);
+        const std::vector<uint64_t> pb(words.begin() + o_prodB_q, words.begin() + o_prodB_q + L);
+        put_conv(out.dev.ext_conv, o_qhat_ext, L, qe.data(), Bsk);
+        put_conv(out.dev.floor_conv, o_qhat_floor, L, nullptr, Bsk);
+        put_conv(out.dev.sk_conv, o_bhat_q, (uint32_t)bsz, pb.data(), q);
+    }
+
     out.tables = DevBuf(words.size() * 8);
     SHC_HIP(hipMemcpy(out.tables.ptr, words.data(), words.size() * 8, hipMemcpyHostToDevice));
     std::vector<DevPrime> bp;
@@ -362,6 +590,10 @@ void build_behz_level(Context &c, uint32_t L, BehzLevel &out) {
 
     const uint64_t *base = out.tables.as<const uint64_t>();
     BehzDev &d = out.dev;
+    for (const Conv &v : convs) {
+        v.dev->a = base + v.o_a;
+        v.dev->out = reinterpret_cast<const ConvOut *>(base + v.o_out);
+    }
     d.L = L;
     d.bsz = (uint32_t)bsz;
     d.bsk = bsk;
@@ -424,10 +656,15 @@ void bfv_multiply(const Context &c, const uint64_t *a, const uint64_t *b, uint64
     const DevPrime *bp = B.bsk_primes;
     const size_t ext = (size_t)count * 2 * n;
     const size_t lds = (size_t)(L > B.bsz ? L : B.bsz) * CW * 8;
-    with_group(out_group(B.bsk), [&](auto ob) {
-        behz_extend_kernel<decltype(ob)::value><<<grid_for(ext), BT, lds, st>>>(a, Ab, B, qp, logn, ext);
-        behz_extend_kernel<decltype(ob)::value><<<grid_for(ext), BT, lds, st>>>(b, Bb, B, qp, logn, ext);
-    });
+    if (B.ext_conv.terms) {
+        launch_conv<CONV_EXTEND>(a, nullptr, Ab, B, B.ext_conv, qp, logn, ext, st);
+        launch_conv<CONV_EXTEND>(b, nullptr, Bb, B, B.ext_conv, qp, logn, ext, st);
+    } else {
+        with_group(out_group(B.bsk), [&](auto ob) {
+            behz_extend_kernel<decltype(ob)::value><<<grid_for(ext), BT, lds, st>>>(a, Ab, B, qp, logn, ext);
+            behz_extend_kernel<decltype(ob)::value><<<grid_for(ext), BT, lds, st>>>(b, Bb, B, qp, logn, ext);
+        });
+    }
     launch_check("behz_extend");
     // the four forward transforms in one launch per pass, a and b read in place (their
     // transforms land in Aq, Bq); then the two tensor products and the two inverse
@@ -457,13 +694,19 @@ void bfv_multiply(const Context &c, const uint64_t *a, const uint64_t *b, uint64
         ntt_inverse(Tb, count * 3 * bsk, bsk, bp, logn, NTT_FULL, st);
     }
     const size_t fl = (size_t)count * 3 * n;
-    with_group(out_group(B.bsk), [&](auto ob) {
-        behz_floor_kernel<decltype(ob)::value><<<grid_for(fl), BT, lds, st>>>(Tq, Tb, Z, B, qp, logn, fl);
-    });
+    if (B.floor_conv.terms)
+        launch_conv<CONV_FLOOR>(Tq, Tb, Z, B, B.floor_conv, qp, logn, fl, st);
+    else
+        with_group(out_group(B.bsk), [&](auto ob) {
+            behz_floor_kernel<decltype(ob)::value><<<grid_for(fl), BT, lds, st>>>(Tq, Tb, Z, B, qp, logn, fl);
+        });
     launch_check("behz_floor");
-    with_group(out_group(B.L), [&](auto ob) {
-        behz_sk_kernel<decltype(ob)::value><<<grid_for(fl), BT, lds, st>>>(Z, out, B, qp, logn, fl);
-    });
+    if (B.sk_conv.terms)
+        launch_conv<CONV_SK>(Z, nullptr, out, B, B.sk_conv, qp, logn, fl, st);
+    else
+        with_group(out_group(B.L), [&](auto ob) {
+            behz_sk_kernel<decltype(ob)::value><<<grid_for(fl), BT, lds, st>>>(Z, out, B, qp, logn, fl);
+        });
     launch_check("behz_sk");
 }
 

@@ -206,6 +206,42 @@ def test_bfv_multiply(logn, bits, L, t, count):
         np.testing.assert_array_equal(got[c], ck.bfv_multiply(a[c], b[c], moduli[:L], t, logn))
 
 
+@pytest.mark.parametrize("logn,bits,L,count", [
+    # base conversions on the matrix cores: one tile of 128 coefficients, 1 to 12 steps of
+    # four terms with and without the correction word opening a new one, outputs that fill
+    # and leave part of a wave's four, primes of 34 to 60 bits
+    (7, [34, 36, 40, 60], 3, 1),
+    (8, [60] * 5, 4, 3),
+    (9, [45, 50, 55, 60, 60, 48, 47, 46, 60], 8, 2),
+    (8, [60] * 48, 47, 1),
+    # past 48 terms, and 30-bit outputs: the vector unit
+    (8, [60] * 49, 48, 1),
+    (8, [30, 60, 60], 2, 2),
+])
+@pytest.mark.parametrize("words", ["uniform", "largest", "small"])
+def test_bfv_multiply_conversions(logn, bits, L, count, words):
+    t = 65537 if logn >= 8 else 257
+    ctx, moduli = make_ctx(BFV, logn, bits, t)
+    n = 1 << logn
+    rng = np.random.default_rng(400 + logn + L)
+    a = ck.uniform_residues(rng, (count, 2, L, n), moduli[:L])
+    b = ck.uniform_residues(rng, (count, 2, L, n), moduli[:L])
+    q = np.array(moduli[:L], dtype=np.uint64)[None, None, :, None]
+    if words == "largest":
+        a[:], b[:] = q - 1, q - 1
+    elif words == "small":  # single small coefficients: digits and corrections near zero
+        a[:], b[:] = 0, 0
+        a[..., 3], b[..., 5] = 1, 2
+        a[:, 1] = (q - 1)[0]
+    da, db, do = to_dev(a), to_dev(b), empty_dev((count, 3, L, n))
+    ws_bytes = ctx.multiply_workspace_size(count, L)
+    ws = empty_dev((ws_bytes + 7) // 8)
+    ctx.multiply(da.data_ptr(), db.data_ptr(), do.data_ptr(), count, L, ws.data_ptr(), ws_bytes, stream())
+    got = from_dev(do)
+    for c in range(count):
+        np.testing.assert_array_equal(got[c], ck.bfv_multiply(a[c], b[c], moduli[:L], t, logn))
+
+
 def test_bfv_multiply_target_shape():
     """N = 2^16, 24 data primes of 60 bits, t = 65537 (one pair)."""
     logn, L, t = 16, 24, 65537
