@@ -10,6 +10,7 @@
 #include "ckks_encoder.h"
 #include "modarith.h"
 #include "ntt.h"
+#include "ntt_device.h"
 #include <algorithm>
 #include <cmath>
 #include <complex>
@@ -175,33 +176,41 @@ __device__ __forceinline__ void wave_max_atomic(unsigned long long *dst, unsigne
     }
 }
 
+// |d| too large (2^128 up), inf or NaN: rejected by the range check, zero meanwhile.
+__device__ __forceinline__ double coeff_or_zero(double d) {
+    return fabs(d) < 340282366920938463463374607431768211456.0 ? d : 0.0;
+}
+// d mod q for a whole d below 2^128 in magnitude; wide: some |d| >= 2^63 in the wave (else one
+// word per coefficient, a third of the instructions).
+__device__ __forceinline__ uint64_t coeff_mod(double d, bool wide, const DevPrime &P) {
+    const double two64 = 18446744073709551616.0;
+    const bool neg = signbit(d);
+    d = fabs(d);
+    uint64_t r;
+    if (wide) {
+        // d = hi 2^64 + lo exactly: scaling by a power of two is exact, and d mod 2^64 (the
+        // low bits of a 53-bit mantissa) is representable, so the subtraction is exact
+        const double hid = floor(d * (1.0 / two64));
+        r = barrett128(u128{(uint64_t)(d - hid * two64), (uint64_t)hid}, P.q, P.ratio_lo, P.ratio_hi);
+    } else {
+        r = barrett64((uint64_t)d, P.q, P.ratio_hi);
+    }
+    return neg ? negmod(r, P.q) : r;
+}
+
 __global__ void round_reduce_kernel(const double2 *__restrict__ a, uint64_t *__restrict__ out,
                                     const DevPrime *__restrict__ primes, uint32_t L, int logn,
                                     unsigned long long *maxbits) {
     const size_t n = (size_t)1 << logn;
-    const double two64 = 18446744073709551616.0;
     a += blockIdx.y * n;
     out += blockIdx.y * L * n;
     maxbits += blockIdx.y;
     for (size_t c = (size_t)blockIdx.x * TPB + threadIdx.x; c < n; c += (size_t)gridDim.x * TPB) {
         double d = round(a[c].x);
-        const bool neg = signbit(d);
-        d = fabs(d);
-        wave_max_atomic(maxbits, (unsigned long long)__double_as_longlong(d));
-        if (!(d < two64 * two64)) d = 0;  // too large, inf or NaN: rejected on the host after the range check
-        // d = hi 2^64 + lo exactly: scaling by a power of two is exact, and d mod 2^64 (the
-        // low bits of a 53-bit mantissa) is representable, so the subtraction is exact
-        const double hid = floor(d * (1.0 / two64));
-        const uint64_t hi = (uint64_t)hid;
-        const uint64_t lo = (uint64_t)(d - hid * two64);
-        // below 2^64 (any usual scale) one word per coefficient: a third of the instructions
-        const bool wide = __any(hi != 0);
-        for (uint32_t l = 0; l < L; l++) {
-            const DevPrime &P = primes[l];
-            const uint64_t r = wide ? barrett128(u128{lo, hi}, P.q, P.ratio_lo, P.ratio_hi)
-                                    : barrett64(lo, P.q, P.ratio_hi);
-            out[l * n + c] = neg ? negmod(r, P.q) : r;
-        }
+        wave_max_atomic(maxbits, (unsigned long long)__double_as_longlong(fabs(d)));
+        d = coeff_or_zero(d);
+        const bool wide = __any(!(fabs(d) < 9223372036854775808.0));
+        for (uint32_t l = 0; l < L; l++) out[l * n + c] = coeff_mod(d, wide, primes[l]);
     }
 }
 
@@ -254,39 +263,79 @@ __global__ void zero_if_rejected_kernel(uint64_t *__restrict__ plain, const int 
     for (size_t i = (size_t)blockIdx.x * TPB + threadIdx.x; i < words; i += (size_t)gridDim.x * TPB) plain[i] = 0;
 }
 
-__global__ void compose_kernel(const uint64_t *__restrict__ c, double2 *__restrict__ a, CkksLevelDev T,
-                               const DevPrime *__restrict__ primes, int logn, double inv_scale) {
-    const size_t n = (size_t)1 << logn;
-    const double two64 = 18446744073709551616.0;
-    c += blockIdx.y * T.L * n;
-    a += blockIdx.y * n;
-    for (size_t i = (size_t)blockIdx.x * TPB + threadIdx.x; i < n; i += (size_t)gridDim.x * TPB) {
-        double f = 0.0;
-        uint64_t lo = 0, hi = 0;
-        for (uint32_t j = 0; j < T.L; j++) {
-            const uint64_t y = shoup(c[j * n + i], T.qhat_inv[2 * j], T.qhat_inv[2 * j + 1], primes[j].q);
-            f += (double)y * T.inv_q[j];
-            // (lo, hi) += y * qhat_j mod 2^128
-            const u128 p = mul64x64(y, T.qhat128[2 * j]);
-            const uint64_t nlo = lo + p.lo;
-            hi += p.hi + y * T.qhat128[2 * j + 1] + (nlo < lo ? 1ull : 0ull);
-            lo = nlo;
-        }
+// The CRT composition of one coefficient: limb by limb (add), then the centred value.
+struct Compose {
+    double f = 0.0;
+    uint64_t lo = 0, hi = 0;
+    __device__ __forceinline__ void add(uint64_t x, const CkksLevelDev &T, uint32_t j, uint64_t q) {
+        const uint64_t y = shoup(x, T.qhat_inv[2 * j], T.qhat_inv[2 * j + 1], q);
+        f += (double)y * T.inv_q[j];
+        // (lo, hi) += y * qhat_j mod 2^128
+        const u128 p = mul64x64(y, T.qhat128[2 * j]);
+        const uint64_t nlo = lo + p.lo;
+        hi += p.hi + y * T.qhat128[2 * j + 1] + (nlo < lo ? 1ull : 0ull);
+        lo = nlo;
+    }
+    __device__ __forceinline__ double value(const CkksLevelDev &T) const {
+        const double two64 = 18446744073709551616.0;
         const uint64_t k = (uint64_t)llrint(f);
         // x = acc - k Q (mod 2^128), read as a signed 128-bit integer
         const u128 kq = mul64x64(k, T.Q_lo);
         const uint64_t kq_hi = kq.hi + k * T.Q_hi;
         const uint64_t xlo = lo - kq.lo;
         const uint64_t xhi = hi - kq_hi - (lo < kq.lo ? 1ull : 0ull);
-        double v;
         if (xhi >> 63) {
             const uint64_t nlo = ~xlo + 1, nhi = ~xhi + (nlo == 0 ? 1ull : 0ull);
-            v = -((double)nhi * two64 + (double)nlo);
-        } else {
-            v = (double)xhi * two64 + (double)xlo;
+            return -((double)nhi * two64 + (double)nlo);
         }
-        a[i] = make_double2(v * inv_scale, 0.0);
+        return (double)xhi * two64 + (double)xlo;
     }
+};
+
+__global__ void compose_kernel(const uint64_t *__restrict__ c, double2 *__restrict__ a, CkksLevelDev T,
+                               const DevPrime *__restrict__ primes, int logn, double inv_scale) {
+    const size_t n = (size_t)1 << logn;
+    c += blockIdx.y * T.L * n;
+    a += blockIdx.y * n;
+    for (size_t i = (size_t)blockIdx.x * TPB + threadIdx.x; i < n; i += (size_t)gridDim.x * TPB) {
+        Compose x;
+        for (uint32_t j = 0; j < T.L; j++) x.add(c[j * n + i], T, j, primes[j].q);
+        a[i] = make_double2(x.value(T) * inv_scale, 0.0);
+    }
+}
+
+// The same composition fused into the inverse transforms' columns pass, for batches that fill
+// the chip with one block per 16 columns of a plaintext: a block takes its tile of every limb
+// in turn (after the rows pass) and keeps the composition in registers, so that the
+// coefficients never go to HBM (written and read back, 3.2 GB for 128 plaintexts at N = 2^16,
+// L = 24: 823 + 400 us, fused 1,094, of which some 0.9 ms is instruction issue).  8 values per
+// thread.  (The encoder's rounding fused into its columns pass the same way measured no
+// different, 1,118 against 611 + 515 us: its reductions bound it.)
+constexpr int EF = 3;
+constexpr uint64_t FUSED_BLOCKS = 512;
+
+template <int LOGN>
+__global__ __launch_bounds__(16 << (LOGN / 2 - EF)) void ntt_cols_compose_kernel(
+    const uint64_t *__restrict__ rows, double2 *__restrict__ a, CkksLevelDev T, const DevPrime *__restrict__ primes,
+    double inv_scale) {
+    constexpr int K = LOGN / 2, C = 1 << (LOGN - K), SUBS = 16, TILES = C / SUBS;
+    __shared__ uint64_t tile[SUBS << K];
+    const int tid = threadIdx.x, col = tid % SUBS, t = tid / SUBS;
+    const size_t p = blockIdx.x / TILES, c = (size_t)(blockIdx.x % TILES) * SUBS + col;
+    auto addr = [col](int idx) { return idx * SUBS + col; };
+    Compose x[1 << EF];
+    for (uint32_t l = 0; l < T.L; l++) {
+        const DevPrime &P = primes[l];
+        const uint64_t *in = rows + ((p * T.L + l) << LOGN) + c;
+        auto load = [in](int idx, int) { return in[(size_t)idx * C]; };
+        auto store = [&](int, uint64_t v, int j) { x[j].add(finish<true, true>(v, P), T, l, P.q); };
+        if (l) __syncthreads();  // the previous limb's last phase has read the tile
+        run_phases<K, EF, true, false>(tile, addr, load, store, t, GlobalTw<LOGN, true, ulonglong2>{P.inv, 0, 0},
+                                       bf_const(P), true);
+    }
+#pragma unroll
+    for (int j = 0; j < (1 << EF); j++)
+        a[(p << LOGN) + (size_t)phase_index<K, EF, 0, EF>(t, j) * C + c] = make_double2(x[j].value(T) * inv_scale, 0.0);
 }
 
 __global__ void gather_kernel(const double2 *__restrict__ a, double *__restrict__ values, int logn) {
@@ -298,6 +347,43 @@ __global__ void gather_kernel(const double2 *__restrict__ a, double *__restrict_
         values[2 * i] = v.x;
         values[2 * i + 1] = v.y;
     }
+}
+
+// Plaintexts enough that one block per 16 columns of each fills the chip (N >= 2^13).
+bool fused_columns(int logn, uint32_t batch) {
+    return logn >= 13 && logn <= 17 && ((uint64_t)batch << (logn - logn / 2 - 4)) >= FUSED_BLOCKS;
+}
+
+template <class F>
+void with_degree(int logn, F &&f) {
+    switch (logn) {
+        case 13: f(std::integral_constant<int, 13>{}); break;
+        case 14: f(std::integral_constant<int, 14>{}); break;
+        case 15: f(std::integral_constant<int, 15>{}); break;
+        case 16: f(std::integral_constant<int, 16>{}); break;
+        default: f(std::integral_constant<int, 17>{}); break;
+    }
+}
+
+// Inverse transforms of plain [batch][L][N] (through `rows`) composed into a [batch][N].
+void inverse_compose(const Context &c, const uint64_t *plain, uint64_t *rows, double2 *a, const CkksLevelDev &T,
+                     uint32_t L, uint32_t batch, double inv_scale, hipStream_t st) {
+    const LimbGrid lg{1, L, L, batch};
+    with_degree(c.logn, [&](auto ln) {
+        constexpr int LOGN = decltype(ln)::value;
+        with_shape<LOGN>((uint64_t)L * batch, [&](auto s) {
+            using S = PassShape<LOGN, decltype(s)::value>;
+            const bool mx = rows_mixed<LOGN, S::K2, S::RS>(batch);
+            const uint32_t blocks = L * rows_blocks_per_prime<LOGN, S::K2, S::E, S::RS>(batch, mx);
+            with_bool(mx, [&](auto m) {
+                ntt_rows_from_kernel<LOGN, S::K2, S::E, S::RS, true, false, true, decltype(m)::value>
+                    <<<blocks, S::RS << (S::K2 - S::E), 0, st>>>(plain, lg, rows, c.primes(), lg, 0, batch);
+            });
+        });
+        ntt_cols_compose_kernel<LOGN><<<batch << (LOGN - LOGN / 2 - 4), 16 << (LOGN / 2 - EF), 0, st>>>(
+            rows, a, T, c.primes(), inv_scale);
+    });
+    launch_check("ckks inverse compose");
 }
 
 // ComplexRoots::getRoot (src/utils/croots.cpp:31-60)
@@ -474,9 +560,13 @@ void ckks_decode_many(const Context &c, const uint64_t *plain, uint32_t L, uint3
     const size_t n = c.n;
     uint64_t *cp = static_cast<uint64_t *>(ws);
     double2 *a = reinterpret_cast<double2 *>(static_cast<char *>(ws) + (((size_t)batch * L * n * 8 + 255) & ~size_t(255)));
-    const LimbGrid lg{1, L, L, batch};  // the plaintexts' limbs, transformed out of place
-    ntt_inverse_from(plain, lg, cp, lg, c.primes(), c.logn, NTT_FULL, st);
-    compose_kernel<<<dim3(blocks_for(n), batch), TPB, 0, st>>>(cp, a, T, c.primes(), c.logn, 1.0 / scale);
+    if (fused_columns(c.logn, batch) && (uint64_t)batch * L <= ((uint64_t(1) << 34) >> c.logn)) {
+        inverse_compose(c, plain, cp, a, T, L, batch, 1.0 / scale, st);
+    } else {
+        const LimbGrid lg{1, L, L, batch};  // the plaintexts' limbs, transformed out of place
+        ntt_inverse_from(plain, lg, cp, lg, c.primes(), c.logn, NTT_FULL, st);
+        compose_kernel<<<dim3(blocks_for(n), batch), TPB, 0, st>>>(cp, a, T, c.primes(), c.logn, 1.0 / scale);
+    }
     launch_dwt<false>(a, c.ckks->roots.as<const double2>(), c.logn, batch, 0.0, st);
     gather_kernel<<<dim3(blocks_for(n / 2), batch), TPB, 0, st>>>(a, values, c.logn);
     launch_check("ckks decode");

@@ -29,22 +29,6 @@
 namespace shc {
 namespace {
 
-// Rows pass of a transform whose input lies elsewhere: reads limb (i, j) from `src`
-// (grid slg) and writes it to `data` (grid lg), same shape.
-template <int LOGN, int K, int E, int SUBS, bool INV, bool LAST, bool FULL, bool MX = false>
-__global__ __launch_bounds__(SUBS << (K - E)) void ntt_rows_from_kernel(const uint64_t *__restrict__ src,
-                                                                       LimbGrid slg, uint64_t *__restrict__ data,
-                                                                       const DevPrime *__restrict__ primes,
-                                                                       LimbGrid lg, uint32_t j0, uint32_t jn) {
-    const GridAccess g{data, lg, LOGN};
-    const GridAccess s{const_cast<uint64_t *>(src), slg, LOGN};
-    rows_body<LOGN, K, E, SUBS, INV, false, MX>(
-        blockIdx.x, primes, lg.I, j0, jn, [&](uint32_t i, uint32_t j, size_t off) { return *s.at(i, j, off); },
-        [&](uint32_t i, uint32_t j, size_t off, uint64_t x) {
-            *g.at(i, j, off) = LAST ? finish<INV, FULL>(x, primes[i]) : x;
-        });
-}
-
 template <int LOGN, bool INV, bool FULL, bool SMALL>
 void launch_ntt_as(uint64_t *data, LimbGrid lg, uint32_t j0, uint32_t jn, const DevPrime *primes, hipStream_t st) {
     if constexpr (LOGN <= 12) {

@@ -108,7 +108,7 @@ __device__ __forceinline__ void phase_compute(uint64_t (&r)[1 << E], int t, cons
 // Runs all phases of a sub-transform.  The first phase reads its registers straight
 // from global memory through `load(idx, j)` (j: the register) and the last writes them
 // back through
-// `store(idx, value)`; in between, values cross threads through LDS at `addr(idx)`,
+// `store(idx, value)` or `store(idx, value, j)`; in between, values cross threads through LDS at `addr(idx)`,
 // so a pass makes one LDS round trip per phase boundary and one barrier each.
 template <int K, int E, bool INV, bool W, int P = 0, class Addr, class Load, class Store, class Tw>
 __device__ __forceinline__ void run_phases(uint64_t *tile, const Addr &addr, const Load &load, const Store &store,
@@ -130,8 +130,13 @@ __device__ __forceinline__ void run_phases(uint64_t *tile, const Addr &addr, con
 #pragma unroll
             for (int j = 0; j < (1 << E); j++) {
                 const int idx = phase_index<K, E, S0, EP>(t, j);
-                if (P == NP - 1) store(idx, W ? sub_if_ge_neg(r[j], bc.neg_eight_q) : r[j]);  // wide: [0,16q) -> [0,8q)
-                else tile[addr(idx)] = r[j];
+                if constexpr (P == NP - 1) {
+                    const uint64_t v = W ? sub_if_ge_neg(r[j], bc.neg_eight_q) : r[j];  // wide: [0,16q) -> [0,8q)
+                    if constexpr (std::is_invocable_v<Store, int, uint64_t, int>) store(idx, v, j);
+                    else store(idx, v);
+                } else {
+                    tile[addr(idx)] = r[j];
+                }
             }
         }
         if constexpr (P + 1 < NP) {
@@ -387,6 +392,22 @@ __global__ __launch_bounds__(SUBS << (K - E)) void ntt_cols_kernel(uint64_t *__r
     const GridAccess g{data, lg, LOGN};
     cols_body<LOGN, K, E, SUBS, INV>(
         blockIdx.x, primes, j0, jn, [&](uint32_t i, uint32_t j, size_t off) { return *g.at(i, j, off); },
+        [&](uint32_t i, uint32_t j, size_t off, uint64_t x) {
+            *g.at(i, j, off) = LAST ? finish<INV, FULL>(x, primes[i]) : x;
+        });
+}
+
+// Rows pass of a transform whose input lies elsewhere: reads limb (i, j) from `src`
+// (grid slg) and writes it to `data` (grid lg), same shape.
+template <int LOGN, int K, int E, int SUBS, bool INV, bool LAST, bool FULL, bool MX = false>
+__global__ __launch_bounds__(SUBS << (K - E)) void ntt_rows_from_kernel(const uint64_t *__restrict__ src,
+                                                                       LimbGrid slg, uint64_t *__restrict__ data,
+                                                                       const DevPrime *__restrict__ primes,
+                                                                       LimbGrid lg, uint32_t j0, uint32_t jn) {
+    const GridAccess g{data, lg, LOGN};
+    const GridAccess s{const_cast<uint64_t *>(src), slg, LOGN};
+    rows_body<LOGN, K, E, SUBS, INV, false, MX>(
+        blockIdx.x, primes, lg.I, j0, jn, [&](uint32_t i, uint32_t j, size_t off) { return *s.at(i, j, off); },
         [&](uint32_t i, uint32_t j, size_t off, uint64_t x) {
             *g.at(i, j, off) = LAST ? finish<INV, FULL>(x, primes[i]) : x;
         });

@@ -353,3 +353,23 @@ def test_encode_polynomial_rejects():
         ctx.ckks_encode_polynomial(bad.data_ptr(), 2, 2.0 ** 20, 2, plain.data_ptr(), eb.data_ptr(), ew, stream())
     with pytest.raises(hip().SealHipError, match="too large"):
         ctx.ckks_encode_polynomial(big.data_ptr(), n + 1, 1.0, 2, plain.data_ptr(), eb.data_ptr(), ew, stream())
+
+
+@pytest.mark.parametrize("logn,L,batch", [(13, 3, 64), (13, 1, 65), (14, 5, 64), (15, 2, 33), (16, 3, 32), (17, 2, 16)])
+def test_decode_batches_equal_single_plaintexts(logn, L, batch):
+    """Batches that take the composition fused into the transforms' last pass (512 blocks of 16
+    columns up) give the same doubles as plaintexts decoded alone."""
+    n = 1 << logn
+    moduli = ck.coeff_modulus_create(n, [60, 40, 50, 45, 60, 60][:L] + [60])
+    ctx = hip().Context(2, n, moduli)
+    rng = np.random.default_rng(logn + batch)
+    plain = to_dev(ck.uniform_residues(rng, (batch, L, n), moduli[:L]))
+    many = torch.empty((batch, n), dtype=torch.float64, device="cuda")
+    wb = ctx.ckks_decode_many_workspace_size(L, batch)
+    w = empty_dev(((wb + 7) // 8,))
+    ctx.ckks_decode_many(plain.data_ptr(), L, batch, 2.0 ** 20, many.data_ptr(), w.data_ptr(), wb, stream())
+    for p in (0, batch // 2, batch - 1):
+        alone = torch.empty((n,), dtype=torch.float64, device="cuda")
+        ctx.ckks_decode(plain[p].data_ptr(), L, 2.0 ** 20, alone.data_ptr(), w.data_ptr(), wb, stream())
+        torch.cuda.synchronize()
+        assert torch.equal(many[p], alone)
