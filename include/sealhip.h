@@ -174,7 +174,7 @@ int shc_keyswitch_shapes_import(const shc_context *ctx, const char *text);
  * A batch of ciphertexts at uneven levels, as groups of one level each (a work table
  * of up to 16 groups per launch; more are taken 16 at a time).  Each grouped call gives
  * every group the words of the one-level call on it, and runs each stage with one
- * launch for all groups: CKKS at N = 2^15 and 2^16 (the fused key switch); other
+ * launch for all groups: CKKS at N = 2^13 to 2^16 (the fused key switch); other
  * degrees and BFV key switches run group by group.  No counterpart in the reference
  * (one ciphertext per call, src/evaluator_cuda.cu:262-281). */
 typedef struct {

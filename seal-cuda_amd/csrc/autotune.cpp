@@ -52,7 +52,7 @@ std::vector<KsShape> keyswitch_candidates(const Context &c, uint32_t L) {
         const uint32_t tc = (L + chunks) / chunks;  // ceil((L + 1) / chunks)
         if (std::find(targets.begin(), targets.end(), tc) == targets.end()) targets.push_back(tc);
     }
-    const bool fused = c.logn == 15 || c.logn == 16;
+    const bool fused = c.logn >= 13 && c.logn <= 16;
     std::vector<KsShape> out{KsShape{}};  // the built-in choice first
     for (uint32_t g : fused ? std::vector<uint32_t>{4, 2, 1} : std::vector<uint32_t>{0})
         for (uint32_t tc : targets) out.push_back(KsShape{tc, g});

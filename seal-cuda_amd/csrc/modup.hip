@@ -14,7 +14,7 @@ __device__ __forceinline__ const void *uniform_ptr(const void *p) {
     return (const void *)((uint64_t)hi << 32 | lo);
 }
 
-// The key switch's ModUp rows pass fused with the products by the key (N = 2^15, 2^16):
+// The key switch's ModUp rows pass fused with the products by the key (N = 2^13 .. 2^16):
 // a block owns RW adjacent rows of target prime i for CG ciphertexts (NS = CG x RW
 // slots).  Each step transforms SUBS rows of T -- NS slots x SUBS/NS digits, the last K
 // layers with the wide schedule -- stages them in LDS, and then every thread multiplies
@@ -513,27 +513,40 @@ void launch_modup(const uint64_t *d, size_t d_stride, uint64_t *T, uint32_t cts,
     });
 }
 
-// The fused rows pass + key products over a batch: groups of 4 ciphertexts, then the
-// rest as a group of 2 and/or 1, so that no row is transformed for a ciphertext that is
-// not there.
+// A batch's groups of ciphertexts.  N = 2^15 up: groups of 4, then the rest as a group of 2
+// and/or 1, so that no row is transformed for a ciphertext that is not there.  Up to
+// N = 2^14 a launch of its own for the rest costs more than its idle slots: the last group
+// of 4 is a short one (products at N = 2^14, L = 7: 101 against 110 us for 3 ciphertexts, 546
+// against 551 for 37; in two kernels 101 and 575).
+struct GroupSplit {
+    uint32_t g4, g2, singles;
+};
+template <int LOGN>
+GroupSplit split_groups(uint32_t cts, uint32_t group) {
+    uint32_t g4 = group == 4 ? cts / 4 : 0;
+    uint32_t rest = cts - 4 * g4;
+    if (LOGN <= 14 && group == 4 && (g4 ? rest : rest == 3)) g4++, rest = 0;
+    const uint32_t g2 = group == 1 ? 0 : rest / 2;
+    return GroupSplit{g4, g2, rest - 2 * g2};
+}
+
+// The fused rows pass + key products over a batch's groups.
 template <int LOGN, bool R4, bool MIXED>
 void launch_keyprod_groups(const uint64_t *T, const uint64_t *key, uint64_t *P, uint64_t *S, const uint64_t *diag,
                            size_t diag_stride, uint32_t cts, uint32_t L, uint32_t K_key, const DevPrime *targets,
                            uint32_t tiles, uint64_t tile_slots, uint32_t group, const KsFold &fold, hipStream_t st) {
     constexpr int K2 = LOGN - LOGN / 2;
     constexpr int E = 4;
-    constexpr int RS = 4096 >> K2;
-    // groups of `group` ciphertexts (4 by default), then a group of 2, then a single one
+    constexpr int RS = 16;
+    // groups of `group` ciphertexts (4 by default), then what is left
     const uint32_t g = group == 1 || group == 2 ? group : 4;
-    const uint32_t g4 = g == 4 ? cts / 4 : 0;
-    const uint32_t g2 = g == 1 ? 0 : (cts - 4 * g4) / 2;
-    const uint32_t singles = cts - 4 * g4 - 2 * g2;
+    const auto [g4, g2, singles] = split_groups<LOGN>(cts, g);
     if (g4)
         ntt_rows_keyprod_kernel<LOGN, K2, E, RS, 4, 1, R4, MIXED><<<(uint32_t)(tile_slots * g4), RS << (K2 - E), 0, st>>>(
             T, key, P, S, targets, diag, diag_stride, cts, L, K_key, 0, g4, tiles, fold);
     if (g2)
         ntt_rows_keyprod_kernel<LOGN, K2, E, RS, 2, 1, R4, MIXED><<<(uint32_t)(tile_slots * g2), RS << (K2 - E), 0, st>>>(
-            T, key, P, S, targets, diag, diag_stride, cts, L, K_key, g4 * 4, g2, tiles, fold);
+            T, key, P, S, targets, diag, diag_stride, cts, L, K_key, cts - 2 * g2 - singles, g2, tiles, fold);
     if (singles) {
         // single ciphertexts: two rows per block
         const uint32_t tiles2 = tiles / 2;
@@ -559,12 +572,21 @@ void launch_modup_keyprod(const uint64_t *d, size_t d_stride, uint64_t *T, const
     constexpr int CS = 16;
     const uint32_t tc = modup_targets_per_block(cts * L * ((1u << K2) / CS), L, shape.cols_targets);
     const uint32_t col_grid = cts * L * ((L + tc) / tc) * ((1u << K2) / CS);
+    auto cols = [&](auto e, auto mx, auto one) {
+        constexpr int E = decltype(e)::value;
+        ntt_cols_modup_kernel<LOGN, K1, E, CS, decltype(one)::value, decltype(mx)::value>
+            <<<col_grid, CS << (K1 - E), 0, st>>>(d, d_stride, T, targets, digits, cts, L, diag != nullptr, tc);
+    };
     with_bool(mixed, [&](auto mx) {
         with_bool(tc == 1, [&](auto one) {
-            constexpr bool MIXED = decltype(mx)::value;
-            constexpr int E = modup_cols_log(MIXED);
-            ntt_cols_modup_kernel<LOGN, K1, E, CS, decltype(one)::value, MIXED><<<col_grid, CS << (K1 - E), 0, st>>>(
-                d, d_stride, T, targets, digits, cts, L, diag != nullptr, tc);
+            constexpr int E = modup_cols_log(decltype(mx)::value);
+            // (up to N = 2^14 a small launch takes 4 values, as the other small passes do)
+            if constexpr (LOGN <= 14)
+                with_shape<LOGN>((uint64_t)cts * L * (L + 1), [&](auto s) {
+                    cols(std::integral_constant<int, decltype(s)::value ? 2 : E>{}, mx, one);
+                });
+            else
+                cols(std::integral_constant<int, E>{}, mx, one);
         });
     });
     const uint32_t tiles = (L + 1) << K1;
@@ -591,7 +613,7 @@ void launch_modup_keyprod_groups(const KsGroup *gs, uint32_t n, const uint64_t *
     constexpr int K2 = LOGN - K1;
     constexpr int E = 4;
     constexpr int CS = 16;
-    constexpr int RS = 4096 >> K2;
+    constexpr int RS = 16;
     // columns pass: targets per block chosen for the whole launch's tile blocks
     uint64_t tile_blocks = 0;
     uint32_t maxL = 0;
@@ -629,7 +651,7 @@ void launch_modup_keyprod_groups(const KsGroup *gs, uint32_t n, const uint64_t *
         const KsGroup &a = gs[g];
         const uint32_t tiles = (a.L + 1) << K1;
         const uint64_t tile_slots = (uint64_t)((tiles + 7) / 8) * 8;
-        const uint32_t g4 = a.count / 4, g2 = (a.count - 4 * g4) / 2, singles = a.count - 4 * g4 - 2 * g2;
+        const auto [g4, g2, singles] = split_groups<LOGN>(a.count, 4);
         if (g4) {
             t4.g[s4.size()] =
                 KeyprodGroup{a.T, a.P, a.S, a.targets, a.diag, a.diag_stride, a.count, a.L, 0, g4, tiles, a.fold};
@@ -637,7 +659,8 @@ void launch_modup_keyprod_groups(const KsGroup *gs, uint32_t n, const uint64_t *
         }
         if (g2) {
             t2.g[s2.size()] =
-                KeyprodGroup{a.T, a.P, a.S, a.targets, a.diag, a.diag_stride, a.count, a.L, 4 * g4, g2, tiles, a.fold};
+                KeyprodGroup{a.T, a.P, a.S, a.targets, a.diag, a.diag_stride, a.count, a.L, a.count - 2 * g2 - singles,
+                                           g2, tiles, a.fold};
             s2.push_back(tile_slots * g2);
         }
         if (singles) {
@@ -701,26 +724,34 @@ bool ntt_modup_keyprod(const uint64_t *d, size_t d_ct_stride, uint64_t *T, const
                        uint64_t *S, const uint64_t *diag, size_t diag_stride, uint32_t count, uint32_t L,
                        uint32_t key_count, const DevPrime *targets, const DevPrime *digits, int logn, bool mixed,
                        hipStream_t st, const KernelProbe *probe, KsShape shape, KsFold fold) {
-    if ((logn != 15 && logn != 16) || count == 0) return false;
+    if (logn < 13 || logn > 16 || count == 0) return false;
     if ((uint64_t)count * L * (L + 1) > ((uint64_t(1) << 34) >> logn))
         fail(ERR_INVALID_ARGUMENT, "key-switch batch too large for one launch");
-    if (logn == 15)
-        launch_modup_keyprod<15>(d, d_ct_stride, T, key, P, S, diag, diag_stride, count, L, key_count, targets,
-                                 digits, mixed, probe, st, shape, fold);
-    else
-        launch_modup_keyprod<16>(d, d_ct_stride, T, key, P, S, diag, diag_stride, count, L, key_count, targets,
-                                 digits, mixed, probe, st, shape, fold);
+    auto go = [&](auto n) {
+        launch_modup_keyprod<decltype(n)::value>(d, d_ct_stride, T, key, P, S, diag, diag_stride, count, L, key_count,
+                                                 targets, digits, mixed, probe, st, shape, fold);
+    };
+    switch (logn) {
+        case 13: go(std::integral_constant<int, 13>{}); break;
+        case 14: go(std::integral_constant<int, 14>{}); break;
+        case 15: go(std::integral_constant<int, 15>{}); break;
+        default: go(std::integral_constant<int, 16>{}); break;
+    }
     launch_check("ntt modup keyprod launch");
     return true;
 }
 
 bool ntt_modup_keyprod_groups(const KsGroup *gs, uint32_t n, const uint64_t *key, uint32_t key_count,
                               const DevPrime *digits, int logn, bool mixed, hipStream_t st) {
-    if (logn != 15 && logn != 16) return false;
+    if (logn < 13 || logn > 16) return false;
     if (n > MAX_GROUPS) fail(ERR_INVALID_ARGUMENT, "too many groups for one launch");
     if (n == 0) return true;
-    if (logn == 15) launch_modup_keyprod_groups<15>(gs, n, key, key_count, digits, mixed, st);
-    else launch_modup_keyprod_groups<16>(gs, n, key, key_count, digits, mixed, st);
+    switch (logn) {
+        case 13: launch_modup_keyprod_groups<13>(gs, n, key, key_count, digits, mixed, st); break;
+        case 14: launch_modup_keyprod_groups<14>(gs, n, key, key_count, digits, mixed, st); break;
+        case 15: launch_modup_keyprod_groups<15>(gs, n, key, key_count, digits, mixed, st); break;
+        default: launch_modup_keyprod_groups<16>(gs, n, key, key_count, digits, mixed, st); break;
+    }
     launch_check("grouped modup keyprod launch");
     return true;
 }

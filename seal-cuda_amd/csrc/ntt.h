@@ -51,7 +51,7 @@ bool ntt_forward_modup(const uint64_t *d, size_t d_ct_stride, uint64_t *T, uint3
                        const DevPrime *targets, const DevPrime *digits, int logn, bool skip_diag, bool reduce_4q,
                        bool mixed, hipStream_t stream, const KernelProbe *probe = nullptr, KsShape shape = KsShape{});
 
-// The same ModUp with its rows pass fused into the products by the key (N = 2^15, 2^16;
+// The same ModUp with its rows pass fused into the products by the key (N = 2^13 .. 2^16;
 // returns false and does nothing otherwise): the columns pass fills T as above (diag !=
 // nullptr: skip_diag), then P[ct][k][i] = sum_j NTT_i(d_j mod t_i) key[j][k][ki] for
 // i < L and S[ct][k] for the special target (ki = key_count - 1), the own-prime terms
@@ -183,7 +183,7 @@ struct KsGroup {
     uint32_t count, L;
     KsFold fold;
 };
-// The fused ModUp + key products of every group (N = 2^15, 2^16; false otherwise): one
+// The fused ModUp + key products of every group (N = 2^13 .. 2^16; false otherwise): one
 // columns-pass launch and one rows-pass launch per ciphertext grouping (4, 2, 1).
 bool ntt_modup_keyprod_groups(const KsGroup *groups, uint32_t n, const uint64_t *key, uint32_t key_count,
                               const DevPrime *digits, int logn, bool mixed, hipStream_t stream);

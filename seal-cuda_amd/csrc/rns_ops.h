@@ -75,7 +75,7 @@ void rescale_to_next(const Context &c, const uint64_t *in, uint64_t *out, uint32
 
 // Level groups: each group is a batch at one level with its own buffers; a grouped call
 // gives every group the words of the one-level call, with one launch per stage for all
-// groups (CKKS, N = 2^15 and 2^16 for the key switch; other shapes run group by group).
+// groups (CKKS, N = 2^13 .. 2^16 for the key switch; other shapes run group by group).
 struct TensorGroup {
     const uint64_t *a, *b;  // [count][2][L][N]
     uint64_t *out;          // [count][3][L][N]

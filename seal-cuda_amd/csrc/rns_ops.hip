@@ -14,7 +14,7 @@
 //      are c2's NTT-form limbs themselves (the reference's i == j shortcut)
 //   4. inner_product: P_k[i] = sum_j T[j][i] * key[j][k][i] with 128-bit accumulation,
 //      one Barrett reduction at the end; G ciphertexts per thread share each key load.
-//      At N = 2^15 and 2^16 the NTT's rows pass and this product are one kernel
+//      At N = 2^13 .. 2^16 the NTT's rows pass and this product are one kernel
 //      (ntt_modup_keyprod): the transformed limbs never return to HBM
 //   5. ModDown: inverse NTT of the special limbs, rounding correction, forward NTT
 //      (CKKS) or inverse NTT of P (BFV), then ct_k[i] += (P_k[i] - t) * p^-1.
@@ -455,12 +455,14 @@ void switch_key_chunk(const Context &c, const uint64_t *target, size_t target_st
         dstride = (size_t)L * n;
     }
     // 2-4. ModUp and the inner product with the key: fused past the columns pass where
-    // the transform shape allows (N = 2^15, 2^16), else T goes through HBM once more
+    // the transform shape allows (N = 2^13 .. 2^16), else T goes through HBM once more
     // (CKKS: the fused products also take p times the ciphertext the switch adds into, so
     // that the ModDown writes it without reading it)
     const KsShape shape = c.ks_shape(L, count);
     const KsFold fold = ckks ? KsFold{fold_c0 ? fold_c0 : ct, ct_stride, c.ks_consts(), fold_c0 != nullptr} : KsFold{};
-    const bool fused = ntt_modup_keyprod(digits, dstride, T, key, P, S, diag, target_stride, count, L,
+    // (a single ciphertext at N = 2^13 leaves the fused kernel 16 blocks per prime to wait
+    // in: 54.7 us per product at L = 3 in two kernels, 55.8 in one)
+    const bool fused = (logn > 13 || count > 1 || fold_c0) && ntt_modup_keyprod(digits, dstride, T, key, P, S, diag, target_stride, count, L,
                                          (uint32_t)c.key_count(), c.keyswitch_primes(L), c.primes(), logn,
                                          c.fp_primes, st, probe, shape, fold);
     if (fold_c0 && !fused) fail(ERR_LOGIC, "a key switch into (c0, 0) needs the fused key products");
@@ -540,7 +542,7 @@ void moddown_into(const Context &c, uint64_t *P, uint64_t *S, uint64_t *U, uint6
     launch_check("moddown_finish");
 }
 
-bool keyswitch_folds(const Context &c) { return c.scheme == SCHEME_CKKS && (c.logn == 15 || c.logn == 16); }
+bool keyswitch_folds(const Context &c) { return c.scheme == SCHEME_CKKS && c.logn >= 13 && c.logn <= 16; }
 
 void switch_key(const Context &c, const uint64_t *target, size_t target_stride, uint64_t *ct, size_t ct_stride,
                 const uint64_t *key, uint32_t count, uint32_t L, void *ws, size_t ws_bytes, hipStream_t st,
@@ -671,7 +673,7 @@ void relinearize_groups(const Context &c, const RelinGroup *gs, uint32_t n, cons
     const int logn = c.logn;
     const size_t nn = c.n;
     // one launch per stage needs the fused CKKS path and every group within one launch
-    bool grouped = c.scheme == SCHEME_CKKS && (logn == 15 || logn == 16);
+    bool grouped = c.scheme == SCHEME_CKKS && logn >= 13 && logn <= 16;
     for (uint32_t g = 0; g < n && grouped; g++)
         grouped = (uint64_t)gs[g].count * gs[g].L * (gs[g].L + 1) <= ((uint64_t(1) << 34) >> logn);
     char *base = static_cast<char *>(ws);

@@ -114,6 +114,28 @@ def test_relinearize_fp64_primes(scheme, logn, bits, L, count, words):
         np.testing.assert_array_equal(got[c], ck.relinearize(scheme, ct3[c], key, moduli, L, logn))
 
 
+@pytest.mark.parametrize("scheme,logn,bits,L,counts", [
+    (CKKS, 13, [60, 40, 60, 50], 3, (1, 2, 3, 4, 5)),
+    (CKKS, 14, [60] * 10, 9, (1, 3, 6)),
+    (CKKS, 14, [50] * 3, 1, (2, 7)),
+    (BFV, 13, [45, 43, 44, 60], 3, (1, 2, 5)),
+    (BFV, 14, [60] * 4, 3, (3,)),
+    # 32 digits: words below 4q before the products
+    (CKKS, 13, [60] * 33, 32, (5,)),
+])
+def test_relinearize_small_rings_fused(scheme, logn, bits, L, counts):
+    """N = 2^13 and 2^14 fuse the rows pass and the key products, in groups of 4 of which the
+    last may be short (one ciphertext at N = 2^13 does not)."""
+    ctx, moduli = make_ctx(scheme, logn, bits)
+    rng = np.random.default_rng(logn * 31 + L)
+    key = ck.random_key(rng, moduli, logn)
+    for count in counts:
+        ct3 = ck.uniform_residues(rng, (count, 3, L, 1 << logn), moduli[:L])
+        got = run_relin(ctx, ct3, key, L)
+        for c in {0, count // 2, count - 1}:
+            np.testing.assert_array_equal(got[c], ck.relinearize(scheme, ct3[c], key, moduli, L, logn))
+
+
 def test_relinearize_columns_all_targets():
     """A batch large enough that each ModUp columns block transforms its digit tile for
     all L + 1 targets (104 x 20 x 8 tiles >= 16384 blocks); three ciphertexts against the

@@ -78,6 +78,12 @@ def test_relinearize_groups_equal_one_level_calls(scheme, logn, bits, spec):
                                   ck.relinearize(scheme, ct3[c - 1], key_h, moduli, L, int(np.log2(n))))
 
 
+@pytest.mark.parametrize("logn,spec", [(13, [(4, 1), (2, 3), (1, 2), (3, 9)]), (14, [(3, 5), (4, 1), (1, 1)])])
+def test_relinearize_groups_small_rings(logn, spec):
+    """One launch per stage at N = 2^13 and 2^14 too, with short last groups of 4."""
+    test_relinearize_groups_equal_one_level_calls(CKKS, logn, [60, 40, 60, 40, 60], spec)
+
+
 @pytest.mark.parametrize("logn,bits,spec", [
     (15, [60] + [40] * 14 + [60], [(15, 2), (9, 5), (4, 3), (7, 1), (12, 7), (2, 2)]),
     (16, [60] * 6, [(5, 3), (3, 2), (4, 1)]),
