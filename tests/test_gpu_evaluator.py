@@ -126,7 +126,7 @@ def test_relinearize_fp64_primes(scheme, logn, bits, L, count, words):
 def test_relinearize_small_rings_fused(scheme, logn, bits, L, counts):
     """N = 2^13 and 2^14 fuse the rows pass and the key products, in groups of 4 of which the
     last may be short (one ciphertext at N = 2^13 does not)."""
-    ctx, moduli = make_ctx(scheme, logn, bits)
+    ctx, moduli = make_ctx(scheme, logn, bits, 65537 if scheme == BFV else 0)
     rng = np.random.default_rng(logn * 31 + L)
     key = ck.random_key(rng, moduli, logn)
     for count in counts:
