@@ -139,16 +139,21 @@ static bool check_fp(u64 q, long &cases) {
         const double x = (k & 1 ? -1 : 1) * (double)(next() % (17 * (q / 10) + 1));
         if (shc::fp_to_u52(x, up) != (u64)((int64_t)x + (int64_t)(2 * q))) return std::printf("fp_to_u52\n"), false;
     }
-    for (int ext = 0; ext < 2; ext++) {
+    const wide r = ~(wide)0 / q;  // floor(2^128 / q), q not a power of 2
+    for (int ext = 0; ext < 64; ext++) {
         shc::Acc26 a{0, 0, 0};
         wide sum = 0;
-        for (int k = 0; k < 64; k++) {
-            const u64 t = ext ? 4 * q - 1 : next() % (4 * q), f = ext ? q - 1 : next() % q;
+        for (int k = 0; k < (ext == 1 ? 512 : 64); k++) {
+            if (ext > 1 && shc::acc_reduce26(a, q, (u64)r, (u64)(r >> 64)) != (u64)(sum % q))
+                return std::printf("acc_reduce26 q=%llu\n", (unsigned long long)q), false;
+            const u64 t = ext == 1 ? 4 * q - 1 : next() % (4 * q), f = ext == 1 ? q - 1 : next() % q;
             shc::mac(a, shc::cut26(t), shc::cut26(f));
             sum += (wide)t * f;
         }
         const shc::u128 v = shc::acc_value(a);
         if ((((wide)v.hi << 64) | v.lo) != sum) return std::printf("Acc26 q=%llu\n", (unsigned long long)q), false;
+        if (shc::acc_reduce26(a, q, (u64)r, (u64)(r >> 64)) != (u64)(sum % q))
+            return std::printf("acc_reduce26 q=%llu\n", (unsigned long long)q), false;
         cases += 64;
     }
     return true;
@@ -170,6 +175,16 @@ int main() {
     for (u64 q : primes) {
         if (q < shc::FP_PRIME_LIMIT && !check_fp(q, cases)) return 1;
         const u64 neg_q = 0 - q, four_q = q << 2;
+        const wide r = ~(wide)0 / q;
+        for (int k = 0; k < 4096; k++) {
+            // words at 0, 1, multiples of q and the top, and any
+            auto word = [&](int c) { return c == 0 ? 0 : c == 1 ? ~u64(0) : c == 2 ? q - 1 : c == 3 ? (~u64(0) / q) * q - 1 : next(); };
+            const wide x = k < 2048 ? (wide)word(k % 5) << 64 | word(k / 5 % 5) : (wide)(next() % q) * (next() % q) + k % 3;
+            if (shc::barrett128(shc::u128{(u64)x, (u64)(x >> 64)}, q, (u64)r, (u64)(r >> 64)) != (u64)(x % q)) {
+                printf("barrett128 q=%llu case %d\n", (unsigned long long)q, k);
+                return 1;
+            }
+        }
         for (int wi = 0; wi < 24; wi++) {
             const u64 w = wi == 0 ? 0 : wi == 1 ? 1 : wi == 2 ? q - 1 : next() % q;
             const u64 wq = (u64)(((wide)w << 64) / q);
