@@ -779,7 +779,8 @@ void encrypt_chunk(const Context &c, const uint64_t *pk, const uint64_t *plain, 
         sample_encrypt_kernel<false><<<blocks_for(total), TPB, 0, st>>>(key, seed, logn, total, Us, Es);
     }
     launch_check("sample_encrypt");
-    if (!ntt_forward_small(Us, U, L1, m, primes, logn, st)) {
+    const bool u_cols = ckks && ntt_encrypt_takes_columns(m, L, L1, logn);
+    if (!ntt_forward_small(Us, U, L1, m, u_cols ? L : 0, primes, logn, st)) {
         const size_t uw = (size_t)m * L1 * n;
         lift_small_kernel<<<blocks_for(uw), TPB, 0, st>>>(Us, U, primes, L1, logn, uw);
         launch_check("lift_small");
@@ -793,7 +794,7 @@ void encrypt_chunk(const Context &c, const uint64_t *pk, const uint64_t *plain, 
             launch_check("enc_products");
             ntt_inverse(P, m * 2, 1, primes + L, logn, NTT_FULL, st);
         }
-        const EncArgs ea{Es, drop ? P : nullptr, pk, U, plain, out, dc, p, K, L1, L, drop};
+        const EncArgs ea{Es, drop ? P : nullptr, pk, U, plain, out, dc, p, K, L1, L, drop, u_cols};
         if (ntt_encrypt_ckks(ea, m, primes, logn, st)) return;
         enc_error_kernel<<<blocks_for(out_words), TPB, 0, st>>>(Es, drop ? P : nullptr, out, primes, dc, p, L, logn,
                                                                 out_words);

@@ -84,16 +84,19 @@ __global__ __launch_bounds__(SUBS << (K - E)) void ntt_cols_small_kernel(const i
 }
 
 template <int LOGN, bool SMALL>
-void launch_small_as(const int8_t *Us, uint64_t *U, uint32_t L1, uint32_t m, const DevPrime *primes, hipStream_t st) {
+void launch_small_as(const int8_t *Us, uint64_t *U, uint32_t L1, uint32_t m, uint32_t rows_from,
+                     const DevPrime *primes, hipStream_t st) {
     using S = PassShape<LOGN, SMALL>;
     constexpr int K1 = S::K1, K2 = S::K2, E = S::E, CS = S::CS, RS = S::RS;
     const bool mx = rows_mixed<LOGN, K2, RS>(m);
-    const uint32_t row_blocks = L1 * rows_blocks_per_prime<LOGN, K2, E, RS>(m, mx);
+    const uint32_t rows = L1 - rows_from;  // primes whose rows pass runs
+    const uint32_t row_blocks = rows * rows_blocks_per_prime<LOGN, K2, E, RS>(m, mx);
     ntt_cols_small_kernel<LOGN, K1, E, CS><<<L1 * m * ((1u << K2) / CS), CS << (K1 - E), 0, st>>>(Us, U, primes, L1, m);
-    const LimbGrid lg{1, L1, L1, m};
+    if (!rows) return;
+    const LimbGrid lg{1, L1, rows, m};
     with_bool(mx, [&](auto x) {
-        ntt_rows_kernel<LOGN, K2, E, RS, false, true, true, decltype(x)::value>
-            <<<row_blocks, RS << (K2 - E), 0, st>>>(U, primes, lg, 0, m);
+        ntt_rows_kernel<LOGN, K2, E, RS, false, true, true, decltype(x)::value><<<row_blocks, RS << (K2 - E), 0, st>>>(
+            U + ((size_t)rows_from << LOGN), primes + rows_from, lg, 0, m);
     });
 }
 
@@ -133,6 +136,71 @@ __global__ __launch_bounds__(SUBS << (K - E)) void ntt_rows_encrypt_kernel(const
         });
 }
 
+// The rows pass for batches: a block owns row g of prime i for SUBS ciphertexts and runs the
+// rows of their u, e0 and e1 one after another, so that NTT(u) stays in registers (16 words per
+// thread) instead of in memory, and the public key's words -- a thread's position is the same
+// in every ciphertext -- get Shoup constants once per block: their quotients come from
+// floor(2^128 / q), at most 1 short, which leaves the products in [0, 5q) (q < 2^60; with the
+// transform's [0, 8q) they fit a word).  128 ciphertexts at N = 2^16, L = 24: u's rows pass
+// 0.78 + e's 3.87 ms -> 3.46 in all, still VALU issue (24 layers and 3 products per word).
+template <int LOGN, int K, int E, int SUBS>
+__global__ __launch_bounds__(SUBS << (K - E), 4) void ntt_rows_encrypt_batch_kernel(const DevPrime *__restrict__ primes,
+                                                                                EncArgs a, uint32_t m) {
+    constexpr int T = 1 << (K - E), RPL = LOGN - K;
+    static_assert(SUBS * T == 1 << K, "one position of the row per thread");
+    __shared__ uint64_t tile[SUBS * row_words(K)];
+    const int tid = threadIdx.x, sub = tid / T, t = tid % T;
+    const uint32_t chunks = (m + SUBS - 1) / SUBS;
+    const uint32_t g0 = blockIdx.x % chunks * SUBS, r = blockIdx.x / chunks;
+    const int row = (int)(r & ((1u << RPL) - 1));
+    const uint32_t i = r >> RPL;
+    const int nsub = (int)min<uint32_t>(SUBS, m - g0);
+    const bool active = sub < nsub;
+    const uint32_t mine = g0 + (uint32_t)(active ? sub : 0);
+    const size_t row_off = (size_t)row << K;
+    const DevPrime &Q = primes[i];
+    const BfConst bc = bf_const(Q);
+    const ulonglong2 *table = Q.fwd;
+    auto addr = [sub](int idx) { return sub * row_words(K) + row_slot(idx); };
+    auto transform = [&](const uint64_t *in) {
+        asm volatile("" : "+s"(table));  // twiddles are loaded again rather than kept
+        const GlobalTw<LOGN, false, ulonglong2> tw{table, row, RPL};
+        auto load = [in](int idx, int) { return in[idx]; };
+        auto stage = [&](int idx, uint64_t x) { tile[addr(idx)] = x; };
+        run_phases<K, E, false, true>(tile, addr, load, stage, t, tw, bc, active);
+        __syncthreads();
+    };
+    transform(a.U + (((size_t)mine * a.L1 + i) << LOGN) + row_off);
+    // word v of the thread: position tid of the block's ciphertext v
+    uint64_t u[SUBS];
+#pragma unroll
+    for (int v = 0; v < SUBS; v++) u[v] = tile[v * row_words(K) + row_slot(tid)];
+    const size_t limb = ((size_t)i << LOGN) + row_off, ct_words = (size_t)a.L << LOGN;
+#pragma unroll 1
+    for (uint32_t k = 0; k < 2; k++) {
+        __syncthreads();  // the tile has been read
+        transform(a.out + (2 * mine + k) * ct_words + limb);
+        const uint64_t pk = a.pk[((size_t)(k * a.K + i) << LOGN) + row_off + tid];
+        const uint64_t pkq = pk * Q.ratio_hi + mulhi64(pk, Q.ratio_lo);
+        const bool add = a.plain && k == 0;
+#pragma unroll
+        for (int v = 0; v < SUBS; v++) {
+            if (v >= nsub) break;  // uniform
+            uint64_t x = shoup_lazier(u[v], pk, pkq, bc.neg_q) + tile[v * row_words(K) + row_slot(tid)];
+            if (a.drop) x = shoup(x, a.dc[i].inv, a.dc[i].inv_shoup, Q.q);
+            else x = barrett64(x, Q.q, Q.ratio_hi);
+            // (uniform slices: the thread's part of the addresses is tid alone)
+            if (add) x = addmod(x, (a.plain + (g0 + v) * ct_words + limb)[tid], Q.q);
+            (a.out + (2 * (g0 + v) + k) * ct_words + limb)[tid] = x;
+        }
+    }
+}
+
+// The ciphertexts of such a block, and the fewest it is taken for (N = 2^15, 2^16: rows of 256;
+// the 32 rows of 128 and the 8 of 512 that a block of 256 threads has need more than one
+// position per thread, and registers that spill).
+constexpr uint32_t ENC_BATCH = 16;
+
 template <int LOGN, bool SMALL>
 void launch_encrypt_as(const EncArgs &a, uint32_t jn, const DevPrime *primes, hipStream_t st) {
     using S = PassShape<LOGN, SMALL>;
@@ -141,6 +209,14 @@ void launch_encrypt_as(const EncArgs &a, uint32_t jn, const DevPrime *primes, hi
     const bool mx = rows_mixed<LOGN, K2, RS>(jn);
     const uint32_t row_blocks = a.L * rows_blocks_per_prime<LOGN, K2, E, RS>(jn, mx);
     ntt_cols_encrypt_kernel<LOGN, K1, E, CS><<<col_blocks, CS << (K1 - E), 0, st>>>(primes, a, jn);
+    if constexpr (!SMALL && RS == ENC_BATCH) {
+        if (a.u_cols) {
+            const uint32_t m = jn / 2;
+            ntt_rows_encrypt_batch_kernel<LOGN, K2, E, RS>
+                <<<(a.L << K1) * ((m + RS - 1) / RS), RS << (K2 - E), 0, st>>>(primes, a, m);
+            return;
+        }
+    }
     if (mx)
         ntt_rows_encrypt_kernel<LOGN, K2, E, RS, true><<<row_blocks, RS << (K2 - E), 0, st>>>(primes, a, jn);
     else
@@ -375,13 +451,13 @@ void ntt_inverse_galois(const uint64_t *src, LimbGrid slg, const GaloisPerm &per
     launch_check("permuted inverse ntt launch");
 }
 
-bool ntt_forward_small(const int8_t *Us, uint64_t *U, uint32_t L1, uint32_t m, const DevPrime *primes, int logn,
-                       hipStream_t st) {
+bool ntt_forward_small(const int8_t *Us, uint64_t *U, uint32_t L1, uint32_t m, uint32_t rows_from,
+                       const DevPrime *primes, int logn, hipStream_t st) {
     if (logn < 13 || logn > 17 || m == 0 || (uint64_t)L1 * m > ((uint64_t(1) << 34) >> logn)) return false;
     auto go = [&](auto n) {
         constexpr int LOGN = decltype(n)::value;
         with_shape<LOGN>((uint64_t)L1 * m, [&](auto s) {
-            launch_small_as<LOGN, decltype(s)::value>(Us, U, L1, m, primes, st);
+            launch_small_as<LOGN, decltype(s)::value>(Us, U, L1, m, rows_from, primes, st);
         });
     };
     switch (logn) {
@@ -393,6 +469,12 @@ bool ntt_forward_small(const int8_t *Us, uint64_t *U, uint32_t L1, uint32_t m, c
     }
     launch_check("small ntt launch");
     return true;
+}
+
+bool ntt_encrypt_takes_columns(uint32_t m, uint32_t L, uint32_t L1, int logn) {
+    const uint64_t most = (uint64_t(1) << 34) >> logn;
+    return (logn == 15 || logn == 16) && m >= ENC_BATCH && (uint64_t)2 * m * L <= most &&
+           (uint64_t)m * L1 <= most && ((uint64_t)2 * m * L << logn) > SMALL_WORDS;
 }
 
 bool ntt_encrypt_ckks(const EncArgs &a, uint32_t m, const DevPrime *primes, int logn, hipStream_t st) {

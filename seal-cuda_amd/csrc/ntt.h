@@ -144,11 +144,16 @@ struct EncArgs {
     uint64_t p;
     uint32_t K, L1, L;
     bool drop;
+    bool u_cols;  // U's limbs i < L hold the columns pass's words
 };
 // U[g][i] = forward transform (fully reduced) of the signed bytes Us[g] modulo primes[i],
-// g < m, i < L1 (N >= 2^13; returns false and does nothing otherwise).
-bool ntt_forward_small(const int8_t *Us, uint64_t *U, uint32_t L1, uint32_t m, const DevPrime *primes, int logn,
-                       hipStream_t stream);
+// g < m, i < L1 (N >= 2^13; returns false and does nothing otherwise).  Limbs below rows_from
+// keep the columns pass's words.
+bool ntt_forward_small(const int8_t *Us, uint64_t *U, uint32_t L1, uint32_t m, uint32_t rows_from,
+                       const DevPrime *primes, int logn, hipStream_t stream);
+// Whether ntt_encrypt_ckks takes U with u_cols (and does, if told so): large launches over
+// 16 ciphertexts or more, N = 2^15 and 2^16.
+bool ntt_encrypt_takes_columns(uint32_t m, uint32_t L, uint32_t L1, int logn);
 bool ntt_encrypt_ckks(const EncArgs &args, uint32_t m, const DevPrime *primes, int logn, hipStream_t stream);
 
 // ---- grouped launches (ciphertexts at several levels, one launch per stage) ----------

@@ -409,6 +409,34 @@ def test_encrypt_many_words_match_oracle(scheme, keyed, logn):
                 np.testing.assert_array_equal(from_dev(one), want[g])
 
 
+@pytest.mark.parametrize("logn,K,L,count", [(15, 21, 20, 52), (15, 33, 33, 32), (16, 9, 8, 65)])
+def test_encrypt_many_batches_take_rows_together(logn, K, L, count):
+    """Large batches run the rows of u, e0 and e1 in one kernel, 16 ciphertexts per block (the
+    last one partial, or full; a prime dropped, or none): the words of single encryptions, the first
+    of which is the oracle's."""
+    n = 1 << logn
+    assert count >= 16 and 2 * count * L * n > 1 << 26
+    moduli = ck.coeff_modulus_create(n, [60, 50, 40][:K] + [60] * (K - 3))
+    ctx = hip().Context(CKKS, n, moduli)
+    sk, pk = empty_dev((K, n)), empty_dev((2, K, n))
+    ctx.keygen_secret(1, sk.data_ptr(), stream())
+    ctx.keygen_public(sk.data_ptr(), 2, pk.data_ptr(), stream())
+    plain = ck.uniform_residues(np.random.default_rng(logn), (count, L, n), moduli[:L])
+    dplain = to_dev(plain)
+    out, one = empty_dev((count, 2, L, n)), empty_dev((2, L, n))
+    w, ew = ctx.encrypt_many_workspace_size(L, count), ctx.encrypt_workspace_size(L)
+    wb, eb = ws(w), ws(ew)
+    for with_plain in (False, True):
+        ctx.encrypt_many(pk.data_ptr(), dplain.data_ptr() if with_plain else 0, count, L, 77, out.data_ptr(),
+                         wb.data_ptr(), w, stream())
+        for g in (0, 15, 16, count - 1):
+            ctx.encrypt(pk.data_ptr(), dplain[g].data_ptr() if with_plain else 0, L, 77 + g, one.data_ptr(),
+                        eb.data_ptr(), ew, stream())
+            np.testing.assert_array_equal(from_dev(out[g]), from_dev(one))
+    want = expected_encryption(CKKS, None, from_dev(pk), 77, L, moduli, logn, plain[0])
+    np.testing.assert_array_equal(from_dev(out[0]), want)
+
+
 def test_encrypt_many_rejects_and_empty():
     logn = 10
     n = 1 << logn
