@@ -42,17 +42,35 @@ __device__ __forceinline__ void moddown_add(const ModDownArgs &a, uint32_t i, ui
     else *dst = addmod(*dst, v, Q.q);
 }
 
+// Columns pass of u_i = the rounded special limb's residue, on load.  One branch per block
+// between a ModDown's own limb and a sum of them (15 floor(p/2) mod q_i < 2^64): inside the load
+// it kept a thread's 16 loads from going out together (1,452 -> 1,695 us for 256 limbs of 2^16 to
+// 23 primes).  Every prime reads the same special limb: i fastest keeps it in L2.
+template <int LOGN, int K, int E, int SUBS>
+__device__ __forceinline__ void cols_moddown_prep(uint64_t *tile, uint32_t bid, uint64_t *__restrict__ U,
+                                                  const DevPrime *__restrict__ primes, const ModDownArgs &a,
+                                                  uint32_t jn) {
+    auto run = [&](const auto &of) {
+        cols_body_t<LOGN, K, E, SUBS, false, true>(
+            tile, bid, primes, 0, jn,
+            [&](uint32_t i, uint32_t j, size_t off) { return of(i, a.S[((size_t)j << LOGN) + off]); },
+            [&](uint32_t i, uint32_t j, size_t off, uint64_t x) { U[((size_t)(j * a.L + i) << LOGN) + off] = x; }, a.L);
+    };
+    if (a.presum)
+        run([&](uint32_t i, uint64_t s) {
+            const DevPrime &Q = primes[i];
+            return submod(barrett64(s, Q.q, Q.ratio_hi), barrett64(a.presum * a.dc[i].half_mod, Q.q, Q.ratio_hi), Q.q);
+        });
+    else
+        run([&](uint32_t i, uint64_t s) { return moddown_prep(s, a.p, primes[i], a.dc[i]); });
+}
+
 template <int LOGN, int K, int E, int SUBS>
 __global__ __launch_bounds__(SUBS << (K - E)) void ntt_cols_moddown_prep_kernel(uint64_t *__restrict__ U,
                                                                                const DevPrime *__restrict__ primes,
                                                                                ModDownArgs a, uint32_t jn) {
-    // every prime reads the same special limb: i fastest keeps it in L2
-    cols_body<LOGN, K, E, SUBS, false, true>(
-        blockIdx.x, primes, 0, jn,
-        [&](uint32_t i, uint32_t j, size_t off) {
-            return moddown_u(a, i, a.S[((size_t)j << LOGN) + off], primes[i]);
-        },
-        [&](uint32_t i, uint32_t j, size_t off, uint64_t x) { U[((size_t)(j * a.L + i) << LOGN) + off] = x; }, a.L);
+    __shared__ uint64_t tile[SUBS << K];
+    cols_moddown_prep<LOGN, K, E, SUBS>(tile, blockIdx.x, U, primes, a, jn);
 }
 
 template <int LOGN, int K, int E, int SUBS, bool MX>
@@ -247,13 +265,8 @@ __global__ __launch_bounds__(SUBS << (K - E)) void ntt_cols_moddown_prep_grouped
     const uint32_t gi = group_of(mg.start, mg.n, blockIdx.x);
     const ModDownGroupDev &gr = mg.g[gi];
     const ModDownArgs &a = gr.a;
-    uint64_t *U = gr.U;
-    cols_body<LOGN, K, E, SUBS, false, true>(
-        blockIdx.x - mg.start[gi], primes, 0, gr.jn,
-        [&](uint32_t i, uint32_t j, size_t off) {
-            return moddown_u(a, i, a.S[((size_t)j << LOGN) + off], primes[i]);
-        },
-        [&](uint32_t i, uint32_t j, size_t off, uint64_t x) { U[((size_t)(j * a.L + i) << LOGN) + off] = x; }, a.L);
+    __shared__ uint64_t tile[SUBS << K];
+    cols_moddown_prep<LOGN, K, E, SUBS>(tile, blockIdx.x - mg.start[gi], gr.U, primes, a, gr.jn);
 }
 
 template <int LOGN, int K, int E, int SUBS, bool MX>
