@@ -1,6 +1,7 @@
 // modup.hip -- the key switch's ModUp transforms, alone and fused with the products by the
 // key (N = 2^13 .. 2^17; the passes are those of ntt_device.h, the schedules ntt.hip's).
 #include "accum.h"
+#include "launch_limits.h"
 #include "ntt_device.h"
 
 namespace shc {
@@ -513,23 +514,6 @@ void launch_modup(const uint64_t *d, size_t d_stride, uint64_t *T, uint32_t cts,
     });
 }
 
-// A batch's groups of ciphertexts.  N = 2^15 up: groups of 4, then the rest as a group of 2
-// and/or 1, so that no row is transformed for a ciphertext that is not there.  Up to
-// N = 2^14 a launch of its own for the rest costs more than its idle slots: the last group
-// of 4 is a short one (products at N = 2^14, L = 7: 101 against 110 us for 3 ciphertexts, 546
-// against 551 for 37; in two kernels 101 and 575).
-struct GroupSplit {
-    uint32_t g4, g2, singles;
-};
-template <int LOGN>
-GroupSplit split_groups(uint32_t cts, uint32_t group) {
-    uint32_t g4 = group == 4 ? cts / 4 : 0;
-    uint32_t rest = cts - 4 * g4;
-    if (LOGN <= 14 && group == 4 && (g4 ? rest : rest == 3)) g4++, rest = 0;
-    const uint32_t g2 = group == 1 ? 0 : rest / 2;
-    return GroupSplit{g4, g2, rest - 2 * g2};
-}
-
 // The fused rows pass + key products over a batch's groups.
 template <int LOGN, bool R4, bool MIXED>
 void launch_keyprod_groups(const uint64_t *T, const uint64_t *key, uint64_t *P, uint64_t *S, const uint64_t *diag,
@@ -540,7 +524,7 @@ void launch_keyprod_groups(const uint64_t *T, const uint64_t *key, uint64_t *P, 
     constexpr int RS = 16;
     // groups of `group` ciphertexts (4 by default), then what is left
     const uint32_t g = group == 1 || group == 2 ? group : 4;
-    const auto [g4, g2, singles] = split_groups<LOGN>(cts, g);
+    const auto [g4, g2, singles] = split_groups(LOGN, cts, g);
     if (g4)
         ntt_rows_keyprod_kernel<LOGN, K2, E, RS, 4, 1, R4, MIXED><<<(uint32_t)(tile_slots * g4), RS << (K2 - E), 0, st>>>(
             T, key, P, S, targets, diag, diag_stride, cts, L, K_key, 0, g4, tiles, fold);
@@ -550,7 +534,7 @@ void launch_keyprod_groups(const uint64_t *T, const uint64_t *key, uint64_t *P, 
     if (singles) {
         // single ciphertexts: two rows per block
         const uint32_t tiles2 = tiles / 2;
-        const uint32_t slots2 = (tiles2 + 7) / 8 * 8;
+        const uint32_t slots2 = (uint32_t)keyprod_slots(LOGN, L, true);
         ntt_rows_keyprod_kernel<LOGN, K2, E, RS, 1, 2, R4, MIXED><<<slots2 * singles, RS << (K2 - E), 0, st>>>(
             T, key, P, S, targets, diag, diag_stride, cts, L, K_key, cts - singles, singles, tiles2, fold);
     }
@@ -590,7 +574,7 @@ void launch_modup_keyprod(const uint64_t *d, size_t d_stride, uint64_t *T, const
         });
     });
     const uint32_t tiles = (L + 1) << K1;
-    const uint64_t tile_slots = (uint64_t)((tiles + 7) / 8) * 8;
+    const uint64_t tile_slots = keyprod_slots(LOGN, L, false);
     if (tile_slots * cts >= (uint64_t(1) << 32))
         fail(ERR_INVALID_ARGUMENT, "key-switch batch too large for one launch");
     if (probe) SHC_HIP(hipEventRecord(probe->begin, st));
@@ -650,8 +634,8 @@ void launch_modup_keyprod_groups(const KsGroup *gs, uint32_t n, const uint64_t *
     for (uint32_t g = 0; g < n; g++) {
         const KsGroup &a = gs[g];
         const uint32_t tiles = (a.L + 1) << K1;
-        const uint64_t tile_slots = (uint64_t)((tiles + 7) / 8) * 8;
-        const auto [g4, g2, singles] = split_groups<LOGN>(a.count, 4);
+        const uint64_t tile_slots = keyprod_slots(LOGN, a.L, false);
+        const auto [g4, g2, singles] = split_groups(LOGN, a.count, 4);
         if (g4) {
             t4.g[s4.size()] =
                 KeyprodGroup{a.T, a.P, a.S, a.targets, a.diag, a.diag_stride, a.count, a.L, 0, g4, tiles, a.fold};
@@ -665,7 +649,7 @@ void launch_modup_keyprod_groups(const KsGroup *gs, uint32_t n, const uint64_t *
         }
         if (singles) {
             const uint32_t tiles2 = tiles / 2;
-            const uint64_t slots2 = (tiles2 + 7) / 8 * 8;
+            const uint64_t slots2 = keyprod_slots(LOGN, a.L, true);
             t1.g[s1.size()] = KeyprodGroup{a.T, a.P, a.S, a.targets, a.diag, a.diag_stride, a.count, a.L,
                                            a.count - singles, singles, tiles2, a.fold};
             s1.push_back(slots2 * singles);

@@ -4,6 +4,7 @@
 #include "ntt.h"
 #include "butterfly.h"
 #include "butterfly_fp.h"
+#include "launch_limits.h"
 #include "modarith.h"
 #include <type_traits>
 #include <vector>
@@ -423,7 +424,7 @@ uint32_t fill_starts(Table &t, const std::vector<uint64_t> &sizes) {
         acc += sizes[g];
     }
     t.start[sizes.size()] = (uint32_t)acc;
-    if (acc >= (uint64_t(1) << 32) / 1024) fail(ERR_INVALID_ARGUMENT, "grouped launch too large");
+    if (acc >= GROUPED_BLOCKS) fail(ERR_INVALID_ARGUMENT, "grouped launch too large");
     return (uint32_t)acc;
 }
 

@@ -19,6 +19,7 @@
 //   5. ModDown: inverse NTT of the special limbs, rounding correction, forward NTT
 //      (CKKS) or inverse NTT of P (BFV), then ct_k[i] += (P_k[i] - t) * p^-1.
 #include "accum.h"
+#include "launch_limits.h"
 #include "modarith.h"
 #include "ntt.h"
 #include "rns_ops.h"
@@ -672,10 +673,19 @@ void relinearize_groups(const Context &c, const RelinGroup *gs, uint32_t n, cons
         fail(ERR_INVALID_ARGUMENT, "workspace too small for key switching");
     const int logn = c.logn;
     const size_t nn = c.n;
-    // one launch per stage needs the fused CKKS path and every group within one launch
+    // one launch per stage needs the fused CKKS path and every group, and every launch's groups
+    // together, within one launch; else group by group
     bool grouped = c.scheme == SCHEME_CKKS && logn >= 13 && logn <= 16;
-    for (uint32_t g = 0; g < n && grouped; g++)
+    std::vector<uint32_t> counts, levels;
+    for (uint32_t g = 0; g < n && grouped; g++) {
         grouped = (uint64_t)gs[g].count * gs[g].L * (gs[g].L + 1) <= ((uint64_t(1) << 34) >> logn);
+        counts.push_back(gs[g].count);
+        levels.push_back(gs[g].L);
+    }
+    if (grouped)
+        in_chunks(n, [&](uint32_t g0, uint32_t m) {
+            grouped = grouped && relinearize_groups_fit(logn, &counts[g0], &levels[g0], m);
+        });
     char *base = static_cast<char *>(ws);
     if (!grouped) {
         for (uint32_t g = 0; g < n; g++) {

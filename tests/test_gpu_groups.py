@@ -4,8 +4,8 @@ Each group's words must equal the one-level calls on that group (shc_ckks_multip
 shc_relinearize, shc_rescale_to_next), which the oracle pins elsewhere; one ciphertext
 per case is also checked against the oracle.  Covered: the fused CKKS path at N = 2^15
 (config 3's primes, levels 2..15, groups of 1..7 so that groups of 4 / 2 / 1 all run)
-and N = 2^16, more than 16 groups (taken 16 at a time), the group-by-group paths (BFV,
-N = 2^13), rescaling straight from size-3 ciphertexts, and a captured graph of a
+and N = 2^16, more than 16 groups (taken 16 at a time), the group-by-group paths (BFV, and
+batches past one grouped launch), rescaling straight from size-3 ciphertexts, and a captured graph of a
 grouped multiply -> relinearize -> rescale replayed with eager work between replays.
 """
 import numpy as np
@@ -59,7 +59,7 @@ def rescale_one(ctx, ct2, count, L):
     (CKKS, 15, [60] + [40] * 14 + [60], [(15, 2), (9, 5), (4, 3), (7, 1), (12, 7), (2, 2)]),
     (CKKS, 16, [60] * 6, [(5, 3), (3, 2), (4, 1)]),
     (CKKS, 15, [60] + [40] * 6 + [60], [(2 + k % 6, 1 + k % 3) for k in range(18)]),  # 18 groups: 16 + 2
-    (CKKS, 13, [60, 40, 40, 40, 60], [(4, 2), (2, 3)]),                               # group by group
+    (CKKS, 13, [60, 40, 40, 40, 60], [(4, 2), (2, 3)]),
     (BFV, 15, [60] * 5, [(4, 2), (2, 3)]),                                             # group by group
 ])
 def test_relinearize_groups_equal_one_level_calls(scheme, logn, bits, spec):
@@ -82,6 +82,28 @@ def test_relinearize_groups_equal_one_level_calls(scheme, logn, bits, spec):
 def test_relinearize_groups_small_rings(logn, spec):
     """One launch per stage at N = 2^13 and 2^14 too, with short last groups of 4."""
     test_relinearize_groups_equal_one_level_calls(CKKS, logn, [60, 40, 60, 40, 60], spec)
+
+
+def test_relinearize_groups_past_one_grouped_launch():
+    """131,072 ciphertexts of one limb at N = 2^13 are more blocks than a grouped launch has
+    (launch_limits.h): they run group by group, with the words of the one-level call."""
+    L, count, logn, n = 1, 131072, 13, 1 << 13
+    words = count * 3 * L * n
+    if torch.cuda.mem_get_info()[0] < 16 * words + (80 << 30):
+        pytest.skip("needs about 130 GB of device memory")
+    moduli = ck.coeff_modulus_create(n, [60, 60])
+    ctx = hip().Context(CKKS, n, moduli, 0)
+    key = to_dev(ck.random_key(np.random.default_rng(2), moduli, logn))
+    d = torch.randint(0, moduli[0], (count, 3, L, n), dtype=torch.int64, device="cuda")
+    ref = d.clone()
+    w = ctx.relinearize_groups_workspace_size([(d.data_ptr(), count, L)])
+    b = ws(max(w, ctx.keyswitch_workspace_size(count, L)))
+    ctx.relinearize_groups([(d.data_ptr(), count, L)], key.data_ptr(), b.data_ptr(), w, stream())
+    ctx.relinearize(ref.data_ptr(), key.data_ptr(), count, L, b.data_ptr(), ctx.keyswitch_workspace_size(count, L),
+                    stream())
+    assert all(torch.equal(d[c:c + 8192, :2], ref[c:c + 8192, :2]) for c in range(0, count, 8192))
+    del d, ref, b
+    torch.cuda.empty_cache()
 
 
 @pytest.mark.parametrize("logn,bits,spec", [
