@@ -471,7 +471,9 @@ int shc_rotate_many(const shc_context *ctx, const uint64_t *d_in, uint32_t count
  * [n][count][2][L][N] (not overlapping d_out): the words of separate
  * shc_apply_galois_keyswitch calls summed, with one ModDown for up to 15 of them -- the
  * giant steps of a BSGS matrix-vector product.  An element of 1 adds d_in[h] as it is (its
- * key may be NULL); d_galois_keys is a host array of device pointers. */
+ * key may be NULL); d_galois_keys is a host array of device pointers.  A workspace of the
+ * queried size holds every smaller batch too; a smaller one, down to one rotation's need, takes
+ * fewer rotations at a time. */
 int shc_rotate_accumulate_workspace_size(const shc_context *ctx, uint32_t count, uint32_t limb_count, size_t *bytes);
 int shc_rotate_accumulate(const shc_context *ctx, const uint64_t *d_in, uint32_t count, uint32_t limb_count,
                           const uint32_t *galois_elts, const uint64_t *const *d_galois_keys, uint32_t n,

@@ -45,11 +45,6 @@ void switch_key(const Context &c, const uint64_t *target, size_t target_stride, 
 //               + i * N.
 //   moddown_into: ct_k[i] += ModDown(P_k, S_k)[i] (folded: P holds p ct_k, and ct_k = ModDown; S is consumed; U is scratch
 //               [count][2][L][N]; P in NTT form).
-// The regions of a key-switch workspace of `count` ciphertexts at level L.
-struct KsRegions {
-    uint64_t *d, *T, *P, *S, *U;
-};
-KsRegions keyswitch_regions(const Context &c, uint32_t count, uint32_t L, void *ws);
 bool modup_to_T(const Context &c, const uint64_t *digits, size_t dstride, uint64_t *T, uint32_t count, uint32_t L,
                 hipStream_t st, const KernelProbe *probe = nullptr, bool skip_diag = false);
 void keyswitch_inner_product(const Context &c, const uint64_t *T, const uint64_t *key, uint64_t *P, uint64_t *S,

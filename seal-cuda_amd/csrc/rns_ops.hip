@@ -23,6 +23,7 @@
 #include "modarith.h"
 #include "ntt.h"
 #include "rns_ops.h"
+#include "workspaces.h"
 #include <type_traits>
 #include <vector>
 
@@ -373,24 +374,6 @@ void launch_elem_groups(const std::vector<ElemGroup> &gs, const DevPrime *primes
     launch_check("grouped elementwise");
 }
 
-struct KsLayout {
-    size_t d, T, P, S, U, total;
-};
-
-KsLayout ks_layout(const Context &c, uint32_t count, uint32_t L) {
-    const size_t limb = c.n * 8;
-    KsLayout l;
-    size_t off = 0;
-    auto take = [&](size_t limbs) { size_t o = off; off += (limbs * limb + 255) & ~size_t(255); return o; };
-    l.d = take((size_t)count * L);
-    l.T = take((size_t)count * L * (L + 1));
-    l.P = take((size_t)count * 2 * L);
-    l.S = take((size_t)count * 2);
-    l.U = take((size_t)count * 2 * L);
-    l.total = off;
-    return l;
-}
-
 }  // namespace
 
 void ckks_tensor(const Context &c, const uint64_t *a, const uint64_t *b, uint64_t *out, uint32_t count, uint32_t L,
@@ -408,14 +391,7 @@ void tensor_strided(const DevPrime *primes, const uint64_t *a, size_t a_stride, 
     launch_check("tensor");
 }
 
-size_t keyswitch_workspace(const Context &c, uint32_t count, uint32_t L) { return ks_layout(c, count, L).total; }
-
-KsRegions keyswitch_regions(const Context &c, uint32_t count, uint32_t L, void *ws) {
-    const KsLayout l = ks_layout(c, count, L);
-    char *b = static_cast<char *>(ws);
-    auto at = [b](size_t off) { return reinterpret_cast<uint64_t *>(b + off); };
-    return KsRegions{at(l.d), at(l.T), at(l.P), at(l.S), at(l.U)};
-}
+size_t keyswitch_workspace(const Context &c, uint32_t count, uint32_t L) { return ks_layout(c.logn, count, L).total; }
 
 namespace {
 
@@ -424,7 +400,7 @@ namespace {
 void switch_key_chunk(const Context &c, const uint64_t *target, size_t target_stride, uint64_t *ct,
                       size_t ct_stride, const uint64_t *key, uint32_t count, uint32_t L, void *ws, hipStream_t st,
                       const KernelProbe *probe, const uint64_t *fold_c0) {
-    const KsLayout lay = ks_layout(c, count, L);
+    const KsLayout lay = ks_layout(c.logn, count, L);
     char *base = static_cast<char *>(ws);
     uint64_t *d = reinterpret_cast<uint64_t *>(base + lay.d);
     uint64_t *T = reinterpret_cast<uint64_t *>(base + lay.T);
@@ -553,7 +529,7 @@ void switch_key(const Context &c, const uint64_t *target, size_t target_stride, 
     if (K < 2) fail(ERR_LOGIC, "keyswitching is not supported by the context");
     if (L < 1 || L > K - 1) fail(ERR_INVALID_ARGUMENT, "level out of range for key switching");
     if (!count) return;
-    if (!ws || ws_bytes < ks_layout(c, count, L).total)
+    if (!ws || ws_bytes < ks_layout(c.logn, count, L).total)
         fail(ERR_INVALID_ARGUMENT, "workspace too small for key switching");
     // The ModUp buffer has room for L(L+1) limbs per ciphertext; one NTT launch covers at most
     // 2^34 / N limbs, so large batches run in slices of whole ciphertexts.
@@ -657,7 +633,7 @@ void ckks_tensor_groups(const Context &c, const TensorGroup *gs, uint32_t n, hip
 
 size_t relinearize_groups_workspace(const Context &c, const RelinGroup *gs, uint32_t n) {
     size_t total = 0;
-    for (uint32_t g = 0; g < n; g++) total += ks_layout(c, gs[g].count, gs[g].L).total;
+    for (uint32_t g = 0; g < n; g++) total += ks_layout(c.logn, gs[g].count, gs[g].L).total;
     return total;
 }
 
@@ -689,7 +665,7 @@ void relinearize_groups(const Context &c, const RelinGroup *gs, uint32_t n, cons
     char *base = static_cast<char *>(ws);
     if (!grouped) {
         for (uint32_t g = 0; g < n; g++) {
-            const size_t poly = (size_t)gs[g].L * nn, bytes = ks_layout(c, gs[g].count, gs[g].L).total;
+            const size_t poly = (size_t)gs[g].L * nn, bytes = ks_layout(c.logn, gs[g].count, gs[g].L).total;
             switch_key(c, gs[g].ct + 2 * poly, 3 * poly, gs[g].ct, 3 * poly, key, gs[g].count, gs[g].L, base, bytes, st);
             base += bytes;
         }
@@ -703,7 +679,7 @@ void relinearize_groups(const Context &c, const RelinGroup *gs, uint32_t n, cons
         for (uint32_t g = g0; g < g0 + m; g++) {
             const RelinGroup &r = gs[g];
             const uint32_t L = r.L;
-            const KsLayout lay = ks_layout(c, r.count, L);
+            const KsLayout lay = ks_layout(c.logn, r.count, L);
             char *const gb = base;  // this group's workspace
             auto at = [gb](size_t off) { return reinterpret_cast<uint64_t *>(gb + off); };
             base += lay.total;

@@ -28,6 +28,7 @@
 #include "modarith.h"
 #include "ntt.h"
 #include "rns_ops.h"
+#include "workspaces.h"
 #include <algorithm>
 #include <type_traits>
 
@@ -91,7 +92,7 @@ __global__ void correction_kernel(const uint64_t *__restrict__ negntt, const uin
 // CU's cache; blocks of one tile run on one XCD (XCD = block % 8), whose L2 serves the
 // tile's key words to the other blocks.  Sums are Acc3, or (MIXED, a block of a prime
 // below 2^50: T holds words below 4 q) Acc26 at half the instructions.
-constexpr int RMAX = 4;
+constexpr int RMAX = ROT_MAX;
 static_assert(RMAX <= (int)PERM_MAX, "a pass's rotations fit one permuted ModDown");
 constexpr int RG = 2;
 struct RotBatch {
@@ -417,31 +418,6 @@ __global__ __launch_bounds__(TPB) void zero_digit_fix_kernel(RotBatch rb, const 
     }
 }
 
-struct RotLayout {
-    size_t ks, list, C0, Pm, Sm, U, S2, flag, zc, total;
-};
-
-// N >= 2^13: a pass's rotations share each launch, so the ModDown's scratch (U, S2) has
-// room for RMAX of them; below, one rotation at a time.
-RotLayout rot_layout(const Context &c, uint32_t count, uint32_t L) {
-    const size_t limb = c.n * 8;
-    RotLayout l;
-    size_t off = 0;
-    auto take = [&](size_t bytes) { size_t o = off; off += align256(bytes); return o; };
-    const size_t m = c.logn >= 13 ? RMAX : 1;
-    l.ks = take(keyswitch_workspace(c, count, L));
-    l.list = take((size_t)count * L * limb);
-    l.C0 = take((size_t)count * L * limb);
-    l.Pm = take((size_t)RMAX * count * 2 * L * limb);
-    l.Sm = take((size_t)RMAX * count * 2 * limb);
-    l.U = take(m * count * 2 * L * limb);
-    l.S2 = take(m * count * 2 * limb);
-    l.flag = take(8);
-    l.zc = take(8 * (2 + (size_t)count));
-    l.total = off;
-    return l;
-}
-
 void check_level(const Context &c, uint32_t L) {
     if (c.key_count() < 2) fail(ERR_LOGIC, "keyswitching is not supported by the context");
     if (L < 1 || L > c.key_count() - 1) fail(ERR_INVALID_ARGUMENT, "level out of range for key switching");
@@ -485,7 +461,7 @@ void hoisted_key_prepare(const Context &c, const uint64_t *galois_key, uint32_t 
     c.hoisted_keys[out] = {L, elt};
 }
 
-size_t rotate_sum_workspace(const Context &c, uint32_t count, uint32_t L) { return rot_layout(c, count, L).total; }
+size_t rotate_sum_workspace(const Context &c, uint32_t count, uint32_t L) { return rot_layout(c.logn, count, L).total; }
 
 namespace {
 
@@ -499,7 +475,7 @@ void rotate_hoisted(const Context &c, const uint64_t *in, uint32_t count, uint32
     if (!rotations || !elts || !hoisted || !keys) fail(ERR_INVALID_ARGUMENT, "no rotations given");
     KernelProbe probe{nullptr, nullptr};
     const bool armed = c.take_probe(probe);  // brackets the first pass of hoisted products
-    const RotLayout lay = rot_layout(c, count, L);
+    const RotLayout lay = rot_layout(c.logn, count, L);
     if (!ws || ws_bytes < lay.total) fail(ERR_INVALID_ARGUMENT, "workspace too small for rotation sums");
     if (in == out) fail(ERR_INVALID_ARGUMENT, "rotate_sum cannot run in place");
     const uint64_t max_cts = ((uint64_t(1) << 34) >> c.logn) / ((uint64_t)L * (L + 1));
@@ -508,12 +484,11 @@ void rotate_hoisted(const Context &c, const uint64_t *in, uint32_t count, uint32
     const int logn = c.logn;
     const size_t n = c.n, lw = (size_t)L * n;
     char *base = static_cast<char *>(ws);
-    uint64_t *list = reinterpret_cast<uint64_t *>(base + lay.list);
-    uint64_t *U = reinterpret_cast<uint64_t *>(base + lay.U);
-    uint64_t *S2 = reinterpret_cast<uint64_t *>(base + lay.S2);
-    uint64_t *C0 = reinterpret_cast<uint64_t *>(base + lay.C0);
+    auto at = [base](size_t off) { return reinterpret_cast<uint64_t *>(base + off); };
+    uint64_t *T = at(lay.T), *list = at(lay.list), *U = at(sum ? lay.U_sum : lay.U), *S2 = at(lay.S2);
+    uint64_t *c_limbs = at(lay.c);  // CKKS: the digits; BFV, N >= 2^13: c0 in NTT form
+    uint64_t *Pm = at(lay.Pm), *Sm = at(sum ? lay.Sm_sum : lay.Sm);
     auto *flag = reinterpret_cast<unsigned long long *>(base + lay.flag);
-    const KsRegions ks = keyswitch_regions(c, count, L, base + lay.ks);
 
     // each prepared key must be the one of this level and element: checked on the
     // host for keys prepared through this context; other keys' header words are read
@@ -548,14 +523,14 @@ void rotate_hoisted(const Context &c, const uint64_t *in, uint32_t count, uint32
         if (flags & 2)
             fail(ERR_INVALID_ARGUMENT, "a hoisted key was prepared for another level or Galois element");
     }
-    // 1. digits of c1 in coefficient form (CKKS: transformed into ks.d; c1 itself, in NTT
+    // 1. digits of c1 in coefficient form (CKKS: transformed into the workspace; c1 itself, in NTT
     // form, supplies the own-prime terms of the products)
     const uint64_t *digits = in + lw;
     size_t dstride = 2 * lw;
     if (ckks) {
-        ntt_inverse_from(in + lw, LimbGrid{1, 2 * L, L, count}, ks.d, LimbGrid{1, L, L, count}, c.primes(), logn,
+        ntt_inverse_from(in + lw, LimbGrid{1, 2 * L, L, count}, c_limbs, LimbGrid{1, L, L, count}, c.primes(), logn,
                          NTT_FULL, st);
-        digits = ks.d;
+        digits = c_limbs;
         dstride = lw;
     }
     // 2. zero digits, listed for the products' fix (the list has room for every word)
@@ -565,35 +540,31 @@ void rotate_hoisted(const Context &c, const uint64_t *in, uint32_t count, uint32
     launch_check("zero digits");
     const size_t ct_words = (size_t)count * 2 * lw;
     // 3. one ModUp for every rotation
-    const bool skipped = modup_to_T(c, digits, dstride, ks.T, count, L, st, nullptr, ckks);
+    const bool skipped = modup_to_T(c, digits, dstride, T, count, L, st, nullptr, ckks);
     // T words below 4 q_i where the fp64 transforms (N >= 2^13) or full reduction made them
     const bool acc26 = c.fp_primes;
     const uint64_t *diag = skipped ? in + lw : nullptr;
     const DevPrime *targets = c.keyswitch_primes(L);
     const size_t K = c.key_count();
     const size_t corr_off = (K - 1) * 2 * K * n;
-    uint64_t *Pm = reinterpret_cast<uint64_t *>(base + lay.Pm);
-    uint64_t *Sm = reinterpret_cast<uint64_t *>(base + lay.Sm);
     // N >= 2^13: c0 joins the products (in NTT form: BFV's c0 is transformed once for all
     // rotations), the products are permuted as the ModDown reads them, and a pass's
     // rotations -- or, when summing, up to 15 of them -- take one ModDown
-    const bool batched = logn >= 13;
     KsFold fold{};
-    if (batched) {
+    if (lay.batched) {
         fold = KsFold{in, 2 * lw, c.ks_consts()};
         if (!ckks) {
-            const NttGroup g{C0, in, LimbGrid{1, L, L, count}, LimbGrid{1, 2 * L, L, count}, c.primes()};
+            const NttGroup g{c_limbs, in, LimbGrid{1, L, L, count}, LimbGrid{1, 2 * L, L, count}, c.primes()};
             ntt_forward_groups(&g, 1, logn, NTT_FULL, st);
-            fold = KsFold{C0, lw, c.ks_consts()};
+            fold = KsFold{c_limbs, lw, c.ks_consts()};
         }
     }
-    const RotArgs args{ks.T, corr_off, targets, L, (uint32_t)K, logn, count, 0, diag, 2 * lw, fold};
-    constexpr uint32_t SUM_MAX = 15;  // rotations per summed ModDown (15 words below 2^60)
+    const RotArgs args{T, corr_off, targets, L, (uint32_t)K, logn, count, 0, diag, 2 * lw, fold};
     // rotations per pass: RMAX, fewer where one launch cannot hold their limbs
     uint32_t pass = RMAX;
-    while (batched && pass > 1 && (uint64_t)pass * count * 2 * L > ((uint64_t(1) << 34) >> logn)) pass--;
+    while (lay.batched && pass > 1 && (uint64_t)pass * count * 2 * L > ((uint64_t(1) << 34) >> logn)) pass--;
     const uint64_t p = c.moduli[K - 1];
-    uint32_t summed = 0;  // rotations in ks.U, ks.S
+    uint32_t summed = 0;  // rotations in Psum, V
     for (uint32_t r0 = 0; r0 < rotations; r0 += pass) {
         const uint32_t nr = std::min(rotations - r0, pass);
         // products with the prepared keys (corrections included), RMAX rotations per pass over T
@@ -615,7 +586,8 @@ void rotate_hoisted(const Context &c, const uint64_t *in, uint32_t count, uint32
             default: zero_digit_fix_kernel<4><<<fix_blocks, TPB, 0, st>>>(rb, zc, list, targets, c.primes(), L, (uint32_t)K, logn, count, fold); break;
         }
         launch_check("zero_digit_fix");
-        if (!batched) {
+        if (!lay.batched) {
+            uint64_t *C0 = at(lay.C0), *P2 = at(lay.P2);
             for (uint32_t q = 0; q < nr; q++) {
                 const uint32_t r = r0 + q;
                 uint64_t *dst = sum ? out : out + r * ct_words;
@@ -625,9 +597,9 @@ void rotate_hoisted(const Context &c, const uint64_t *in, uint32_t count, uint32
                                                                              !sum || r == 0, count * lw);
                 launch_check("accumulate_c0");
                 // the products permuted by sigma, then this rotation's ModDown added into dst
-                apply_galois(c, rb.P[q], lw, U, lw, count * 2, L, elts[r], true, st);
+                apply_galois(c, rb.P[q], lw, P2, lw, count * 2, L, elts[r], true, st);
                 apply_galois(c, rb.S[q], n, S2, n, count * 2, 1, elts[r], true, st);
-                moddown_into(c, U, S2, ks.U, dst, 2 * lw, count, L, st);
+                moddown_into(c, P2, S2, U, dst, 2 * lw, count, L, st);
             }
             continue;
         }
@@ -644,7 +616,8 @@ void rotate_hoisted(const Context &c, const uint64_t *in, uint32_t count, uint32
             ntt_moddown(ckks, U, md, count * nr, c.primes(), logn, st);
             continue;
         }
-        SumArgs sa{Pm, S2, ks.U, ks.S, {}, p};
+        uint64_t *Psum = at(lay.Psum), *V = at(lay.V);
+        SumArgs sa{Pm, S2, Psum, V, {}, p};
         for (uint32_t q = 0; q < nr; q++) sa.elt[q] = elts[r0 + q];
         const size_t total = (size_t)2 * count * (L + 1) * n;
         sum_products_kernel<<<blocks_for(total), TPB, 0, st>>>(sa, nr, c.primes(), L, logn, 2 * count, summed == 0, total);
@@ -652,12 +625,12 @@ void rotate_hoisted(const Context &c, const uint64_t *in, uint32_t count, uint32
         summed += nr;
         const uint32_t next = std::min(rotations - (r0 + nr), pass);
         if (!next || summed + next > SUM_MAX) {
-            md.S = ks.S;
-            md.P = ks.U;
+            md.S = V;
+            md.P = Psum;
             md.ct = out;
             md.folded = r0 + nr == summed;  // the first sums write out, later ones add
             md.presum = summed;
-            ntt_moddown(ckks, ckks ? U : ks.U, md, count, c.primes(), logn, st);
+            ntt_moddown(ckks, ckks ? U : Psum, md, count, c.primes(), logn, st);
             summed = 0;
         }
     }
@@ -734,45 +707,10 @@ __global__ void galois_digits_kernel(SumC0Args a, uint64_t *__restrict__ d, cons
     }
 }
 
-struct AccLayout {
-    bool batched;   // else one rotation at a time through tmp
-    uint32_t nb;    // rotations per batch
-    size_t d, T, P, S, Psum, V, U, tmp, total;
-};
-
-// N = 2^15, 2^16: the fused key products take one rotation's T at a time; other degrees a
-// batch's.
-AccLayout acc_layout(const Context &c, uint32_t count, uint32_t L) {
-    const size_t limb = c.n * 8;
-    AccLayout l{};
-    size_t off = 0;
-    auto take = [&](size_t limbs) { size_t o = off; off += align256(limbs * limb); return o; };
-    const uint64_t most = (uint64_t(1) << 34) >> c.logn, per = (uint64_t)count * L * (L + 1);
-    l.batched = c.logn >= 13 && per <= most;
-    if (!l.batched) {
-        l.tmp = take((size_t)count * 2 * L);
-        off += galois_keyswitch_workspace(c, count, L);
-        l.total = off;
-        return l;
-    }
-    const bool fused = c.logn == 15 || c.logn == 16;
-    l.nb = PERM_MAX;
-    while (l.nb > 1 && l.nb * per > most) l.nb--;
-    l.d = take((size_t)l.nb * count * L);
-    l.T = take((fused ? 1 : l.nb) * (size_t)count * L * (L + 1));
-    l.P = take((size_t)l.nb * count * 2 * L);
-    l.S = take((size_t)l.nb * count * 2);
-    l.Psum = take((size_t)count * 2 * L);
-    l.V = take((size_t)count * 2);
-    l.U = take((size_t)count * 2 * L);
-    l.total = off;
-    return l;
-}
-
 }  // namespace
 
 size_t rotate_accumulate_workspace(const Context &c, uint32_t count, uint32_t L) {
-    return acc_layout(c, count, L).total;
+    return acc_workspace(c.logn, count, L);
 }
 
 void rotate_accumulate(const Context &c, const uint64_t *in, uint32_t count, uint32_t L, const uint32_t *elts,
@@ -782,8 +720,9 @@ void rotate_accumulate(const Context &c, const uint64_t *in, uint32_t count, uin
     if (!count) return;
     if (!n || !elts || !keys) fail(ERR_INVALID_ARGUMENT, "no rotations given");
     if (in == out) fail(ERR_INVALID_ARGUMENT, "rotate_accumulate cannot run in place");
-    const AccLayout lay = acc_layout(c, count, L);
-    if (!ws || ws_bytes < lay.total) fail(ERR_INVALID_ARGUMENT, "workspace too small for rotation sums");
+    const uint32_t most_nb = ws ? acc_rotations(c.logn, count, L, ws_bytes) : 0;
+    if (!most_nb) fail(ERR_INVALID_ARGUMENT, "workspace too small for rotation sums");
+    const AccLayout lay = acc_layout(c.logn, count, L, most_nb);
     const size_t N = c.n, lw = (size_t)L * N, ctw = 2 * lw, step = (size_t)count * ctw;
     for (uint32_t h = 0; h < n; h++) {
         if (!(elts[h] & 1) || elts[h] >= 2 * N) fail(ERR_INVALID_ARGUMENT, "Galois element is not valid");
@@ -830,7 +769,7 @@ void rotate_accumulate(const Context &c, const uint64_t *in, uint32_t count, uin
             continue;
         }
         uint32_t nb = 1;  // consecutive switches, at most a summed ModDown's 15 in all
-        while (nb < lay.nb && h0 + nb < n && elts[h0 + nb] != 1 && summed + nb < 15) nb++;
+        while (nb < most_nb && h0 + nb < n && elts[h0 + nb] != 1 && summed + nb < SUM_MAX) nb++;
         const uint64_t *x = in + h0 * step;
         GaloisPerm perm{count, {}};
         InnerKeys ik{};
@@ -852,7 +791,7 @@ void rotate_accumulate(const Context &c, const uint64_t *in, uint32_t count, uin
             galois_digits_kernel<<<blocks_for(total), TPB, 0, st>>>(ga, d, c.primes(), total);
             launch_check("galois_digits");
         }
-        if (logn == 15 || logn == 16) {
+        if (acc_fused(logn)) {
             for (uint32_t h = 0; h < nb; h++)
                 ntt_modup_keyprod(d + h * count * lw, lw, T, ik.key[h], P + h * step, S + (size_t)h * count * 2 * N,
                                   ckks ? x + h * step + lw : nullptr, ctw, count, L, K, targets, c.primes(), logn,
@@ -870,7 +809,7 @@ void rotate_accumulate(const Context &c, const uint64_t *in, uint32_t count, uin
         summed += nb;
         left -= nb;
         h0 += nb;
-        if (summed == 15 || !left) {
+        if (summed == SUM_MAX || !left) {
             ModDownArgs md{V, Psum, out, ctw, c.ks_consts(), c.moduli[K - 1], L, false};
             md.presum = summed;
             ntt_moddown(ckks, ckks ? at(lay.U) : Psum, md, count, c.primes(), logn, st);

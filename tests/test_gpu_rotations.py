@@ -131,6 +131,23 @@ def test_rotation_passes_zero_digits(scheme, zeros):
     (BFV, 15, [60, 50, 60], 2, 2, [1, 0]),
 ])
 def test_rotate_accumulate(scheme, logn, bits, L, count, steps):
+    accumulate_case(scheme, logn, bits, L, count, steps)
+
+
+@pytest.mark.parametrize("scheme,logn,bits,count", [
+    (CKKS, 13, [60, 40, 60], 3), (BFV, 13, [43, 44, 44], 2), (CKKS, 15, [60, 40, 60], 2), (BFV, 17, [60, 60, 60], 1)])
+def test_rotate_accumulate_in_smaller_workspaces(scheme, logn, bits, count):
+    """Every workspace from one rotation's need up gives the words, with as many rotations at a
+    time as it holds (regions of whole limbs: digits, T, products, sums, corrections)."""
+    L, n = 2, 1 << logn
+    for nb in (1, 2, 3):
+        T = 6 * (1 if logn in (15, 16) else nb)
+        accumulate_case(scheme, logn, bits, L, count, [1, 2, None, 3, 4, 5],
+                        (T + nb * (3 * L + 2) + 4 * L + 2) * count * n * 8, refused=nb == 1)
+
+
+def accumulate_case(scheme, logn, bits, L, count, steps, ws_bytes=None, refused=False):
+    """ws_bytes: None for the size that is asked for.  refused: one byte less is too small."""
     n = 1 << logn
     moduli = ck.coeff_modulus_create(n, bits)
     ctx = hip().Context(scheme, n, moduli, 65537 if scheme == BFV else 0)
@@ -140,9 +157,14 @@ def test_rotate_accumulate(scheme, logn, bits, L, count, steps):
     keys = [None if s is None else ck.random_key(rng, moduli, logn) for s in steps]
     dkeys = [None if k is None else to_dev(k) for k in keys]
     din, out = to_dev(cts), empty_dev((count, 2, L, n))
-    wb = ctx.rotate_accumulate_workspace_size(count, L)
-    ctx.rotate_accumulate(din.data_ptr(), count, L, elts, [None if k is None else k.data_ptr() for k in dkeys],
-                          out.data_ptr(), ws(wb).data_ptr(), wb, stream())
+    wb = ctx.rotate_accumulate_workspace_size(count, L) if ws_bytes is None else ws_bytes
+    buf = ws(wb)
+    args = (din.data_ptr(), count, L, elts, [None if k is None else k.data_ptr() for k in dkeys], out.data_ptr(),
+            buf.data_ptr())
+    if refused:
+        with pytest.raises(hip().SealHipError, match="workspace too small"):
+            ctx.rotate_accumulate(*args, wb - 1, stream())
+    ctx.rotate_accumulate(*args, wb, stream())
     got = from_dev(out)
     for c in range(count):
         want = None
