@@ -701,7 +701,7 @@ __global__ void galois_digits_kernel(SumC0Args a, uint64_t *__restrict__ d, cons
         const uint32_t r = uniform_row(idx, a.logn), g = r / a.L, i = r - g * a.L, h = g / a.count;
         const uint32_t off = (uint32_t)(idx & (n - 1));
         const uint32_t k = (uint32_t)(((uint64_t)off * a.elt_inv[h]) & (n - 1));
-        uint64_t x = a.in[(((size_t)g * 2 + 1) * a.L + i << a.logn) + k];
+        uint64_t x = a.in[((((size_t)g * 2 + 1) * a.L + i) << a.logn) + k];
         if (((uint64_t)k * a.elt[h] >> a.logn) & 1) x = negmod(x, primes[i].q);
         d[idx] = x;
     }
@@ -719,11 +719,12 @@ void rotate_accumulate(const Context &c, const uint64_t *in, uint32_t count, uin
     check_level(c, L);
     if (!count) return;
     if (!n || !elts || !keys) fail(ERR_INVALID_ARGUMENT, "no rotations given");
-    if (in == out) fail(ERR_INVALID_ARGUMENT, "rotate_accumulate cannot run in place");
     const uint32_t most_nb = ws ? acc_rotations(c.logn, count, L, ws_bytes) : 0;
     if (!most_nb) fail(ERR_INVALID_ARGUMENT, "workspace too small for rotation sums");
     const AccLayout lay = acc_layout(c.logn, count, L, most_nb);
     const size_t N = c.n, lw = (size_t)L * N, ctw = 2 * lw, step = (size_t)count * ctw;
+    // (the sums are written while later ciphertexts' permuted words are still to be read)
+    if (out < in + n * step && in < out + step) fail(ERR_INVALID_ARGUMENT, "rotate_accumulate cannot run in place");
     for (uint32_t h = 0; h < n; h++) {
         if (!(elts[h] & 1) || elts[h] >= 2 * N) fail(ERR_INVALID_ARGUMENT, "Galois element is not valid");
         if (elts[h] != 1 && !keys[h]) fail(ERR_INVALID_ARGUMENT, "null key pointer");

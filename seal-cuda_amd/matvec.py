@@ -59,7 +59,8 @@ class BsgsMatvec:
 
     def run(self, d_in, count, d_out, d_baby, d_inner, d_ws, ws_bytes, stream=None, around_sums=None):
         """d_in, d_out: [count][2][L][N]; d_baby: scratch [b][count][2][L][N];
-        d_inner: scratch [g][count][2][L][N]; d_ws: workspace_sizes(count) bytes.
+        d_inner: scratch [g][count][2][L][N]; d_ws: workspace_sizes(count) bytes.  d_out may lie
+        in the scratch: the result is then summed elsewhere in it and copied.
         around_sums: optional (before, after) callables invoked right before and after the
         inner-sum launch (e.g. recording timing events on `stream`)."""
         import ctypes
@@ -85,8 +86,14 @@ class BsgsMatvec:
         if g == 1:
             _memcpy_d2d(d_out, d_inner, ct_bytes, stream)
         else:
-            ctx.rotate_accumulate(d_inner, count, L, [1] + self.giant_elts, [None] + list(self.giant_keys), d_out, d_ws,
+            # the sums are written while d_inner and the workspace are still read; d_baby is free
+            apart = all(d_out + ct_bytes <= at or at + size <= d_out
+                        for at, size in ((d_inner, g * ct_bytes), (d_ws, ws_bytes)))
+            out = d_out if apart else d_baby
+            ctx.rotate_accumulate(d_inner, count, L, [1] + self.giant_elts, [None] + list(self.giant_keys), out, d_ws,
                                   ws_bytes, stream)
+            if not apart:
+                _memcpy_d2d(d_out, out, ct_bytes, stream)
 
 
 _rt = None

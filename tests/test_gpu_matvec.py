@@ -241,13 +241,19 @@ def test_bsgs_matvec_ckks_batch_equals_alone():
                            [h.data_ptr() for h in hoisted], [k.data_ptr() for k in giant])
     cts = to_dev(ck.uniform_residues(rng, (3, 2, L, n), moduli[:L]))
 
-    def run(x, count):
+    def run(x, count, place=None):
         out, bb, inner = empty_dev((count, 2, L, n)), empty_dev((b, count, 2, L, n)), empty_dev((g, count, 2, L, n))
         wsz = mv.workspace_sizes(count)
         wb = ws(wsz)
+        if place is not None:
+            out = place(x, bb, inner)
         mv.run(x.data_ptr(), count, out.data_ptr(), bb.data_ptr(), inner.data_ptr(), wb.data_ptr(), wsz, stream())
         return from_dev(out)
 
     batched = run(cts, 3)
     for k in range(3):
         np.testing.assert_array_equal(run(cts[k:k + 1].contiguous(), 1)[0], batched[k])
+    # the result in the scratch, or over the input
+    for place in (lambda x, bb, inner: inner[0], lambda x, bb, inner: inner[1], lambda x, bb, inner: bb[0],
+                  lambda x, bb, inner: x):
+        np.testing.assert_array_equal(run(cts.clone(), 3, place), batched)

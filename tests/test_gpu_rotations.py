@@ -146,6 +146,32 @@ def test_rotate_accumulate_in_smaller_workspaces(scheme, logn, bits, count):
                         (T + nb * (3 * L + 2) + 4 * L + 2) * count * n * 8, refused=nb == 1)
 
 
+def test_rotate_accumulate_rejects():
+    logn, n, L, count = 13, 1 << 13, 2, 2
+    moduli = ck.coeff_modulus_create(n, [60, 40, 60])
+    ctx = hip().Context(CKKS, n, moduli)
+    rng = np.random.default_rng(4)
+    din = to_dev(ck.uniform_residues(rng, (3, count, 2, L, n), moduli[:L]))
+    key = to_dev(ck.random_key(rng, moduli, logn))
+    out = empty_dev((count, 2, L, n))
+    wb = ctx.rotate_accumulate_workspace_size(count, L)
+    buf = ws(wb)
+    e = ck.galois_elt(logn, 1)
+
+    def call(elts, keys, dst, w=wb):
+        ctx.rotate_accumulate(din.data_ptr(), count, L, elts, keys, dst.data_ptr(), buf.data_ptr(), w, stream())
+
+    k = key.data_ptr()
+    for elts, keys, dst in (([1, e, 2], [None, k, k], out), ([1, e, 2 * n + 1], [None, k, k], out),  # no such element
+                            ([1, e, e], [None, k, None], out),                                       # no key
+                            ([1, e, e], [None, k, k], din[0]), ([1, e, e], [None, k, k], din[2])):   # over the input
+        with pytest.raises(hip().SealHipError):
+            call(elts, keys, dst)
+    with pytest.raises(hip().SealHipError):
+        call([e], [k], out, 0)
+    call([1, e, e], [None, k, k], out)
+
+
 def accumulate_case(scheme, logn, bits, L, count, steps, ws_bytes=None, refused=False):
     """ws_bytes: None for the size that is asked for.  refused: one byte less is too small."""
     n = 1 << logn
