@@ -213,8 +213,8 @@ __global__ __launch_bounds__(TPB, 3) void plain_dot_many_kernel(const uint64_t *
 // 80 GB through L2 for 12 GB of operands (32 terms x 32 outputs x 32 polynomials, N = 2^15,
 // L = 15) and waited for it.  A thread keeps 4 x 4 sums of its position (8 LDS words for 16
 // products); the words of the next JC terms are requested while these are summed.  Primes
-// below 2^50 stage the words cut at 26 bits and sum in Acc26.  That product took 10.2 ms, now
-// 4.8 (12 GB at 2.5 TB/s; 158 VGPRs, three blocks per CU).  32 positions per block (512
+// below 2^50 stage the words cut at 26 bits and sum in Acc26.  That product takes 4.6 ms (12 GB
+// at 2.6 TB/s; 148 VGPRs, three blocks per CU), 10.0 per thread.  32 positions per block (512
 // threads) measured 5.2 ms held to 128 VGPRs (13 spilled) and 5.7 ms without.
 constexpr int PT = 16;           // positions per block (128-byte rows)
 constexpr int DT = 16;           // outputs, and polynomials, per block
@@ -314,6 +314,21 @@ __global__ __launch_bounds__(DB, 3) void plain_dot_tiles_kernel(DotArgs a) {
     const uint32_t h0 = sub / a.gb * DT, g0 = sub % a.gb * DT;
     if (P.fwd_fp) plain_dot_tile<true>(lds, a, r0, P, h0, g0);
     else plain_dot_tile<false>(lds, a, r0, P, h0, g0);
+}
+
+// Where the tiles beat the per-thread form: a tile costs the same however many of its 16 x 16
+// sums are asked for, and its set-up weighs more the fewer terms there are, so the line is a
+// share of the tiles' sums, in sixteenths, for terms >= 16, >= 8, >= 2 and 1, one lower for Acc26
+// sums of 8 terms and more, and for 16 terms of fewer polynomials than outputs.  Measured,
+// per-thread / tiles in us, N = 2^15 (60-bit primes, L = 12 and 15; 40-bit): 32 terms 8x16
+// (outputs x polynomials) 1,291 / 1,325 and 1,290 / 1,051 (a half), 16x8 1,376 / 1,315, 12x12
+// 1,555 / 1,337 (9/16), 20x20 4,082 / 5,026 and 4,080 / 3,979 (6/16); ratios at 8 terms 12x12 1.01, 16x10
+// 1.06 (10/16), 40-bit 1.02; at 2 terms 16x10 0.88, 11x16 1.09 (11/16), 40-bit 0.98 and 1.19; at
+// 1 term 24x16 679 / 757 (12/16), 16x16 458 / 395, 40-bit 679 / 698.
+bool plain_dot_takes_tiles(uint32_t terms, uint32_t outputs, uint32_t polys, bool fp) {
+    const uint64_t slots = (uint64_t)((outputs + DT - 1) / DT) * ((polys + DT - 1) / DT) * DT * DT;
+    const uint32_t line = terms >= 16 ? 9 - (fp || polys < outputs) : terms >= 8 ? 10 - fp : terms >= 2 ? 11 : 14 - 2 * fp;
+    return 16 * (uint64_t)outputs * polys >= line * slots;
 }
 
 template <int H>
@@ -423,11 +438,11 @@ void multiply_plain_accumulate_many(const Context &c, const uint64_t *cts, const
     const uint32_t G = polys >= 2 ? 2 : 1;
     const DevPrime *primes = c.primes();
     const int logn = c.logn;
-    // tiles of 16 outputs x 16 polynomials where both are at least half of one (below, a
-    // tile's idle sums cost more than the per-thread form's repeated loads)
     const uint64_t tiles = ((uint64_t)L << logn) / PT;
     const uint64_t tile_blocks = (tiles + 7) / 8 * 8 * ((outputs + DT - 1) / DT) * ((polys + DT - 1) / DT);
-    if (polys >= DT / 2 && outputs >= DT / 2 && logn >= 5 && tile_blocks < (uint64_t(1) << 32) / DB) {
+    uint32_t fp = 0;
+    for (uint32_t i = 0; i < L; i++) fp += c.host_primes[i].fwd_fp != nullptr;
+    if (plain_dot_takes_tiles(terms, outputs, polys, 2 * fp > L) && logn >= 5 && tile_blocks < (uint64_t(1) << 32) / DB) {
         const DotArgs a{cts, plains, out, primes, terms, outputs, polys, L, logn, (uint32_t)tiles,
                         (outputs + DT - 1) / DT, (polys + DT - 1) / DT};
         plain_dot_tiles_kernel<<<(uint32_t)tile_blocks, DB, 0, st>>>(a);

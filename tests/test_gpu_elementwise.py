@@ -139,7 +139,10 @@ def test_plain_ops_reject_bad_arguments():
 
 
 @pytest.mark.parametrize("terms,outputs,polys,logn", [
-    (1, 8, 8, 5), (3, 16, 16, 10), (2, 17, 15, 11), (65, 9, 33, 10), (130, 33, 8, 6), (64, 16, 17, 12)])
+    (1, 8, 8, 5), (3, 16, 16, 10), (2, 17, 15, 11), (65, 9, 33, 10), (130, 33, 8, 6), (64, 16, 17, 12),
+    # ragged tiles, at and on both sides of the shares from which tiles are taken
+    (1, 14, 14, 5), (1, 13, 14, 6), (2, 15, 31, 6), (5, 16, 11, 10), (5, 16, 10, 10), (65, 13, 47, 6), (64, 9, 15, 12),
+    (64, 31, 9, 5), (9, 16, 10, 5)])
 @pytest.mark.parametrize("words", ["uniform", "largest"])
 def test_plain_dot_tiles(terms, outputs, polys, logn, words):
     """Tiles of 16 outputs x 16 polynomials (edges, odd stage counts, folds every 64 terms,
