@@ -448,9 +448,9 @@ struct PassShape {
 };
 // f(std::true_type) for a small launch over `limbs` limbs, else f(std::false_type).
 template <int LOGN, class F>
-void with_shape(uint64_t limbs, F &&f) {
+void with_shape(uint64_t limbs, F &&f, uint64_t line = SMALL_WORDS) {
     if constexpr (LOGN <= 16) {
-        if (limbs << LOGN <= SMALL_WORDS) {
+        if (limbs << LOGN <= line) {
             f(std::true_type{});
             return;
         }

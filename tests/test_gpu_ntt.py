@@ -133,9 +133,9 @@ def test_multi_degree_transforms_in_one_launch():
 
 @pytest.mark.parametrize("logn", [13, 14, 15, 16])
 def test_launch_forms_agree(logn):
-    """A batch past 2^26 words (16 values per thread) against the same limbs in slices below it
-    (4 values per thread), forward and inverse; the small form is checked against the oracle
-    above."""
+    """A batch past 2^26 words (16 values per thread) against the same limbs in slices below 2^23
+    (4 values per thread), forward and inverse, and batches at the lines themselves (2^23 forward,
+    2^24 inverse); the small form is checked against the oracle above."""
     import torch
     n = 1 << logn
     moduli = ck.coeff_modulus_create(n, [60, 40])
@@ -148,7 +148,14 @@ def test_launch_forms_agree(logn):
     for transform in (ctx.ntt_forward, ctx.ntt_inverse):
         whole, parts = data.clone(), data.clone()
         transform(whole.data_ptr(), polys, 2, stream())
-        for p0 in range(0, polys, polys // 3):
-            transform(parts[p0].data_ptr(), min(polys // 3, polys - p0), 2, stream())
+        step = polys // 17
+        for p0 in range(0, polys, step):
+            transform(parts[p0].data_ptr(), min(step, polys - p0), 2, stream())
         torch.cuda.synchronize()
         assert torch.equal(whole, parts)
+        for line in (1 << 23, 1 << 24):
+            for at in (line // n // 2 - 1, line // n // 2):
+                some = data[:at].clone()
+                transform(some.data_ptr(), at, 2, stream())
+                torch.cuda.synchronize()
+                assert torch.equal(some, parts[:at])
