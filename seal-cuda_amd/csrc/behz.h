@@ -11,9 +11,7 @@ namespace shc {
 
 struct Context;
 
-// Offsets (in 64-bit words) into one device buffer; all Shoup operands are stored as
-// (w, floor(w 2^64 / p)) pairs.
-// A base conversion's matrix for the matrix cores (conv_tile in behz.hip): operand A of
+// A base conversion's matrix for the matrix cores (conv_outputs in behz.hip): operand A of
 // 32 x 32 x 32 int8 products, 4 outputs x 8 byte weights by 4 terms x 8 byte digits per
 // step, and each output's reduction constants.  terms == 0: the shape or the primes are
 // outside its range, and the conversion runs on the vector unit.
@@ -28,6 +26,8 @@ struct ConvDev {
     const ConvOut *out = nullptr;    // [outputs]
 };
 
+// Offsets (in 64-bit words) into one device buffer; all Shoup operands are stored as
+// (w, floor(w 2^64 / p)) pairs.
 struct BehzDev {
     uint32_t L, bsz, bsk;            // |q|, |B|, |Bsk| = |B| + 1
     uint64_t m_sk, m_tilde_neg_inv_q; // m_sk; -prod(q)^-1 mod 2^32

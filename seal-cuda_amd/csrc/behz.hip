@@ -237,7 +237,17 @@ __global__ __launch_bounds__(BT) void behz_sk_kernel(const uint64_t *__restrict_
 // 2 outputs at one coefficient.  CF coefficients' digits are staged in LDS once for all outputs.
 // At N = 2^16, L = 24, 32 pairs: extend 1,073 -> 692 us (each operand), floor 1,836 -> 1,286,
 // Shenoy-Kumaresan 1,626 -> 1,003 (2.4, 3.0 and 2.5 TB/s).  The vector-unit kernels above keep
-// N < 128, more than 48 terms, and outputs below 2^33.
+// N < 128, more than 48 terms, and outputs below 2^33; and the levels at which staging digits
+// and putting bytes together cost more than the products saved.  A product of count pairs,
+// vector / matrix in us: L = 2, 2^14 coefficients 42.4 / 44.0, 2^20 514 / 598; L = 4 53.3 / 53.3 and
+// 918 / 980; L = 6 2^14 65.5 / 61.9, 2^17 180 / 174, 2^18 335 / 335, 2^20 1,353 / 1,381; L = 8 74.5 /
+// 70.3, 225 / 219, 427 / 429, 1,726 / 1,750; L = 10 84.6 / 77.2, 291 / 275, 540 / 523, 2,157 / 2,149;
+// L = 12 2^20 2,672 / 2,563 (N = 2^14; N = 2^7 to 2^16 alike).
+constexpr uint32_t CONV_LEVEL = 6, CONV_LEVEL_ANY = 10;
+constexpr uint64_t CONV_COEFFS = uint64_t(1) << 17;
+bool conv_on_matrix(uint32_t L, uint64_t coeffs) {
+    return L >= CONV_LEVEL_ANY || (L >= CONV_LEVEL && coeffs <= CONV_COEFFS);
+}
 constexpr int CF = 128;
 constexpr int CT = 256;
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -539,7 +549,9 @@ void build_behz_level(Context &c, uint32_t L, BehzLevel &out) {
         const uint32_t T = terms + (extra ? 1 : 0), O = (uint32_t)mods.size();
         for (uint64_t p : mods)
             if (p >> 61 || p < (uint64_t(1) << 33)) return;  // the quotient estimate's range
-        if (T > 48 || c.n < CF) return;  // 64 KB of staged digits; whole tiles of coefficients
+        // 48 KB of staged digits (the int32 sums would hold 63 terms); whole tiles of
+        // coefficients; never taken below CONV_LEVEL
+        if (T > 48 || c.n < CF || L < CONV_LEVEL) return;
         dev.terms = T;
         dev.steps = (T + 3) / 4;
         dev.outputs = O;
@@ -656,7 +668,8 @@ void bfv_multiply(const Context &c, const uint64_t *a, const uint64_t *b, uint64
     const DevPrime *bp = B.bsk_primes;
     const size_t ext = (size_t)count * 2 * n;
     const size_t lds = (size_t)(L > B.bsz ? L : B.bsz) * CW * 8;
-    if (B.ext_conv.terms) {
+    const bool matrix = conv_on_matrix(L, (uint64_t)count << logn);
+    if (matrix && B.ext_conv.terms) {
         launch_conv<CONV_EXTEND>(a, nullptr, Ab, B, B.ext_conv, qp, logn, ext, st);
         launch_conv<CONV_EXTEND>(b, nullptr, Bb, B, B.ext_conv, qp, logn, ext, st);
     } else {
@@ -694,14 +707,14 @@ void bfv_multiply(const Context &c, const uint64_t *a, const uint64_t *b, uint64
         ntt_inverse(Tb, count * 3 * bsk, bsk, bp, logn, NTT_FULL, st);
     }
     const size_t fl = (size_t)count * 3 * n;
-    if (B.floor_conv.terms)
+    if (matrix && B.floor_conv.terms)
         launch_conv<CONV_FLOOR>(Tq, Tb, Z, B, B.floor_conv, qp, logn, fl, st);
     else
         with_group(out_group(B.bsk), [&](auto ob) {
             behz_floor_kernel<decltype(ob)::value><<<grid_for(fl), BT, lds, st>>>(Tq, Tb, Z, B, qp, logn, fl);
         });
     launch_check("behz_floor");
-    if (B.sk_conv.terms)
+    if (matrix && B.sk_conv.terms)
         launch_conv<CONV_SK>(Z, nullptr, out, B, B.sk_conv, qp, logn, fl, st);
     else
         with_group(out_group(B.L), [&](auto ob) {

@@ -236,6 +236,11 @@ def test_bfv_multiply(logn, bits, L, t, count):
     (8, [60] * 5, 4, 3),
     (9, [45, 50, 55, 60, 60, 48, 47, 46, 60], 8, 2),
     (8, [60] * 48, 47, 1),
+    # the lowest level on them, and the level that takes them for 2^17 coefficients at most
+    # and that for any number, past that line
+    (7, [34, 36, 40, 45, 50, 55, 60], 6, 3),
+    (12, [40, 45, 50, 55, 60, 60, 48, 47, 46, 60], 9, 33),
+    (12, [40, 45, 50, 55, 60, 60, 48, 47, 46, 60, 60], 10, 33),
     # past 48 terms, and 30-bit outputs: the vector unit
     (8, [60] * 49, 48, 1),
     (8, [30, 60, 60], 2, 2),
