@@ -17,11 +17,19 @@ __device__ __forceinline__ uint64_t moddown_prep(uint64_t s, uint64_t p, const D
     return submod(barrett64(v, Q.q, Q.ratio_hi), d.half_mod, Q.q);
 }
 
-// u_i of a ModDown at word (j, off) of its special limbs (15 floor(p/2) mod q_i < 2^64).
-__device__ __forceinline__ uint64_t moddown_u(const ModDownArgs &a, uint32_t i, uint64_t s, const DevPrime &Q) {
-    if (a.presum)  // uniform
-        return submod(barrett64(s, Q.q, Q.ratio_hi), barrett64(a.presum * a.dc[i].half_mod, Q.q, Q.ratio_hi), Q.q);
-    return moddown_prep(s, a.p, Q, a.dc[i]);
+// f(u) with u(i, s) = u_i of a ModDown at word s of its special limbs, for a limb of its own or a
+// sum of them (15 floor(p/2) mod q_i < 2^64).  The branch is one per block: inside a pass's load
+// it kept a thread's 16 loads from going out together (1,452 -> 1,695 us for 256 limbs of 2^16 to
+// 23 primes), inside its store the special limbs' (26.6 -> 29.8 us for 16 limbs of 2^17, BFV).
+template <class F>
+__device__ __forceinline__ void with_moddown_u(const ModDownArgs &a, const DevPrime *__restrict__ primes, const F &f) {
+    if (a.presum)
+        f([&](uint32_t i, uint64_t s) {
+            const DevPrime &Q = primes[i];
+            return submod(barrett64(s, Q.q, Q.ratio_hi), barrett64(a.presum * a.dc[i].half_mod, Q.q, Q.ratio_hi), Q.q);
+        });
+    else
+        f([&](uint32_t i, uint64_t s) { return moddown_prep(s, a.p, primes[i], a.dc[i]); });
 }
 
 // Word (limb i of polynomial j, coefficient off) of a ModDown's P.
@@ -42,27 +50,18 @@ __device__ __forceinline__ void moddown_add(const ModDownArgs &a, uint32_t i, ui
     else *dst = addmod(*dst, v, Q.q);
 }
 
-// Columns pass of u_i = the rounded special limb's residue, on load.  One branch per block
-// between a ModDown's own limb and a sum of them (15 floor(p/2) mod q_i < 2^64): inside the load
-// it kept a thread's 16 loads from going out together (1,452 -> 1,695 us for 256 limbs of 2^16 to
-// 23 primes).  Every prime reads the same special limb: i fastest keeps it in L2.
+// Columns pass of u_i = the rounded special limb's residue, on load.  Every prime reads the same
+// special limb: i fastest keeps it in L2.
 template <int LOGN, int K, int E, int SUBS>
 __device__ __forceinline__ void cols_moddown_prep(uint64_t *tile, uint32_t bid, uint64_t *__restrict__ U,
                                                   const DevPrime *__restrict__ primes, const ModDownArgs &a,
                                                   uint32_t jn) {
-    auto run = [&](const auto &of) {
+    with_moddown_u(a, primes, [&](const auto &u) {
         cols_body_t<LOGN, K, E, SUBS, false, true>(
             tile, bid, primes, 0, jn,
-            [&](uint32_t i, uint32_t j, size_t off) { return of(i, a.S[((size_t)j << LOGN) + off]); },
+            [&](uint32_t i, uint32_t j, size_t off) { return u(i, a.S[((size_t)j << LOGN) + off]); },
             [&](uint32_t i, uint32_t j, size_t off, uint64_t x) { U[((size_t)(j * a.L + i) << LOGN) + off] = x; }, a.L);
-    };
-    if (a.presum)
-        run([&](uint32_t i, uint64_t s) {
-            const DevPrime &Q = primes[i];
-            return submod(barrett64(s, Q.q, Q.ratio_hi), barrett64(a.presum * a.dc[i].half_mod, Q.q, Q.ratio_hi), Q.q);
-        });
-    else
-        run([&](uint32_t i, uint64_t s) { return moddown_prep(s, a.p, primes[i], a.dc[i]); });
+    });
 }
 
 template <int LOGN, int K, int E, int SUBS>
@@ -289,13 +288,16 @@ template <int LOGN, int K, int E, int SUBS>
 __global__ __launch_bounds__(SUBS << (K - E)) void ntt_cols_moddown_kernel(const uint64_t *__restrict__ Pt,
                                                                           const DevPrime *__restrict__ primes,
                                                                           ModDownArgs a, uint32_t jn) {
-    cols_body<LOGN, K, E, SUBS, true>(
-        blockIdx.x, primes, 0, jn, [&](uint32_t i, uint32_t j, size_t off) { return Pt[((size_t)(j * a.L + i) << LOGN) + off]; },
-        [&](uint32_t i, uint32_t j, size_t off, uint64_t x) {
-            const DevPrime &Q = primes[i];
-            const uint64_t u = moddown_u(a, i, a.S[((size_t)j << LOGN) + off], Q);
-            moddown_add<LOGN>(a, i, j, off, finish<true, true>(x, Q), u, Q);
-        });
+    __shared__ uint64_t tile[SUBS << K];
+    with_moddown_u(a, primes, [&](const auto &u) {
+        cols_body_t<LOGN, K, E, SUBS, true>(
+            tile, blockIdx.x, primes, 0, jn,
+            [&](uint32_t i, uint32_t j, size_t off) { return Pt[((size_t)(j * a.L + i) << LOGN) + off]; },
+            [&](uint32_t i, uint32_t j, size_t off, uint64_t x) {
+                const DevPrime &Q = primes[i];
+                moddown_add<LOGN>(a, i, j, off, finish<true, true>(x, Q), u(i, a.S[((size_t)j << LOGN) + off]), Q);
+            });
+    });
 }
 
 // Rows pass of an inverse transform of sigma(src).
