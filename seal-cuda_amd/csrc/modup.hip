@@ -36,6 +36,16 @@ __device__ __forceinline__ const void *uniform_ptr(const void *p) {
 // (31 * 8q^2 + q^2 < 2^128 for q < 2^60); beyond, R4 takes them below 4q first.
 // FP: the target's prime is below 2^50 -- T holds the columns pass's doubles, the last
 // layers run in fp64 and the sums are Acc26 of the transformed words' residues in [0, 4q).
+// AHEAD, for groups of 4, and of 2 up to N = 2^14: the row's own twiddles are staged once for all
+// steps, and a step's rows are requested while the step before runs its products, at three
+// waves per SIMD instead of four.  Groups of 4: 20.0 -> 18.5 ms for 128 ciphertexts at N = 2^16,
+// L = 24; 547 -> 434 us for 16 at N = 2^15, L = 15 in fp64.  Groups of 2 at N = 2^15 and 2^16 are
+// better off with the fourth wave, which the registers of both cost them (relinearizations of
+// two without / with, us: N = 2^16, L = 24 731 / 773, L = 8 124 / 129, N = 2^15, L = 15 169 / 184 and
+// in fp64 157 / 163; N = 2^14, L = 8 64.0 / 60.8 and 57.3 / 57.1), and a single ciphertext's short
+// launch too (274 -> 288 us with them).
+constexpr bool keyprod_ahead(int logn, int cg) { return cg == 4 || (cg == 2 && logn <= 14); }
+
 template <int LOGN, int K, int E, int SUBS, int CG, int RW, bool R4, bool FP>
 __device__ __forceinline__ void rows_keyprod_core(
     uint64_t *tile, ulonglong2 *tws, uint32_t i, int g0, uint32_t grp, const uint64_t *__restrict__ T, const uint64_t *__restrict__ key,
@@ -82,12 +92,7 @@ __device__ __forceinline__ void rows_keyprod_core(
     const uint64_t *trow = T + (((size_t)i * count * L + (size_t)(ct0 + min<uint32_t>(gg % CG, gv - 1)) * Lt) << LOGN) +
                            row_off(gg / CG);
     const uint32_t steps = (Lt + DJ - 1) / DJ;
-    // groups of 4 and 2: the row's own twiddles are staged once for all steps, and a step's
-    // rows are requested while the step before runs its products (20.0 -> 18.5 ms for 128
-    // ciphertexts at N = 2^16, L = 24; 547 -> 434 us for 16 at N = 2^15, L = 15 in fp64).  A
-    // single ciphertext's short launch does neither: the registers and LDS of both cost it
-    // its fourth wave per SIMD (274 -> 288 us with them)
-    constexpr bool AHEAD = CG > 1;
+    constexpr bool AHEAD = keyprod_ahead(LOGN, CG);
     using W2 = std::conditional_t<FP, double2, ulonglong2>;
     const W2 *tab;
     if constexpr (FP) tab = P.fwd_fp;
@@ -227,7 +232,7 @@ __device__ __forceinline__ void rows_keyprod_body(
     constexpr int GPL = (1 << (LOGN - K)) / RW;  // row groups per limb
     static_assert(GPL * RW == (1 << (LOGN - K)), "whole row groups");
     __shared__ uint64_t tile[SUBS * row_words(K)];
-    __shared__ ulonglong2 tws[CG > 1 ? 1 << K : 1];
+    __shared__ ulonglong2 tws[keyprod_ahead(LOGN, CG) ? 1 << K : 1];
     // bid & 7 is the XCD (launches, and groups of a grouped launch, start at multiples of 8)
     const uint32_t xcd = bid & 7, kk = bid >> 3;
     const uint32_t tl = (kk / groups) * 8 + xcd;
@@ -247,7 +252,7 @@ __device__ __forceinline__ void rows_keyprod_body(
 }
 
 template <int LOGN, int K, int E, int SUBS, int CG, int RW, bool R4, bool MIXED>
-__global__ __launch_bounds__(SUBS << (K - E), CG == 4 ? 3 : 4) void ntt_rows_keyprod_kernel(
+__global__ __launch_bounds__(SUBS << (K - E), keyprod_ahead(LOGN, CG) ? 3 : 4) void ntt_rows_keyprod_kernel(
     const uint64_t *__restrict__ T, const uint64_t *__restrict__ key, uint64_t *__restrict__ Pout,
     uint64_t *__restrict__ Sout, const DevPrime *__restrict__ primes, const uint64_t *__restrict__ diag,
     size_t diag_stride, uint32_t count, uint32_t L, uint32_t K_key, uint32_t ct_base, uint32_t groups,
@@ -277,7 +282,7 @@ struct KeyprodGroups {
     KeyprodGroup g[MAX_GROUPS];
 };
 template <int LOGN, int K, int E, int SUBS, int CG, int RW, bool R4, bool MIXED>
-__global__ __launch_bounds__(SUBS << (K - E), CG == 4 ? 3 : 4) void ntt_rows_keyprod_grouped_kernel(KeyprodGroups kg) {
+__global__ __launch_bounds__(SUBS << (K - E), keyprod_ahead(LOGN, CG) ? 3 : 4) void ntt_rows_keyprod_grouped_kernel(KeyprodGroups kg) {
     const uint32_t gi = group_of(kg.start, kg.n, blockIdx.x);
     const KeyprodGroup &a = kg.g[gi];
     rows_keyprod_body<LOGN, K, E, SUBS, CG, RW, R4, MIXED>(blockIdx.x - kg.start[gi], a.T, kg.key, a.P, a.S, a.primes,
@@ -341,7 +346,7 @@ __global__ __launch_bounds__(SUBS << (K - E)) void ntt_rows_modup_kernel(uint64_
 // chunk of targets, not once per target.  Large batches take all L + 1 targets per block
 // (measured 0.6 ms faster per 128 ciphertexts than one block per target); small ones
 // split the targets into chunks so that the grid still fills the GPU, down to one target
-// per block (ONE: nothing held in registers, 60 VGPRs instead of 132).
+// per block (ONE: no words held across targets, 97 VGPRs instead of 128).
 // skip_diag: limb (i, i) is not produced (its NTT is the NTT-form input limb) and the
 // targets i < L keep L - 1 limbs per ciphertext, T[i][ct][j - (j > i)].
 // MIXED: targets below 2^50 take the fp64 butterflies and leave doubles in T (their digits
@@ -452,9 +457,12 @@ struct ModupGroups {
     ModupGroup g[MAX_GROUPS];
 };
 
-// (held to 128 VGPRs: four waves per SIMD)
+// (held to 128 VGPRs, four waves per SIMD; the integer form over several targets, whose
+// groups' arguments would spill there, to three: 407 us spilled, 395 with its twiddles from
+// the table, for two groups of 2 at N = 2^16, L = 24 and 20; relinearizations of groups of 4
+// and 8 3,483 -> 3,425 us)
 template <int LOGN, int K, int E, int SUBS, bool ONE, bool MIXED>
-__global__ __launch_bounds__(SUBS << (K - E), 4) void ntt_cols_modup_grouped_kernel(ModupGroups mg) {
+__global__ __launch_bounds__(SUBS << (K - E), ONE || MIXED ? 4 : 3) void ntt_cols_modup_grouped_kernel(ModupGroups mg) {
     const uint32_t gi = group_of(mg.start, mg.n, blockIdx.x);
     const ModupGroup &a = mg.g[gi];
     cols_modup_body<LOGN, K, E, SUBS, ONE, MIXED>(blockIdx.x - mg.start[gi], a.d, a.d_ct_stride, a.T, a.targets, mg.digits,
@@ -471,6 +479,12 @@ inline uint32_t modup_targets_per_block(uint32_t tile_blocks, uint32_t L, uint32
     return (L + chunks) / chunks;  // ceil((L + 1) / chunks)
 }
 
+// log2 of the values per thread of the ModUp columns pass: 8 where targets take the fp64
+// butterflies, whose pass waits more than it issues (289 -> 271 us for 16 ciphertexts at
+// N = 2^15, L = 15 against 16 values), 16 for integer ones (13.5 ms for 128 at N = 2^16,
+// L = 24 against 13.9 with 8, 16.6 with 4).
+constexpr int modup_cols_log(bool mixed) { return mixed ? 3 : 4; }
+
 template <int LOGN, bool SMALL>
 void launch_modup_as(const uint64_t *d, size_t d_stride, uint64_t *T, uint32_t cts, uint32_t L, const DevPrime *targets,
                   const DevPrime *digits, bool skip_diag, bool reduce_4q, bool mixed, const KernelProbe *probe,
@@ -481,11 +495,12 @@ void launch_modup_as(const uint64_t *d, size_t d_stride, uint64_t *T, uint32_t c
     const uint32_t col_grid = cts * L * ((L + tc) / tc) * ((1u << K2) / CS);
     with_bool(mixed, [&](auto mx) {
         constexpr bool MIXED = decltype(mx)::value;
+        constexpr int EC = SMALL ? E : modup_cols_log(MIXED);
         if (tc == 1)
-            ntt_cols_modup_kernel<LOGN, K1, E, CS, true, MIXED><<<col_grid, CS << (K1 - E), 0, st>>>(
+            ntt_cols_modup_kernel<LOGN, K1, EC, CS, true, MIXED><<<col_grid, CS << (K1 - EC), 0, st>>>(
                 d, d_stride, T, targets, digits, cts, L, skip_diag, tc);
         else
-            ntt_cols_modup_kernel<LOGN, K1, E, CS, false, MIXED><<<col_grid, CS << (K1 - E), 0, st>>>(
+            ntt_cols_modup_kernel<LOGN, K1, EC, CS, false, MIXED><<<col_grid, CS << (K1 - EC), 0, st>>>(
                 d, d_stride, T, targets, digits, cts, L, skip_diag, tc);
     });
     const LimbGrid lg{cts * L, 1, L + 1, cts * L};
@@ -539,12 +554,6 @@ void launch_keyprod_groups(const uint64_t *T, const uint64_t *key, uint64_t *P, 
             T, key, P, S, targets, diag, diag_stride, cts, L, K_key, cts - singles, singles, tiles2, fold);
     }
 }
-
-// log2 of the values per thread of the ModUp columns pass: 8 where targets take the fp64
-// butterflies, whose pass waits more than it issues (289 -> 271 us for 16 ciphertexts at
-// N = 2^15, L = 15 against 16 values), 16 for integer ones (13.5 ms for 128 at N = 2^16,
-// L = 24 against 13.9 with 8, 16.6 with 4).
-constexpr int modup_cols_log(bool mixed) { return mixed ? 3 : 4; }
 
 template <int LOGN>
 void launch_modup_keyprod(const uint64_t *d, size_t d_stride, uint64_t *T, const uint64_t *key, uint64_t *P,
