@@ -42,8 +42,6 @@ inline uint32_t blocks_for(size_t n) {
     return (uint32_t)(b < (size_t(1) << 20) ? b : (size_t(1) << 20));
 }
 
-inline size_t align256(size_t bytes) { return (bytes + 255) & ~size_t(255); }
-
 // neg[l][k] = 1 where sigma_elt negates the coefficient that lands at k (the source
 // i = k elt^-1 mod N moves to i elt mod 2N, negated when that is >= N), in each limb.
 __global__ void negated_positions_kernel(uint64_t *__restrict__ neg, uint32_t elt, uint32_t elt_inv, int logn,
@@ -734,14 +732,20 @@ void rotate_accumulate(const Context &c, const uint64_t *in, uint32_t count, uin
     const bool ckks = c.scheme == SCHEME_CKKS;
     const int logn = c.logn;
     if (!lay.batched) {
-        uint64_t *tmp = at(lay.tmp);
-        char *gws = base + align256(step * 8);
+        // (sigma(c0), 0) joins the sum, and the switch of sigma(c1) adds into it
+        uint64_t *sigma = at(lay.d), *C0 = at(lay.C0);
         for (uint32_t h = 0; h < n; h++) {
-            uint64_t *dst = h ? tmp : out;
-            SHC_HIP(hipMemcpyAsync(dst, in + h * step, step * 8, hipMemcpyDeviceToDevice, st));
-            if (elts[h] != 1)
-                apply_galois_keyswitch(c, dst, count, L, elts[h], keys[h], gws, ws_bytes - (gws - base), st);
-            if (h) poly_add(c, out, tmp, out, count * 2, L, st);
+            const uint64_t *x = in + h * step;
+            if (elts[h] == 1) {
+                if (h) poly_add(c, out, x, out, count * 2, L, st);
+                else SHC_HIP(hipMemcpyAsync(out, x, step * 8, hipMemcpyDeviceToDevice, st));
+                continue;
+            }
+            apply_galois(c, x + lw, ctw, sigma, lw, count, L, elts[h], ckks, st);
+            apply_galois(c, x, ctw, C0, lw, count, L, elts[h], ckks, st);
+            accumulate_c0_kernel<<<blocks_for(count * lw), TPB, 0, st>>>(out, C0, c.primes(), L, logn, h == 0, count * lw);
+            launch_check("accumulate_c0");
+            switch_key(c, sigma, lw, out, ctw, keys[h], count, L, base + lay.ks, lay.total - lay.ks, st);
         }
         return;
     }

@@ -88,12 +88,14 @@ inline RotLayout rot_layout(int logn, uint32_t count, uint32_t L) {
 }
 
 // Sums of rotations of different ciphertexts (rotate_accumulate): batches of nb rotations, or one
-// at a time (tmp: the rotated ciphertext, then a Galois switch's workspace) below N = 2^13 and
-// where one rotation's T is more than a launch.  N = 2^15, 2^16: the fused key products take
+// at a time (d: sigma(c1); C0: sigma(c0); a key switch's workspace) below N = 2^13 and where one
+// rotation's T is more than a launch.  N = 2^15, 2^16: the fused key products take
 // one rotation's T at a time; other degrees a batch's.
 struct AccLayout {
     bool batched;
-    size_t d, T, P, S, Psum, V, U, tmp, total;
+    size_t d, T, P, S, Psum, V, U;  // batched
+    size_t C0, ks;                  // one at a time, beside d
+    size_t total;
 };
 inline bool acc_fused(int logn) { return logn == 15 || logn == 16; }
 inline bool acc_batched(int logn, uint32_t count, uint32_t L) {
@@ -103,8 +105,8 @@ inline AccLayout acc_layout(int logn, uint32_t count, uint32_t L, uint32_t nb) {
     WorkspaceRegions r(logn, count);
     AccLayout l{};
     l.batched = acc_batched(logn, count, L);
+    l.d = r.limbs((size_t)(l.batched ? nb : 1) * L);
     if (l.batched) {
-        l.d = r.limbs((size_t)nb * L);
         l.T = r.limbs((acc_fused(logn) ? 1 : nb) * (size_t)L * (L + 1));
         l.P = r.limbs((size_t)nb * 2 * L);
         l.S = r.limbs((size_t)nb * 2);
@@ -112,9 +114,8 @@ inline AccLayout acc_layout(int logn, uint32_t count, uint32_t L, uint32_t nb) {
         l.V = r.limbs(2);
         l.U = r.limbs(2 * (size_t)L);
     } else {
-        l.tmp = r.limbs(2 * (size_t)L);
-        r.limbs(L);
-        r.bytes(ks_layout(logn, count, L).total);
+        l.C0 = r.limbs(L);
+        l.ks = r.bytes(ks_layout(logn, count, L).total);
     }
     l.total = r.off;
     return l;

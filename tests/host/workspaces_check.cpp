@@ -55,7 +55,10 @@ static bool check(int logn, uint32_t L, uint32_t count) {
     if (r.total > hoisted) return std::printf("hoisted rotations ask for more\n"), false;
     for (uint32_t nb = 1; nb <= ROT_MAX; nb++) {
         const AccLayout a = acc_layout(logn, count, L, nb);
-        if (!a.batched) continue;
+        if (!a.batched) {
+            if (!apart({{a.d, L * limb}, {a.C0, L * limb}, {a.ks, k.total}}, a.total)) return false;
+            continue;
+        }
         if (!apart({{a.d, nb * L * limb}, {a.T, (acc_fused(logn) ? 1 : nb) * per * limb}, {a.P, nb * 2 * L * limb},
                     {a.S, nb * 2 * limb}, {a.Psum, 2 * L * limb}, {a.V, 2 * limb}, {a.U, 2 * L * limb}}, a.total))
             return false;

@@ -123,6 +123,9 @@ def test_rotation_passes_zero_digits(scheme, zeros):
 
 @pytest.mark.parametrize("scheme,logn,bits,L,count,steps", [
     (CKKS, 12, [60, 40, 40, 60], 3, 2, [None, 1, -2]),                  # one at a time
+    (CKKS, 11, [60, 40, 60], 2, 3, [1, None, 2, None]),
+    (BFV, 12, [40, 40, 50], 2, 2, [0, 1, None]),
+    (BFV, 10, [40, 50], 1, 1, [None, 3]),
     (CKKS, 13, [60, 40, 50, 60], 3, 3, [None] + list(range(1, 18))),    # two summed ModDowns
     (BFV, 13, [43, 44, 44], 2, 5, [1, 2, None, 3, 0, 4, 5]),            # batches around the identity
     (BFV, 14, [60, 50, 60], 2, 1, [None]),
