@@ -71,6 +71,7 @@ void launch_ntt_as(uint64_t *data, LimbGrid lg, uint32_t j0, uint32_t jn, const 
 // prime at N = 2^16: 2^22 words 38.0 / 36.9, 2^23 63.0 / 64.8, 2^24 113 / 123, 2^26 (62.5 M) 464 /
 // 552; N = 2^13, L = 4: 2^23 58.9 / 57.3, 2^24 102.7 / 107.3.  Inverse, N = 2^16: 2^23 69.4 /
 // 65.7, 2^24 121.6 / 126.6, 62.5 M 512 / 554; N = 2^13: 2^24 111.5 / 107.7, 2^25 220 / 224.
+// (Polynomials count in fours, a block's rows: 5 at N = 2^16, L = 24 68.7 / 74.3.)
 constexpr uint64_t NTT_SMALL_WORDS = (uint64_t(1) << 23) - 1;
 constexpr uint64_t INTT_SMALL_WORDS = (uint64_t(1) << 24) - 1;
 
@@ -79,7 +80,7 @@ void launch_ntt(uint64_t *data, LimbGrid lg, uint32_t j0, uint32_t jn, const Dev
     if constexpr (LOGN <= 12)
         launch_ntt_as<LOGN, INV, FULL, false>(data, lg, j0, jn, primes, st);
     else
-        with_shape<LOGN>((uint64_t)lg.I * jn, [&](auto s) {
+        with_shape<LOGN>((uint64_t)lg.I * (jn < 4 ? jn : (jn + 3) & ~3u), [&](auto s) {
             launch_ntt_as<LOGN, INV, FULL, decltype(s)::value>(data, lg, j0, jn, primes, st);
         }, INV ? INTT_SMALL_WORDS : NTT_SMALL_WORDS);
 }

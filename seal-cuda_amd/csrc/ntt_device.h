@@ -229,16 +229,19 @@ __device__ __forceinline__ uint64_t finish(uint64_t x, const DevPrime &P) {
 // row in the block uses the same twiddles (broadcast loads, L1/L2 hits).  Blocks run
 // with the limb group fastest, so consecutive blocks also share them.  jn_short != 0:
 // primes i < I - 1 have only jn_short limbs (the grid is sized for jn).
-// MX (fewer than SUBS limbs per prime, e.g. one ciphertext): a block takes SUBS
-// (limb, row) pairs of prime i instead, limb fastest, so that its threads are not idle;
-// the rows of a block then differ and so do their twiddles.
+// MX (fewer than SUBS limbs per prime, e.g. one ciphertext, or 5 for blocks of 4): a block
+// takes SUBS (limb, row) pairs of prime i instead, limb fastest, so that its threads are not
+// idle; the rows of a block then differ and so do their twiddles, which costs more than a
+// second block with two rows or more of its four (forward transforms of 5 and 7 polynomials at
+// N = 2^16, L = 12: 42.9 -> 38.6 us and 2% more; 5 at N = 2^15, L = 15 30.5 -> 27.7; 9 for blocks of
+// 8 at N = 2^13, L = 4 2% more).
 template <int LOGN, int K, int E, int SUBS>
 __host__ __device__ constexpr uint32_t rows_blocks_per_prime(uint32_t jn, bool mx) {
     return mx ? ((jn << (LOGN - K)) + SUBS - 1) / SUBS : (1u << (LOGN - K)) * ((jn + SUBS - 1) / SUBS);
 }
 template <int LOGN, int K, int SUBS>
 __host__ __device__ constexpr bool rows_mixed(uint32_t jn) {
-    return LOGN > K && jn < (uint32_t)SUBS;
+    return LOGN > K && (jn < (uint32_t)SUBS || (SUBS == 4 && jn == 5));
 }
 
 // (tile: SUBS * row_words(K) words of LDS, the caller's)

@@ -34,6 +34,14 @@ def test_ntt_all_degrees(logn):
     check_ntt(logn, bits, polys=3, seed=logn)
 
 
+@pytest.mark.parametrize("polys", [4, 5, 6, 8, 9])
+@pytest.mark.parametrize("logn", [13, 15, 16])
+def test_ntt_ragged_rows(logn, polys):
+    """Around a block's rows (4 at N = 2^15 and 2^16, 8 at 2^13): full blocks, a last one with some,
+    and blocks of (limb, row) pairs."""
+    check_ntt(logn, [60, 40], polys=polys, seed=logn + polys)
+
+
 def test_ntt_kat():
     # test/utils/ntt.cpp:75-99 on the GPU path
     ctx = hip().Context(hip().SCHEME_CKKS, 2, [0xFFFFFFFFFFC0001])
