@@ -13,6 +13,7 @@
 // (level, batch) read.  The candidates include the built-in choice, and another shape
 // replaces it only when it is more than 1% faster on the tuning run.
 #include "autotune.h"
+#include "launch_limits.h"
 #include "rns_ops.h"
 #include <algorithm>
 #include <cstdio>
@@ -45,17 +46,18 @@ void set_shape(const Context &c, uint32_t L, uint32_t count, const KsShape *s) {
 
 }  // namespace
 
-std::vector<KsShape> keyswitch_candidates(const Context &c, uint32_t L) {
+std::vector<KsShape> keyswitch_candidates(const Context &c, uint32_t L, uint32_t count) {
     std::vector<uint32_t> targets;
     for (uint32_t chunks : {1u, 2u, 3u, 4u, 6u, 8u, 12u, 16u, L + 1}) {
         if (chunks > L + 1) continue;
         const uint32_t tc = (L + chunks) / chunks;  // ceil((L + 1) / chunks)
         if (std::find(targets.begin(), targets.end(), tc) == targets.end()) targets.push_back(tc);
     }
-    const bool fused = c.logn >= 13 && c.logn <= 16;
+    uint32_t groups[3] = {0}, n_groups = 1;  // of the fused kernel, each split of the batch once
+    if (c.logn >= 13 && c.logn <= 16) n_groups = distinct_groups(c.logn, count, groups);
     std::vector<KsShape> out{KsShape{}};  // the built-in choice first
-    for (uint32_t g : fused ? std::vector<uint32_t>{4, 2, 1} : std::vector<uint32_t>{0})
-        for (uint32_t tc : targets) out.push_back(KsShape{tc, g});
+    for (uint32_t g = 0; g < n_groups; g++)
+        for (uint32_t tc : targets) out.push_back(KsShape{tc, groups[g]});
     return out;
 }
 
@@ -80,7 +82,7 @@ TuneResult autotune_relinearize(const Context &c, uint64_t *ct, const uint64_t *
         return ms / reps;
     };
     try {
-        for (const KsShape &s : keyswitch_candidates(c, L)) {
+        for (const KsShape &s : keyswitch_candidates(c, L, count)) {
             const float ms = time_shape(s);
             r.tried++;
             if (!s.cols_targets && !s.rows_group) r.builtin_ms = ms;

@@ -14,7 +14,7 @@ struct TuneResult {
 
 // The shapes the tuner tries at level L: the built-in choice, then every
 // (targets per columns block, ciphertexts per rows block) pair.
-std::vector<KsShape> keyswitch_candidates(const Context &c, uint32_t L);
+std::vector<KsShape> keyswitch_candidates(const Context &c, uint32_t L, uint32_t count);
 
 // Times `reps` relinearizations of ct [count][3][L][N] (used as scratch: its words are
 // overwritten) per candidate shape and keeps the fastest in c's table for (L, count).

@@ -25,6 +25,22 @@ inline GroupSplit split_groups(int logn, uint32_t cts, uint32_t group) {
     return GroupSplit{g4, g2, rest - 2 * g2};
 }
 
+// The group sizes among 4, 2 and 1 that split cts ciphertexts differently, the largest first;
+// returns how many (out: room for 3).
+inline uint32_t distinct_groups(int logn, uint32_t cts, uint32_t *out) {
+    uint32_t n = 0;
+    for (uint32_t g : {4u, 2u, 1u}) {
+        const GroupSplit s = split_groups(logn, cts, g);
+        bool known = false;
+        for (uint32_t k = 0; k < n; k++) {
+            const GroupSplit o = split_groups(logn, cts, out[k]);
+            known |= o.g4 == s.g4 && o.g2 == s.g2 && o.singles == s.singles;
+        }
+        if (!known) out[n++] = g;
+    }
+    return n;
+}
+
 // Blocks per group of the fused key products at level L: one per row of every target prime (a
 // single ciphertext's blocks take two rows), a multiple of the 8 XCDs.
 inline uint64_t keyprod_slots(int logn, uint32_t L, bool single) {

@@ -437,11 +437,13 @@ void switch_key_chunk(const Context &c, const uint64_t *target, size_t target_st
     // that the ModDown writes it without reading it)
     const KsShape shape = c.ks_shape(L, count);
     const KsFold fold = ckks ? KsFold{fold_c0 ? fold_c0 : ct, ct_stride, c.ks_consts(), fold_c0 != nullptr} : KsFold{};
-    // (a single ciphertext at N = 2^13 leaves the fused kernel 16 blocks per prime to wait
-    // in: 54.7 us per product at L = 3 in two kernels, 55.8 in one)
-    const bool fused = (logn > 13 || count > 1 || fold_c0) && ntt_modup_keyprod(digits, dstride, T, key, P, S, diag, target_stride, count, L,
-                                         (uint32_t)c.key_count(), c.keyswitch_primes(L), c.primes(), logn,
-                                         c.fp_primes, st, probe, shape, fold);
+    // (unless a shape asks for the fused form, one ciphertext at N = 2^13 takes two kernels: its 16
+    // blocks per prime wait in the fused one.  Fused / two kernels in us, CKKS and BFV alike: L = 1
+    // 35.8 / 32.7, 2 36.8 / 33.4, 3 36.4 / 34.2, 4 36.5 / 35.4, 6 38.4 / 38.0, 8 42.0 / 43.8, 12 56.0 / 51.7)
+    const bool fuse = logn > 13 || count > 1 || shape.rows_group || fold_c0;
+    const bool fused = fuse && ntt_modup_keyprod(digits, dstride, T, key, P, S, diag, target_stride, count, L,
+                                                 (uint32_t)c.key_count(), c.keyswitch_primes(L), c.primes(), logn,
+                                                 c.fp_primes, st, probe, shape, fold);
     if (fold_c0 && !fused) fail(ERR_LOGIC, "a key switch into (c0, 0) needs the fused key products");
     if (!fused) {
         const bool skipped = modup_to_T(c, digits, dstride, T, count, L, st, probe, diag != nullptr);

@@ -1,5 +1,6 @@
 // Host check of seal-cuda_amd/csrc/launch_limits.h: a batch's groups cover its ciphertexts once
-// and in order of size, and a grouped relinearization is taken exactly when the blocks of
+// and in order of size, the autotuner's group sizes all split it differently, and a grouped
+// relinearization is taken exactly when the blocks of
 // each launch, counted here from the kernels' grids, stay below the limit of a grouped launch.
 // Prints "ok <cases>" and exits 0, or prints the first failing case and exits 1.
 #include "launch_limits.h"
@@ -36,6 +37,14 @@ int main() {
                 if (slots < cts || slots > cts + 3 || (logn >= 15 && slots != cts))
                     return std::printf("split of %u at 2^%d by %u\n", cts, logn, group), 1;
             }
+        // one ciphertext splits one way, two two ways (4 splits like 2), others by all three
+        for (uint32_t cts = 1; cts < 70; cts++, cases++) {
+            uint32_t g[3] = {};
+            const uint32_t ways = shc::distinct_groups(logn, cts, g);
+            const uint32_t want = cts == 1 ? 1 : cts == 2 || (cts == 3 && logn >= 15) ? 2 : 3;
+            if (ways != want || g[0] != 4 || (ways > 1 && g[ways - 1] != 1))
+                return std::printf("splits of %u at 2^%d\n", cts, logn), 1;
+        }
         for (uint32_t L : {1u, 2u, 3u, 7u, 24u})
             for (uint32_t groups : {1u, 2u, 16u})
                 for (uint32_t base = 1; base < (1u << 20); base = base * 3 / 2 + 1)

@@ -32,7 +32,11 @@ def relin(ctx, ct3, key, count, L):
 @pytest.mark.parametrize("scheme,logn,bits,count", [
     (CKKS, 15, [60] + [40] * 6 + [60], 7),     # fused path: groups 4 + 2 + 1, 2 x 3 + 1, 7 singles
     (BFV, 15, [60] * 5, 5),
-    (CKKS, 13, [60, 40, 40, 40, 60], 3),       # unfused path: only the columns-pass choice
+    (CKKS, 13, [60, 40, 40, 40, 60], 3),
+    (CKKS, 13, [60, 40, 50, 60], 5),           # small rings: 4 + a short 4, 2 x 2 + 1, 5 singles
+    (BFV, 13, [43, 44, 60], 1),                # one ciphertext: two kernels unless a group is set
+    (BFV, 14, [60, 50, 60], 3),
+    (CKKS, 17, [60, 40, 60], 2),               # unfused path: only the columns-pass choice
 ])
 def test_every_candidate_shape_gives_the_same_words(scheme, logn, bits, count):
     n = 1 << logn
@@ -48,7 +52,7 @@ def test_every_candidate_shape_gives_the_same_words(scheme, logn, bits, count):
     np.testing.assert_array_equal(base[count - 1], ck.relinearize(scheme, ct3[count - 1], key_h, moduli, L, logn))
     chunks = (1, 2, 3, 4, 6, 8, 12, 16, L + 1)
     targets = sorted({(L + c) // c for c in chunks if c <= L + 1})
-    groups = (4, 2, 1) if logn in (15, 16) else (0,)
+    groups = (4, 2, 1) if 13 <= logn <= 16 else (0,)
     for g in groups:
         for tc in targets:
             assert ctx.keyswitch_shape(L, count, (tc, g)) == (tc, g)
