@@ -5,7 +5,8 @@ the sign-pattern correction) must give the words of summing (or listing) separat
 applyGaloisInplace restatement, itself pinned against the reference -- for CKKS (NTT
 form) and BFV (coefficient form), for positive, negative and conjugation elements, and
 when c1 has zero digits (fixed on the device), is entirely zero, or has many zeros; and a
-captured HIP graph of the call replays to the same words.
+captured HIP graph of the call replays to the same words.  shc_rotate_accumulate likewise
+must give the words of separate rotations summed, in every workspace that holds one.
 """
 import numpy as np
 import torch
@@ -132,6 +133,10 @@ def test_rotation_passes_zero_digits(scheme, zeros):
     (CKKS, 15, [60, 40, 50, 60], 3, 5, [None, 2, 4, 6, 8, 10]),         # the fused key products
     (CKKS, 15, [60, 60], 1, 1, [3]),
     (BFV, 15, [60, 50, 60], 2, 2, [1, 0]),
+    (CKKS, 16, [60, 40, 60], 2, 3, [None, 1, 2, 3]),
+    (BFV, 16, [60, 60], 1, 1, [1, None]),
+    (CKKS, 17, [60, 50, 60], 2, 1, [1, 2, None, 3, 4, 5]),              # several keys, unfused
+    (BFV, 17, [60, 60], 1, 2, [2, 1]),
 ])
 def test_rotate_accumulate(scheme, logn, bits, L, count, steps):
     accumulate_case(scheme, logn, bits, L, count, steps)
@@ -147,6 +152,50 @@ def test_rotate_accumulate_in_smaller_workspaces(scheme, logn, bits, count):
         T = 6 * (1 if logn in (15, 16) else nb)
         accumulate_case(scheme, logn, bits, L, count, [1, 2, None, 3, 4, 5],
                         (T + nb * (3 * L + 2) + 4 * L + 2) * count * n * 8, refused=nb == 1)
+
+
+@pytest.mark.parametrize("scheme,logn,count", [(CKKS, 13, 1040), (BFV, 13, 1040), (CKKS, 15, 264)])
+def test_rotation_launch_forms_agree(scheme, logn, count):
+    """Batches whose permuted inverse transforms and permuted ModDowns pass 2^26 words (16 values
+    per thread) against the same ciphertexts in slices below (4 values), which the oracle
+    checks above."""
+    L, n = 2, 1 << logn
+    moduli = ck.coeff_modulus_create(n, [60, 40, 60])
+    ctx = hip().Context(scheme, n, moduli, 65537 if scheme == BFV else 0)
+    gen = torch.Generator(device="cuda").manual_seed(logn)
+    x = torch.empty((4, count, 2, L, n), dtype=torch.int64, device="cuda")
+    for i in range(L):
+        x[..., i, :] = torch.randint(0, moduli[i], (4, count, 2, n), generator=gen, device="cuda", dtype=torch.int64)
+    rng = np.random.default_rng(logn)
+    elts = [ck.galois_elt(logn, s) for s in (1, 2, -1, 3)]
+    keys = [to_dev(ck.random_key(rng, moduli, logn)) for _ in elts]
+    hb, hw = ctx.hoisted_key_size(L), ctx.hoisted_key_workspace_size(L)
+    hws, hoisted = ws(hw), []
+    for e, k in zip(elts, keys):
+        hoisted.append(empty_dev(((hb + 7) // 8,)))
+        ctx.hoisted_key_prepare(k.data_ptr(), e, L, hoisted[-1].data_ptr(), hws.data_ptr(), hw, stream())
+    kp, hp = [k.data_ptr() for k in keys], [h.data_ptr() for h in hoisted]
+
+    def run(x):
+        m = x.shape[1]
+        # room for four rotations at a time in both
+        wb = max(ctx.rotate_sum_workspace_size(m, L), (24 + 4 * (3 * L + 2) + 4 * L + 2) * m * n * 8)
+        buf = ws(wb)
+        many, one, acc = empty_dev((4, m, 2, L, n)), empty_dev((m, 2, L, n)), empty_dev((m, 2, L, n))
+        ctx.rotate_many(x.data_ptr(), m, L, elts, hp, kp, many.data_ptr(), buf.data_ptr(), wb, stream())
+        ctx.rotate_sum(x.data_ptr(), m, L, elts, hp, kp, one.data_ptr(), buf.data_ptr(), wb, stream())
+        ctx.rotate_accumulate(x.data_ptr(), m, L, elts, kp, acc.data_ptr(), buf.data_ptr(), wb, stream())
+        torch.cuda.synchronize()
+        return many, one, acc
+
+    assert 4 * 2 * count * n > 1 << 26       # the special limbs of a pass
+    assert 4 * count * L * n > 1 << 26       # the digits of a batch
+    many, one, acc = run(x)
+    step = count // 8 + 1
+    for c in range(0, count, step):
+        sl = slice(c, min(c + step, count))
+        m, o, a = run(x[:, sl].contiguous())
+        assert torch.equal(many[:, sl], m) and torch.equal(one[sl], o) and torch.equal(acc[sl], a)
 
 
 def test_rotate_accumulate_rejects():
