@@ -118,8 +118,9 @@ __host__ __device__ __forceinline__ u128 acc_value(const Acc26 &a) {
     const uint32_t hi = (uint32_t)a2 << 20 | ((uint32_t)a1 >> 6 & 0xfffffu);
     return u128{(uint64_t)hi << 32 | lo, a2 >> 12};
 }
-// The value mod q for q of b bits, 2 < b <= 50, and values below 2^(b + 60) (over 500 products
-// of t < 4q and k < q).  One quotient estimate: with t = value >> (b - 2) < 2^62 and
+// The value mod q for q of b bits, 2 < b <= 50, and values below 2^(b + 60): 2^(58 - b) products
+// of t < 4q and k < q, 256 at b = 50 (key switches and rotations sum at most 63 and two terms
+// more, plain products fold every 64 of t < q).  One quotient estimate: with t = value >> (b - 2) < 2^62 and
 // ratio = floor(2^(b + 62) / q) < 2^63, mulhi64_approx(t, ratio) is short by less than
 // 1/2 (t) + 1/4 (ratio) + 1 (floor) + 2 (approx), so the remainder lies in [0, 4q).  About
 // 55 instructions with the sum's own against 95 for a 128-bit quotient: plain_dot_tiles 4.86 ->

@@ -12,7 +12,9 @@
 //   * for q < 2^50, the fp64 forms (butterfly_fp.h): products and butterflies congruent and
 //     within the bound each layer states for operands at the ends of the passes' ranges,
 //     the passes' schedules within 8q and the ranges they hand over, the conversions, and
-//     the 26-bit product sums (accum.h) over 64 terms;
+//     the 26-bit product sums (accum.h) and their remainders: 64 terms t < 4q, k < q, and as
+//     many as stay below the remainder's bound of 2^(b + 60) for q of b bits, up to 512, with
+//     every operand at its end or random within 2^10 of it;
 // for primes from 17 to 61 bits, random and extreme operands (0, range ends,
 // multiples of q +- 1, all-ones words).  Exact products come from unsigned __int128.
 // Prints "ok <cases>" and exits 0, or prints the first failing case and exits 1.
@@ -140,13 +142,17 @@ static bool check_fp(u64 q, long &cases) {
         if (shc::fp_to_u52(x, up) != (u64)((int64_t)x + (int64_t)(2 * q))) return std::printf("fp_to_u52\n"), false;
     }
     const wide r = ~(wide)0 / q;  // floor(2^128 / q), q not a power of 2
+    const int bits = 64 - __builtin_clzll(q);
+    const int most = bits >= 50 ? 256 : 512;  // t k < 2^(2 b + 2)
     for (int ext = 0; ext < 64; ext++) {
         shc::Acc26 a{0, 0, 0};
         wide sum = 0;
-        for (int k = 0; k < (ext == 1 ? 512 : 64); k++) {
-            if (ext > 1 && shc::acc_reduce26(a, q, (u64)r, (u64)(r >> 64)) != (u64)(sum % q))
+        const bool ends = ext >= 1 && ext < 8;
+        for (int k = 0; k < (ends ? most : 64); k++) {
+            if (ext > 0 && shc::acc_reduce26(a, q, (u64)r, (u64)(r >> 64)) != (u64)(sum % q))
                 return std::printf("acc_reduce26 q=%llu\n", (unsigned long long)q), false;
-            const u64 t = ext == 1 ? 4 * q - 1 : next() % (4 * q), f = ext == 1 ? q - 1 : next() % q;
+            const u64 t = ext == 1 ? 4 * q - 1 : ends ? 4 * q - 1 - next() % 1024 : next() % (4 * q);
+            const u64 f = ext == 1 ? q - 1 : ends ? q - 1 - next() % 1024 : next() % q;
             shc::mac(a, shc::cut26(t), shc::cut26(f));
             sum += (wide)t * f;
         }
