@@ -26,8 +26,11 @@ N=8192), batches of 128.
 
 `--workload copy`: a 1 GiB device copy, the calibration run for HBM byte counters.
 
-Prints one JSON line.  Data are seeded uniform residues (synthetic) and injected
-uniform key words; every word is fully reduced.
+Prints one JSON line of at most LINE_LIMIT characters (a log's tail holds it whole): the
+headline with its roofline and baselines, and value and unit of each other workload.  The
+whole result, with every workload's roofline, baseline and shape, goes to stderr (`--full`:
+to stdout instead).  Data are seeded uniform residues (synthetic) and injected uniform key
+words; every word is fully reduced.
 """
 import argparse
 import json
@@ -74,6 +77,7 @@ def parse():
     p.add_argument("--headline-only", action="store_true",
                    help="mulrelin: skip the other workloads' sub-objects in the JSON line")
     p.add_argument("--sub-steps", type=int, default=5, help="timed steps of each sub-workload in the default line")
+    p.add_argument("--full", action="store_true", help="print the whole result on stdout instead of the short line")
     p.add_argument("--no-tune", action="store_true", help="keep the built-in key-switch launch shapes")
     return p.parse_args()
 
@@ -374,7 +378,7 @@ def bench_mulrelin(args):
                      "frac": achieved_rows / HBM_PEAK_GBS,
                      "traffic": KEYPROD_TRAFFIC_B128 if valu_known else None,
                      "butterflies_per_launch": rows_bfly, "macs_per_launch": rows_macs,
-                     "kernel": f"ntt_rows_keyprod_kernel<16,8,4,16,{kname},false>: key-switch ModUp NTT rows pass over "
+                     "kernel": f"ntt_rows_keyprod_kernel<16,8,4,16,{kname},false,false>: key-switch ModUp NTT rows pass over "
                                f"{tlimbs} limbs (last {logn - logn // 2} layers) fused with the key products",
                      "algorithmic_bytes": rows_bytes, "avg_ms": rows_ms,
                      "butterflies_per_s": rows_bfly / (rows_ms * 1e-3),
@@ -1897,6 +1901,41 @@ def bench_copy(args):
             "config": {"workload": "device copy of 2^27 int64 words", "parallelism": "single GPU"}}
 
 
+LINE_LIMIT = 1800
+LINE_KEYS = ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling",
+             "vs_baseline", "dtype", "data", "config", "roofline", "cpu_baseline", "batched_over_plain",
+             "served_latency", "configs")
+
+
+def short_line(out):
+    """The printed line of a result: its contract keys; of the roofline, the CPU baseline and the
+    served latency their figures; of every other workload "value unit" (or its error)."""
+    def digits(v):
+        return float(f"{v:.5g}") if isinstance(v, float) else v
+
+    def only(d, keys):
+        return {k: digits(d[k]) for k in keys if d.get(k) is not None}
+
+    line = {k: out[k] if k in ("value", "ms_per_step") else digits(out[k]) for k in LINE_KEYS if k in out}
+    for k, keys in (("roofline", ("bound", "achieved", "peak", "unit", "frac", "avg_ms")),
+                    ("cpu_baseline", ("value", "unit", "cores", "kind"))):
+        if line.get(k):
+            line[k] = only(line[k], keys)
+    served = line.pop("served_latency", None)
+    if served:
+        line["served_ms"] = {k: only(v, ("p50", "p99", "p50_ms", "p99_ms")) for k, v in served.items()
+                             if isinstance(v, dict) and any(q.startswith("p50") for q in v)}
+    if "configs" in out:
+        line["configs"] = {k: f"{d['value']:.5g} {d['unit']}" if d.get("value") is not None else
+                           str(d.get("error", ""))[:60] for k, d in out["configs"].items()}
+    # what a longer line drops first
+    for k in ("served_ms", "cpu_baseline", "configs", "roofline"):
+        if len(json.dumps(line)) <= LINE_LIMIT:
+            break
+        line.pop(k, None)
+    return line
+
+
 def main():
     args = parse()
     if args.gpus != 1:
@@ -1906,6 +1945,9 @@ def main():
     out = {"mulrelin": bench_default, "ntt": bench_ntt, "copy": bench_copy, "chain": bench_chain,
            "rotsum": bench_rotsum, "matvec": bench_matvec, "serve": bench_serve,
            "bfv8192": bench_bfv8192, "bfv": bench_bfv, "primitives": bench_primitives}[args.workload](args)
+    if not args.full:
+        print("[bench] whole result: " + json.dumps(out), file=sys.stderr, flush=True)
+        out = short_line(out)
     print(json.dumps(out), flush=True)
 
 
