@@ -312,7 +312,6 @@ __global__ void compose_kernel(const uint64_t *__restrict__ c, double2 *__restri
 // thread.  (The encoder's rounding fused into its columns pass the same way measured no
 // different, 1,118 against 611 + 515 us: its reductions bound it.)
 constexpr int EF = 3;
-constexpr uint64_t FUSED_BLOCKS = 512;
 
 template <int LOGN>
 __global__ __launch_bounds__(16 << (LOGN / 2 - EF)) void ntt_cols_compose_kernel(
@@ -349,9 +348,18 @@ __global__ void gather_kernel(const double2 *__restrict__ a, double *__restrict_
     }
 }
 
-// Plaintexts enough that one block per 16 columns of each fills the chip (N >= 2^13).
+// Plaintexts enough that one block per 16 columns of each fills the chip (N >= 2^13), which holds
+// 2^18 of its threads (N / 8 per plaintext; 116 VGPRs): three quarters of it up to N = 2^15, and,
+// with the two blocks per CU that fit at N = 2^16 and 2^17, all of it and three quarters of the
+// last round of blocks.  Decoding in us, separate / fused: N = 2^13, L = 4 64 plaintexts 72.1 / 77.7,
+// 160 107 / 105, 256 137 / 127; N = 2^15, L = 15 32 202 / 203, 40 238 / 247, 48 273 / 266, 64 366 / 335;
+// N = 2^16, L = 24 24 447 / 458, 32 574 / 516, 33 621 / 670, 40 739 / 716, 48 865 / 823, 68 1,239 /
+// 1,249, 128 2,208 / 2,045; N = 2^17, L = 12 16 336 / 336, 17 393 / 441, 24 517 / 493, 32 658 / 628.
 bool fused_columns(int logn, uint32_t batch) {
-    return logn >= 13 && logn <= 17 && ((uint64_t)batch << (logn - logn / 2 - 4)) >= FUSED_BLOCKS;
+    if (logn < 13 || logn > 17) return false;
+    const uint64_t chip = 1 << 18, threads = (uint64_t)batch << (logn - EF);
+    if (logn <= 15) return 4 * threads >= 3 * chip;
+    return threads >= chip && 4 * threads >= 3 * ((threads + chip - 1) / chip * chip);
 }
 
 template <class F>

@@ -355,10 +355,12 @@ def test_encode_polynomial_rejects():
         ctx.ckks_encode_polynomial(big.data_ptr(), n + 1, 1.0, 2, plain.data_ptr(), eb.data_ptr(), ew, stream())
 
 
-@pytest.mark.parametrize("logn,L,batch", [(13, 3, 64), (13, 1, 65), (14, 5, 64), (15, 2, 33), (16, 3, 32), (17, 2, 16)])
+@pytest.mark.parametrize("logn,L,batch", [(13, 3, 64), (13, 1, 65), (14, 5, 64), (15, 2, 33), (16, 3, 32), (17, 2, 16),
+                                           (13, 3, 191), (13, 3, 192), (14, 2, 97), (15, 4, 48), (16, 1, 33), (16, 2, 49),
+                                           (17, 1, 24)])
 def test_decode_batches_equal_single_plaintexts(logn, L, batch):
-    """Batches that take the composition fused into the transforms' last pass (512 blocks of 16
-    columns up) give the same doubles as plaintexts decoded alone."""
+    """Batches that take the composition fused into the transforms' last pass, and ones on the other
+    side of its lines, give the same doubles as plaintexts decoded alone."""
     n = 1 << logn
     moduli = ck.coeff_modulus_create(n, [60, 40, 50, 45, 60, 60][:L] + [60])
     ctx = hip().Context(2, n, moduli)
