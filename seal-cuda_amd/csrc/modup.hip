@@ -495,7 +495,9 @@ void launch_modup_as(const uint64_t *d, size_t d_stride, uint64_t *T, uint32_t c
     const uint32_t col_grid = cts * L * ((L + tc) / tc) * ((1u << K2) / CS);
     with_bool(mixed, [&](auto mx) {
         constexpr bool MIXED = decltype(mx)::value;
-        constexpr int EC = SMALL ? E : modup_cols_log(MIXED);
+        // (at N = 2^16 16 values win here although they spill: 1,230 against 1,280 us for 16
+        // ciphertexts at L = 24; 8 at N = 2^15 for 16 at L = 15 save 19 us of 1,266)
+        constexpr int EC = SMALL ? E : LOGN == 16 ? 4 : modup_cols_log(MIXED);
         if (tc == 1)
             ntt_cols_modup_kernel<LOGN, K1, EC, CS, true, MIXED><<<col_grid, CS << (K1 - EC), 0, st>>>(
                 d, d_stride, T, targets, digits, cts, L, skip_diag, tc);
