@@ -7,7 +7,7 @@
 
 namespace shc {
 
-DevPrime upload_prime(Context &c, uint64_t q) {
+DevPrime upload_prime(Context &c, uint64_t q, bool ciphertext) {
     // the NTT's lazy ranges reach 8q, which must fit 64 bits
     if (q >> 61) fail(ERR_INVALID_ARGUMENT, "modulus above 61 bits");
     const hm::NttTables t = hm::make_ntt_tables(c.logn, q);
@@ -20,21 +20,18 @@ DevPrime upload_prime(Context &c, uint64_t q) {
     p.inv_n = t.inv_n;
     p.inv_n_shoup = t.inv_n_shoup;
     const size_t bytes = t.fwd.size() * sizeof(uint64_t);
-    DevBuf buf(2 * bytes);
+    const bool fp = ciphertext && q < FP_PRIME_LIMIT;
+    DevBuf buf(2 * bytes + (fp ? c.n * sizeof(double2) : 0));
     SHC_HIP(hipMemcpy(buf.ptr, t.fwd.data(), bytes, hipMemcpyHostToDevice));
     SHC_HIP(hipMemcpy(static_cast<char *>(buf.ptr) + bytes, t.inv.data(), bytes, hipMemcpyHostToDevice));
     p.fwd = buf.as<const ulonglong2>();
     p.inv = reinterpret_cast<const ulonglong2 *>(static_cast<char *>(buf.ptr) + bytes);
-    c.table_bufs.push_back(std::move(buf));
-    if (q < FP_PRIME_LIMIT) {
-        DevBuf fp(c.n * sizeof(double2));
-        build_fp_table(p.fwd, fp.as<double2>(), q, c.logn, nullptr);
-        SHC_HIP(hipStreamSynchronize(nullptr));  // built before any stream's transform reads it
-        p.fwd_fp = fp.as<const double2>();
+    if (fp) {  // (built by make_context, for all primes at once)
+        p.fwd_fp = reinterpret_cast<const double2 *>(static_cast<char *>(buf.ptr) + 2 * bytes);
         p.q_fp = (double)q;
         p.q_inv_fp = 1.0 / (double)q;
-        c.table_bufs.push_back(std::move(fp));
     }
+    c.table_bufs.push_back(std::move(buf));
     return p;
 }
 
@@ -43,7 +40,7 @@ DevPrime Context::aux_prime(uint64_t q) {
     if (it != aux.end()) return it->second;
     for (size_t i = 0; i < moduli.size(); i++)
         if (moduli[i] == q) return aux[q] = host_primes[i];
-    return aux[q] = upload_prime(*this, q);
+    return aux[q] = upload_prime(*this, q, false);
 }
 
 const BehzLevel &Context::behz(size_t level) const {
@@ -78,12 +75,13 @@ std::unique_ptr<Context> make_context(Scheme scheme, int logn, const std::vector
     c->moduli = moduli;
     c->plain = plain;
     for (uint64_t q : moduli) {
-        c->host_primes.push_back(upload_prime(*c, q));
+        c->host_primes.push_back(upload_prime(*c, q, true));
         c->fp_primes |= q < FP_PRIME_LIMIT;
     }
 
     const size_t K = moduli.size();
     c->d_primes = upload(c->host_primes);
+    if (c->fp_primes) build_fp_tables(c->primes(), (uint32_t)K, logn, nullptr);
     if (K >= 2) {
         std::vector<DevPrime> ks((K - 1) * K);
         for (size_t L = 1; L < K; L++) {
@@ -138,6 +136,8 @@ std::unique_ptr<Context> make_context(Scheme scheme, int logn, const std::vector
         }
     }
     if (scheme == SCHEME_CKKS) build_ckks_tables(*c);
+    // the fp64 tables are there before any stream's transform reads them
+    if (c->fp_primes) SHC_HIP(hipStreamSynchronize(nullptr));
     return c;
 }
 

@@ -113,6 +113,6 @@ struct Context {
 std::unique_ptr<Context> make_context(Scheme scheme, int logn, const std::vector<uint64_t> &moduli, uint64_t plain);
 
 // Uploads NTT tables of q; throws invalid_argument when q has no 2N-th root of unity.
-DevPrime upload_prime(Context &c, uint64_t q);
+DevPrime upload_prime(Context &c, uint64_t q, bool ciphertext);
 
 }  // namespace shc

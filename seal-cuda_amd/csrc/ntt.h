@@ -201,7 +201,7 @@ struct ModDownGroup {
 };
 bool ntt_moddown_groups(const ModDownGroup *groups, uint32_t n, const DevPrime *primes, int logn, hipStream_t stream);
 
-// The fp64 form of a forward twiddle table (N entries) of a prime below FP_PRIME_LIMIT.
-void build_fp_table(const ulonglong2 *table, double2 *out, uint64_t q, int logn, hipStream_t stream);
+// The fp64 forms (fwd_fp) of the forward twiddle tables of those of `count` primes that have one.
+void build_fp_tables(const DevPrime *primes, uint32_t count, int logn, hipStream_t stream);
 
 }  // namespace shc

@@ -190,19 +190,20 @@ LimbGrid poly_grid(uint32_t count, uint32_t lpp) {
 }  // namespace
 
 namespace {
-__global__ void fp_table_kernel(const ulonglong2 *__restrict__ tw, double2 *__restrict__ out, uint64_t q, size_t n) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int64_t w = (int64_t)tw[i].x;
-    const double c = (double)(2 * (uint64_t)w > q ? w - (int64_t)q : w);
-    out[i] = double2{c, c / (double)q};
+__global__ void fp_tables_kernel(const DevPrime *__restrict__ primes, uint32_t n) {
+    const DevPrime &P = primes[blockIdx.y];
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (!P.fwd_fp || i >= n) return;
+    const int64_t w = (int64_t)P.fwd[i].x;
+    const double c = (double)(2 * (uint64_t)w > P.q ? w - (int64_t)P.q : w);
+    const_cast<double2 *>(P.fwd_fp)[i] = double2{c, c / (double)P.q};
 }
 }  // namespace
 
-void build_fp_table(const ulonglong2 *table, double2 *out, uint64_t q, int logn, hipStream_t st) {
-    const size_t n = (size_t)1 << logn;
-    fp_table_kernel<<<(uint32_t)((n + 255) / 256), 256, 0, st>>>(table, out, q, n);
-    launch_check("fp table");
+void build_fp_tables(const DevPrime *primes, uint32_t count, int logn, hipStream_t st) {
+    const uint32_t n = 1u << logn;
+    fp_tables_kernel<<<dim3((n + 255) / 256, count), 256, 0, st>>>(primes, n);
+    launch_check("fp tables");
 }
 
 void ntt_forward(uint64_t *data, uint32_t count, uint32_t lpp, const DevPrime *primes, int logn, NttOut out,
