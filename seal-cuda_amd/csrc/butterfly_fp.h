@@ -9,6 +9,11 @@
 //   h = RN(y w), l = y w - h (exact, one fma), b = rint(RN(y RN(w/q))),
 //   v = (h - b q) + l = y w - b q   exactly.
 //
+// (The error-free product by fma, Ogita, Rump and Oishi, "Accurate sum and dot product", 2005,
+// and the modular product with a quotient from a precomputed inverse that van der Hoeven,
+// Lecerf and Quintin build on it, "Modular SIMD arithmetic in Mathemagix", 2016; the bounds and
+// schedules below are for this transform.)
+//
 // With q < 2^50, |y| <= c q, c <= 8 and |w| <= q/2 (centred): RN(y RN(w/q)) is within
 // |y w / q| 2^-52 <= c 2^-3 of the quotient, so |v| <= (0.5 + c/8) q <= 1.5 q; |h| < 2^102,
 // so |l| <= 2^49, and h - b q = v - l is an integer below 2^52: both additions are exact.

@@ -439,7 +439,10 @@ uint32_t fill_starts(Table &t, const std::vector<uint64_t> &sizes) {
 // values and takes 54.4 with 4; 37 of them at N = 2^14, L = 7 645 and 581 us; a chain round
 // over 64 at N = 2^15 7.41 and 6.82 ms.  The line lies at 2^26 words (1,024 limbs of 2^16):
 // beyond it the forms differ by under 1% (encryption) or 16 values win (decryption of 128
-// ciphertexts at N = 2^16, L = 24: 3.13 against 3.26 ms).
+// ciphertexts at N = 2^16, L = 24: 3.13 against 3.26 ms).  (The transforms in place have lines
+// of their own, ntt.hip.)  N = 2^17 and the launches of several degrees are not compiled in the
+// small form; measured there, it would win for one or two ciphertexts (relinearization of one
+// at L = 2 93 -> 61 us, L = 8 213 -> 183, L = 24 1,132 -> 1,100) and is even at four.
 constexpr uint64_t SMALL_WORDS = uint64_t(1) << 26;
 template <int LOGN, bool SMALL>
 struct PassShape {

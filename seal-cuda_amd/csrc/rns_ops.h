@@ -43,8 +43,9 @@ void switch_key(const Context &c, const uint64_t *target, size_t target_stride, 
 //               S[ct][k] the special target's; with diag (after a skipped diagonal)
 //               the term j == i reads the NTT-form input limb diag + ct * diag_stride
 //               + i * N.
-//   moddown_into: ct_k[i] += ModDown(P_k, S_k)[i] (folded: P holds p ct_k, and ct_k = ModDown; S is consumed; U is scratch
-//               [count][2][L][N]; P in NTT form).
+//   moddown_into: ct_k[i] += ModDown(P_k, S_k)[i]; S is consumed; U is scratch
+//               [count][2][L][N]; P in NTT form.  folded: P also holds p ct_k, and ct_k is
+//               written unread.
 bool modup_to_T(const Context &c, const uint64_t *digits, size_t dstride, uint64_t *T, uint32_t count, uint32_t L,
                 hipStream_t st, const KernelProbe *probe = nullptr, bool skip_diag = false);
 void keyswitch_inner_product(const Context &c, const uint64_t *T, const uint64_t *key, uint64_t *P, uint64_t *S,

@@ -15,9 +15,10 @@ void hoisted_key_prepare(const Context &c, const uint64_t *galois_key, uint32_t 
 
 // out[ct] = sum_r rotate_{elt_r}(in[ct]) for ciphertexts [count][2][L][N], with the same
 // words as summing `rotations` separate apply_galois_keyswitch results.  hoisted[r] is
-// the prepared key of elts[r] at level L, keys[r] its Galois key (used when a digit of
-// c1 is zero, where hoisting is not exact, for the whole call).  Synchronises the
-// stream once (the zero-digit test), so it cannot be captured in a graph.
+// the prepared key of elts[r] at level L, keys[r] its Galois key.  Zero digits of c1, where
+// hoisting is not exact, are put right on the device.  Waits for nothing on the host (and so
+// can be captured in a graph) unless a key was not prepared through this context, whose
+// header is then read back.
 size_t rotate_sum_workspace(const Context &c, uint32_t count, uint32_t L);
 void rotate_sum(const Context &c, const uint64_t *in, uint32_t count, uint32_t L, const uint32_t *elts,
                 const uint64_t *const *hoisted, const uint64_t *const *keys, uint32_t rotations, uint64_t *out,
@@ -31,7 +32,8 @@ void rotate_many(const Context &c, const uint64_t *in, uint32_t count, uint32_t 
 
 // out[ct] = sum_h rotate_{elts[h]}(in[h][ct]), in: [n][count][2][L][N] (elts[h] == 1: in[h]
 // itself, no key), with the words of separate apply_galois_keyswitch calls summed, and one
-// ModDown for up to 15 of them: the giant steps of a BSGS matrix-vector product.
+// ModDown for up to 15 of them: the giant steps of a BSGS matrix-vector product.  A workspace
+// below the size asked for, down to one rotation's need, takes fewer rotations at a time.
 size_t rotate_accumulate_workspace(const Context &c, uint32_t count, uint32_t L);
 void rotate_accumulate(const Context &c, const uint64_t *in, uint32_t count, uint32_t L, const uint32_t *elts,
                        const uint64_t *const *keys, uint32_t n, uint64_t *out, void *ws, size_t ws_bytes,
