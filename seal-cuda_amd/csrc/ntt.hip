@@ -71,9 +71,20 @@ void launch_ntt_as(uint64_t *data, LimbGrid lg, uint32_t j0, uint32_t jn, const 
 // prime at N = 2^16: 2^22 words 38.0 / 36.9, 2^23 63.0 / 64.8, 2^24 113 / 123, 2^26 (62.5 M) 464 /
 // 552; N = 2^13, L = 4: 2^23 58.9 / 57.3, 2^24 102.7 / 107.3.  Inverse, N = 2^16: 2^23 69.4 /
 // 65.7, 2^24 121.6 / 126.6, 62.5 M 512 / 554; N = 2^13: 2^24 111.5 / 107.7, 2^25 220 / 224.
-// (Polynomials count in fours, a block's rows: 5 at N = 2^16, L = 24 68.7 / 74.3.)
+// (Polynomials count in fours, a block's rows: 5 at N = 2^16, L = 24 68.7 / 74.3.)  Where 16 values'
+// blocks of rows (16 of them at N = 2^15 and 2^16, 32 below) would idle for too many rows that are
+// not there, 4 values go on to SMALL_WORDS: N = 2^16, L = 24, forward 17 polynomials 218 / 204, 20
+// 242 / 238, 24 301 / 312; inverse 17 250 / 208, 20 278 / 245, 24 363 / 316, 26 377 / 347, 28 387 / 370.
 constexpr uint64_t NTT_SMALL_WORDS = (uint64_t(1) << 23) - 1;
 constexpr uint64_t INTT_SMALL_WORDS = (uint64_t(1) << 24) - 1;
+
+template <int LOGN, bool INV>
+uint64_t in_place_line(uint32_t jn) {
+    constexpr uint32_t RS = PassShape<LOGN, false>::RS;
+    const uint64_t rows = (uint64_t)((jn + RS - 1) / RS) * RS;
+    const bool ragged = jn >= RS && 16 * (uint64_t)jn <= (INV ? 13 : 10) * rows;
+    return ragged ? SMALL_WORDS : INV ? INTT_SMALL_WORDS : NTT_SMALL_WORDS;
+}
 
 template <int LOGN, bool INV, bool FULL>
 void launch_ntt(uint64_t *data, LimbGrid lg, uint32_t j0, uint32_t jn, const DevPrime *primes, hipStream_t st) {
@@ -82,7 +93,7 @@ void launch_ntt(uint64_t *data, LimbGrid lg, uint32_t j0, uint32_t jn, const Dev
     else
         with_shape<LOGN>((uint64_t)lg.I * (jn < 4 ? jn : (jn + 3) & ~3u), [&](auto s) {
             launch_ntt_as<LOGN, INV, FULL, decltype(s)::value>(data, lg, j0, jn, primes, st);
-        }, INV ? INTT_SMALL_WORDS : NTT_SMALL_WORDS);
+        }, in_place_line<LOGN, INV>(jn));
 }
 
 // Inverse transform of src's limbs into data (rows pass from src, columns pass in place).

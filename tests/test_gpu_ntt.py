@@ -42,6 +42,24 @@ def test_ntt_ragged_rows(logn, polys):
     check_ntt(logn, [60, 40], polys=polys, seed=logn + polys)
 
 
+@pytest.mark.parametrize("logn,limbs,polys", [(16, 24, 17), (15, 20, 26), (13, 40, 75)])
+def test_ragged_batches_agree(logn, limbs, polys):
+    """Batches past 2^23 (2^24) words whose last block of 16 (32) rows is mostly empty stay with 4
+    values per thread: the words of single polynomials, which the oracle checks above."""
+    import torch
+    n = 1 << logn
+    moduli = ck.coeff_modulus_create(n, [60, 40] * (limbs // 2))
+    ctx = hip().Context(2, n, moduli)
+    data = torch.randint(0, min(moduli), (polys, limbs, n), dtype=torch.int64, device="cuda")
+    for transform in (ctx.ntt_forward, ctx.ntt_inverse):
+        whole, one = data.clone(), data.clone()
+        transform(whole.data_ptr(), polys, limbs, stream())
+        for p in (0, polys // 2, polys - 1):
+            transform(one[p].data_ptr(), 1, limbs, stream())
+            torch.cuda.synchronize()
+            assert torch.equal(whole[p], one[p])
+
+
 def test_ntt_kat():
     # test/utils/ntt.cpp:75-99 on the GPU path
     ctx = hip().Context(hip().SCHEME_CKKS, 2, [0xFFFFFFFFFFC0001])
